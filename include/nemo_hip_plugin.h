@@ -122,6 +122,7 @@ typedef struct nemo_hip_neuron_group {
 	unsigned levels;
 	const uint32_t* level_ptr;
 	const uint32_t* level_idx;
+	uint64_t incoming; /* the group's incoming synapses in the all-synapse reverse matrix (0: none built) */
 } nemo_hip_neuron_group;
 
 /* The all-synapse reverse matrix (construction/RCM.cpp:76-98), built when a

@@ -759,6 +759,7 @@ void Simulation::buildNeurons(const std::vector<const Network*>& nets)
 		g.dev.levels = 1;
 		g.dev.level_ptr = nullptr;
 		g.dev.level_idx = nullptr;
+		g.dev.incoming = 0;
 		if(g.type.scratchPlanes && g.count) {
 			g.scratch.allocate(size_t(g.type.scratchPlanes) * pitch);
 			g.dev.scratch = g.scratch.ptr;
@@ -1001,6 +1002,7 @@ void Simulation::buildConnectivity(const std::vector<const Network*>& nets, cons
 			for(size_t k = 0; k < s.ax->target.size(); ++k) ptr[ltgt[s.seq + k] + 1] += 1;
 		}
 		for(size_t n = 0; n < N; ++n) ptr[n + 1] += ptr[n];
+		for(Group& g : m_groups) g.dev.incoming = ptr[g.start + g.count] - ptr[g.start];
 		std::vector<uint32_t> fill(ptr.begin(), ptr.end() - 1);
 		std::vector<uint32_t> sd(std::max<size_t>(1, m_nsynapses));
 		std::vector<float> w(std::max<size_t>(1, m_nsynapses));

@@ -263,6 +263,7 @@ gather_currents_kernel(nemo_hip_step_buffers b, const uint32_t* dev_to_sim, floa
 	g.state = nullptr;
 	g.rng = nullptr;
 	g.scratch = nullptr;
+	g.incoming = 0;
 	nemo_dev::gather_input(b, g, L);
 	const unsigned ng = blockIdx.x * NEMO_TILE + threadIdx.x;
 	float e, i;
