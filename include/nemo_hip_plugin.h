@@ -36,6 +36,10 @@
  *     fired_bits[(s % NEMO_STEP_RING) * fired_words + index / 64];
  *   - when co.push is set, deliver the delay-1 events of the step's firing
  *     for step s+1 (see nemo_hip_colaunch);
+ *   - when direct.ring is not NULL, the input is the step's slot of the ring
+ *     instead, and the delay-1 events of the step's firing and the others of
+ *     the step before are added to the slots of their arrival (see
+ *     nemo_hip_direct);
  *   - when stdp.rcm_ptr is not NULL, run the STDP accumulation of step s-1 for
  *     the tile's neurons (see nemo_hip_stdp).
  * The helpers in nemo_amd/csrc/plugin_device.h implement all of this but the
@@ -246,6 +250,31 @@ typedef struct nemo_hip_colaunch {
 	nemo_propagate_args args;
 } nemo_hip_colaunch;
 
+/* Direct delivery (networks of few synapses): a ring of input accumulators,
+ * slot s & mask holding the input of step s.  The update launches of step t
+ * add the events of a firing to its arrival steps' slots with atomics: its
+ * tiles' blocks the delay-1 events of step t, and late_blocks more blocks
+ * (after the group's tiles, `parts` per tile of the network: tile * parts +
+ * part) the events of delays 2.. of step t - 1, beside the tiles' own work;
+ * one group's launch of the step carries them.  The update of step s
+ * reads and clears its own slot.  No delivery launch runs, and bins,
+ * bin_table and acc are unused.  arrivals counts, per source tile, the events
+ * of each slot; the update of the step adds its tile's entry to the tile's
+ * event counter and clears it.  ring NULL: not direct. */
+typedef struct nemo_hip_direct {
+	int64_t* ring;             /* [mask + 1][2][acc_pitch]: E plane, then I plane of each slot */
+	const uint2* first_rows;   /* per device index: fcm [x, y) of its synapses of delay 1 */
+	const uint2* late_rows;    /* per device index: fcm [x, y) of its other synapses */
+	const int2* fcm;           /* {target device index, Q11.20 weight} */
+	const uint8_t* delay;      /* per fcm entry: its delay - 1 */
+	uint32_t* arrivals;        /* [mask + 1][tiles] */
+	unsigned long long* events; /* per 64 device indices; a tile uses its first */
+	unsigned mask;             /* slots - 1, a power of two less one; at least the longest delay */
+	unsigned tiles;
+	unsigned parts;            /* 0: no synapse has a delay above 1 */
+	unsigned late_blocks;      /* of this launch: tiles * parts, or 0 */
+} nemo_hip_direct;
+
 /* Per-simulation buffers shared by all groups in a step. */
 typedef struct nemo_hip_step_buffers {
 	uint64_t step_offset;      /* step = clock->base_step + step_offset */
@@ -285,6 +314,7 @@ typedef struct nemo_hip_step_buffers {
 	                              set's columns only, [0, bin_first_set) of each table row (with
 	                              bin_ranged: in the tile's first range only); the delay-1 events
 	                              were pushed into acc by the previous step's update */
+	nemo_hip_direct direct;    /* direct delivery (ring NULL: binned) */
 } nemo_hip_step_buffers;
 
 typedef hipError_t hip_update_neurons_t(hipStream_t stream,

@@ -529,6 +529,7 @@ void Simulation::construct(const std::vector<const Network*>& nets, const Config
 	buildConnectivity(nets, conf);
 	buildStdp(conf);
 	allocateStepState();
+	buildDirect();
 	applyShape(defaultShape());
 
 	size_t models = 0;
@@ -866,6 +867,8 @@ void Simulation::buildConnectivity(const std::vector<const Network*>& nets, cons
 	for(size_t r = 0; r < N * D; ++r) rowptr[r + 1] += rowptr[r];
 
 	/* fill rows (stable within a source) */
+	const bool direct = directPays();
+	if(direct) m_fcmDelayHost.resize(std::max<size_t>(1, m_nsynapses));
 	std::vector<int2> fcm(std::max<size_t>(1, m_nsynapses));
 	m_synAddr.resize(m_nsynapses);
 	if(!m_writeOnly) {
@@ -893,6 +896,7 @@ void Simulation::buildConnectivity(const std::vector<const Network*>& nets, cons
 			}
 			fcm[pos].x = int(ltgt[s.seq + k]);
 			fcm[pos].y = wf;
+			if(direct) m_fcmDelayHost[pos] = uint8_t(d - 1);
 			m_synAddr[s.seq + k] = pos;
 			if(!m_writeOnly) {
 				m_synTarget[s.seq + k] = s.ax->target[k];
@@ -922,6 +926,11 @@ void Simulation::buildConnectivity(const std::vector<const Network*>& nets, cons
 		for(size_t n = 0; n < N; ++n) d1[n] = make_uint2(rowptr[n * D], rowptr[n * D + 1]);
 		m_d1Rows.allocate(N);
 		HIP_CHECK(hipMemcpy(m_d1Rows.ptr, d1.data(), m_d1Rows.bytes(), hipMemcpyHostToDevice));
+		if(direct) {
+			for(size_t n = 0; n < N; ++n) d1[n] = make_uint2(rowptr[n * D + 1], rowptr[n * D + D]);
+			m_lateRows.allocate(N);
+			HIP_CHECK(hipMemcpy(m_lateRows.ptr, d1.data(), m_lateRows.bytes(), hipMemcpyHostToDevice));
+		}
 	}
 	m_fcm.allocate(fcm.size());
 	HIP_CHECK(hipMemcpy(m_fcm.ptr, fcm.data(), m_fcm.bytes(), hipMemcpyHostToDevice));
@@ -1190,7 +1199,97 @@ static Partition partitionPairs(const std::vector<uint64_t>& pairWeight, const s
 	return P;
 }
 
-/* Default shape: bin capacity 4096 events (halved while the LDS does not
+/* Direct delivery pays while a step's events are few: it costs a step the
+ * atomics of all of them (23 G a second), the binned delivery a chain of
+ * dependent phases that is nearly as long for 1000 neurons as for 30,000.
+ * Measured on 80/20 Izhikevich networks firing at 6 to 9 Hz (neurons x
+ * synapses, us a step, direct / binned): 500 x 50 5.8 / 9.4, 1000 x 100 5.5 /
+ * 8.9, 10000 x 200 6.2 / 10.0, 10000 x 1000 9.1 / 12.3, 30000 x 333 8.6 /
+ * 11.3, 100000 x 100 8.8 / 20.4, 30000 x 600 11.0 / 11.8, 50000 x 400 11.2 /
+ * 11.6, 30000 x 1000 16.5 / 12.5, 100000 x 400 18.9 / 13.3.  So up to
+ * DIRECT_MAX_SYNAPSES synapses, of which such a step delivers under 1%; the
+ * ring of accumulators must not be out of proportion either (many neurons of
+ * few synapses and long delays).  The tuning variables of the binned
+ * delivery, or of the STDP placement, ask for that delivery. */
+static const size_t DIRECT_MAX_SYNAPSES = size_t(16) << 20;
+static const size_t DIRECT_MAX_RING = size_t(1) << 30;
+static const unsigned DIRECT_PARTS = 16;
+
+static unsigned ringSlots(unsigned D)
+{
+	unsigned slots = 2;
+	while(slots < D + 1) slots *= 2;
+	return slots;
+}
+
+bool Simulation::directPays() const
+{
+	for(const char* v : {"NEMO_HIP_DELIVER_BLOCKS", "NEMO_HIP_LATE_BLOCKS", "NEMO_HIP_BIN_CAPACITY", "NEMO_HIP_OVERLAP",
+			"NEMO_HIP_BIN_RANGED", "NEMO_HIP_STDP_MODE"}) {
+		if(std::getenv(v)) return false;
+	}
+	return m_nsynapses > 0 && m_nsynapses <= DIRECT_MAX_SYNAPSES
+		&& size_t(ringSlots(m_D)) * 2 * m_npad * sizeof(int64_t) <= DIRECT_MAX_RING;
+}
+
+/* The ring, cleared: no step has run, so no event is under way. */
+void Simulation::buildDirect()
+{
+	std::memset(&m_direct, 0, sizeof(m_direct));
+	if(!directPays()) return;
+	const unsigned slots = ringSlots(m_D);
+	m_ring.allocate(size_t(slots) * 2 * m_accPitch);
+	HIP_CHECK(hipMemset(m_ring.ptr, 0, m_ring.bytes()));
+	m_arrivals.allocate(size_t(slots) * m_tiles);
+	HIP_CHECK(hipMemset(m_arrivals.ptr, 0, m_arrivals.bytes()));
+	m_fcmDelay.allocate(m_fcmDelayHost.size());
+	HIP_CHECK(hipMemcpy(m_fcmDelay.ptr, m_fcmDelayHost.data(), m_fcmDelay.bytes(), hipMemcpyHostToDevice));
+	std::vector<uint8_t>().swap(m_fcmDelayHost);
+	m_direct.ring = m_ring.ptr;
+	m_direct.mask = slots - 1;
+	m_direct.tiles = m_tiles;
+	m_direct.first_rows = m_d1Rows.ptr;
+	m_direct.late_rows = m_lateRows.ptr;
+	/* about one block per CU beside the tiles: enough that a tile which fires
+	 * a lot is spread out (10k neurons of 200 and 1000 synapses, us a step: a
+	 * block per CU 6.0 and 9.0, two 6.1 and 9.1, four 6.1 and 9.4) */
+	m_direct.parts = m_D > 1 ? std::max(1u, std::min(DIRECT_PARTS, m_cuCount / std::max(1u, m_tiles))) : 0;
+	m_direct.fcm = m_fcm.ptr;
+	m_direct.delay = m_fcmDelay.ptr;
+	m_direct.arrivals = m_arrivals.ptr;
+	m_direct.events = m_blockEvents.ptr + NEMO_MAX_BIN_BLOCKS;
+	m_ringStale = false;
+}
+
+/* The group whose launch carries the blocks for the events of delays 2..: one
+ * whose step is a single launch, if there is any, as those that split theirs
+ * (with scratch planes) wait for the first launch of a step (HH beside LIF:
+ * 5 us a step). */
+size_t Simulation::directCarrier() const
+{
+	size_t first = m_groups.size();
+	for(size_t gi = 0; gi < m_groups.size(); ++gi) {
+		if(m_groups[gi].dev.count == 0) continue;
+		if(!m_groups[gi].dev.scratch) return gi;
+		first = std::min(first, gi);
+	}
+	return first;
+}
+
+/* The ring holds events added with the weights of the time their neuron
+ * fired, for the steps that follow one another; after anything else (applyStdp,
+ * another shape's steps, a restored state) it is set up again from the firing
+ * bitmaps before the next step. */
+void Simulation::ensureRing()
+{
+	if(!m_shape.direct || !m_ringStale) return;
+	HIP_CHECK(nemo_launch_direct_rebuild(m_stream, &m_direct, m_accPitch, m_rowptr.ptr, m_D, m_firedBits.ptr,
+				m_firedWords, m_hostStep));
+	m_ringStale = false;
+}
+
+/* Default shape: direct delivery where it pays, beside the binned shape that
+ * follows from the sizes: bin capacity 4096 events (halved while the LDS does not
  * allow it), enough delivery blocks for about 1% of the synapses per step,
  * and, with delays above 1 and few enough blocks to be resident together, a
  * delay-1 set of about 1/D of them, so that the update launches carry the
@@ -1227,6 +1326,7 @@ LaunchShape Simulation::defaultShape() const
 	}
 	s.stdpMode = 4;
 	s.stdpWords = NEMO_STDP_BATCH_WORDS; /* about one batch block per CU disturbs the steps least */
+	s.direct = m_direct.ring != nullptr;
 	auto env = [](const char* name, int lo, int hi, unsigned& field) {
 		if(const char* e = std::getenv(name)) field = unsigned(std::max(lo, std::min(std::atoi(e), hi)));
 	};
@@ -1313,6 +1413,8 @@ void Simulation::applyShape(const LaunchShape& s)
 	clearGraphs();
 	m_shape = s;
 	m_shape.deliverBlocks = Be;
+	m_shape.direct = s.direct && m_direct.ring;
+	if(m_hostStep > 0) m_ringStale = true;
 
 	/* both sets back to back: bounds [Be+1 | Bl+1], windows [Be | Bl]; the
 	 * per-tile ranges in absolute table columns, early set then late set */
@@ -1499,6 +1601,10 @@ nemo_hip_step_buffers Simulation::stepBuffers(uint64_t offset, bool ext, bool fs
 	b.fbits = m_fbits;
 	b.debug_current = m_debug ? m_debugCurrent.ptr : nullptr;
 	b.stdp = m_stdpArgs;
+	if(m_shape.direct) {
+		b.direct = m_direct;
+		b.direct.late_blocks = m_direct.tiles * m_direct.parts;
+	}
 	if(m_shape.stdpMode != 1) b.stdp.rcm_ptr = nullptr; /* STDP runs in a launch of its own */
 	b.rcm_all.ptr = m_rcmAllPtr.ptr;
 	b.rcm_all.source_delay = m_rcmAllSd.ptr;
@@ -1624,7 +1730,9 @@ void Simulation::launchDelivery(const nemo_propagate_args& set, uint64_t offset,
 void Simulation::enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, hipEvent_t* ev, bool forkPending,
 		bool advanceBase)
 {
-	const bool split = m_late.deliver_blocks && m_early.deliver_blocks;
+	/* direct delivery: the updates are the whole step */
+	const bool direct = m_shape.direct;
+	const bool split = !direct && m_late.deliver_blocks && m_early.deliver_blocks;
 	const bool overlap = split && m_shape.overlap == 1 && k > 1;
 	/* the update of step t carries the delivery of the delays 2..D of step
 	 * t+1 as extra blocks (and, with fused STDP, the STDP blocks); with
@@ -1681,8 +1789,8 @@ void Simulation::enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, 
 		/* with ev: four events per step, recorded by the kernels: start
 		 * and end of the delivery on this stream, of the neuron updates */
 		hipEvent_t ps = ev ? ev[4 * i] : nullptr, pe = ev ? ev[4 * i + 1] : nullptr;
-		if(split && pushed && i > 0) {
-			/* delivered by the previous step's update launch (no propagate
+		if(direct || (split && pushed && i > 0)) {
+			/* delivered by the updates of the steps before, or by the previous step's update launch (no propagate
 			 * launch to time: ps and pe stay unrecorded) */
 		} else if(split) {
 			const bool early = i == 0 || (!overlap && !colaunch);
@@ -1721,6 +1829,8 @@ void Simulation::enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, 
 			b.co.push_rows = m_d1Rows.ptr;
 		}
 		if(pushed && i > 0) b.bin_first_set = m_early.deliver_blocks;
+		const unsigned late = b.direct.late_blocks;
+		const size_t carrier = direct ? directCarrier() : m_groups.size();
 		size_t last = m_groups.size();
 		for(size_t gi = 0; gi < m_groups.size(); ++gi) {
 			if(m_groups[gi].dev.count) last = gi;
@@ -1731,6 +1841,7 @@ void Simulation::enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, 
 				Group& g = m_groups[gi];
 				if(g.dev.count == 0) continue;
 				if(ev && gi == last) b.time_stop = ev[4 * i + 3];
+				b.direct.late_blocks = gi == carrier ? late : 0;
 				HIP_CHECK(g.plugin->update(m_stream, &g.dev, &b));
 				b.co.deliver_blocks = 0; /* the first group's launch carries them */
 				b.co.stdp_blocks = 0;
@@ -1752,6 +1863,7 @@ void Simulation::enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, 
 			for(size_t gi = 0; gi < m_groups.size(); ++gi) {
 				Group& g = m_groups[gi];
 				if(g.dev.count == 0) continue;
+				b.direct.late_blocks = gi == carrier ? late : 0;
 				if(first) {
 					HIP_CHECK(g.plugin->update(m_stream, &g.dev, &b));
 					b.co.deliver_blocks = 0; /* the first group's launch carries them */
@@ -2002,6 +2114,7 @@ const std::vector<unsigned>& Simulation::step(const unsigned* fstim, size_t nf,
 		HIP_CHECK(nemo_launch_fstim(m_stream, m_fstim.ptr, m_stimIdx.ptr, fIdx.size(), 1));
 	}
 	const uint64_t t = m_hostStep;
+	ensureRing();
 	setBase(t);
 	enqueueSteps(0, 1, !iIdx.empty(), !fIdx.empty());
 	advanceSteps(1);
@@ -2189,6 +2302,7 @@ void Simulation::run(unsigned nsteps, unsigned stdpPeriod, float reward, bool re
 			hipGraphExec_t g = graphFor(k, batchPending);
 			batchPending = true; /* each chunk leaves its steps pending */
 			const bool advances = graphsAdvanceBase();
+			ensureRing();
 			if(!advances || m_base != t0) setBase(t0);
 			/* the ring slots this chunk overwrites were copied out */
 			if(inFlight[half]) HIP_CHECK(hipStreamWaitEvent(m_stream, copied[half], 0));
@@ -2279,6 +2393,7 @@ void Simulation::profile(unsigned nsteps, double avgUs[4], uint64_t counters[4])
 	std::vector<hipEvent_t> ev(4 * size_t(nsteps));
 	for(hipEvent_t& e : ev) HIP_CHECK(hipEventCreate(&e));
 	const uint64_t t0 = m_hostStep;
+	ensureRing();
 	setBase(t0);
 	/* runs of up to 64 steps, as in a graph, with events between the launches */
 	for(unsigned s = 0; s < nsteps; s += 64) {
@@ -2287,10 +2402,11 @@ void Simulation::profile(unsigned nsteps, double avgUs[4], uint64_t counters[4])
 	advanceSteps(nsteps);
 	HIP_CHECK(hipStreamSynchronize(m_stream));
 	const bool pushed = m_late.deliver_blocks && m_early.deliver_blocks && m_shape.overlap == 3;
+	const bool direct = m_shape.direct;
 	double sum[3] = {0, 0, 0};
 	unsigned launches = 0;
 	for(unsigned s = 0; s < nsteps; ++s) {
-		const bool propagate = !(pushed && s % 64 != 0);
+		const bool propagate = !direct && !(pushed && s % 64 != 0);
 		launches += propagate ? 1 : 0;
 		for(int k = propagate ? 0 : 1; k < 2; ++k) {
 			float ms = 0;
@@ -2392,6 +2508,7 @@ void Simulation::restoreSnapshot(const Snapshot& s)
 	m_base = s.base;
 	m_lastCycle = s.lastCycle;
 	m_updated = s.updated;
+	m_ringStale = true;
 }
 
 /* Advance nsteps steps in graphs of up to 64 steps, then their pending STDP
@@ -2408,6 +2525,7 @@ double Simulation::timeSteps(unsigned nsteps)
 		const unsigned k = std::min(64u, nsteps - done);
 		hipGraphExec_t g = graphFor(k, true);
 		const bool advances = graphsAdvanceBase();
+		ensureRing();
 		if(!advances || m_base != m_hostStep) setBase(m_hostStep);
 		HIP_CHECK(hipGraphLaunch(g, m_stream));
 		if(advances) m_base = m_hostStep + k;
@@ -2452,7 +2570,8 @@ LaunchShape Simulation::autotune(unsigned stepsPerTrial)
 	};
 	LaunchShape best = start;
 	double tBest = trial(best);
-	auto consider = [&](const LaunchShape& c) {
+	auto consider = [&](LaunchShape c, bool delivery = true) {
+		if(delivery) c.direct = false; /* the candidate differs in what direct delivery has no use for */
 		const double t = trial(c);
 		if(t < tBest) {
 			tBest = t;
@@ -2524,7 +2643,7 @@ LaunchShape Simulation::autotune(unsigned stepsPerTrial)
 			if(w == best.stdpWords) continue;
 			LaunchShape c = best;
 			c.stdpWords = w;
-			consider(c);
+			consider(c, false);
 		}
 	}
 	/* the descent keeps whatever won one trial; a shape other than the
@@ -2532,7 +2651,8 @@ LaunchShape Simulation::autotune(unsigned stepsPerTrial)
 	 * only if it is faster in total (single trials vary by a few percent) */
 	auto same = [](const LaunchShape& x, const LaunchShape& y) {
 		return x.deliverBlocks == y.deliverBlocks && x.lateBlocks == y.lateBlocks && x.binCapacity == y.binCapacity
-			&& x.stdpMode == y.stdpMode && x.stdpWords == y.stdpWords && x.overlap == y.overlap;
+			&& x.stdpMode == y.stdpMode && x.stdpWords == y.stdpWords && x.overlap == y.overlap
+			&& x.direct == y.direct;
 	};
 	if(!same(best, start)) {
 		double tb = 0, ts = 0;
@@ -2582,6 +2702,7 @@ void Simulation::applyStdp(float reward)
 	a.fbits = m_fbits;
 	HIP_CHECK(nemo_launch_apply_stdp(m_stream, &a));
 	m_fcmHostValid = false;
+	m_ringStale = true;
 }
 
 /* ------------------------------------------------ externally given firing */
@@ -2610,13 +2731,16 @@ void Simulation::propagateDevice(const uint32_t* flags, float** E, float** I)
 	}
 	joinStdp();
 	const uint64_t s = m_hostStep;
+	ensureRing();
 	setBase(s);
 	nemo_hip_step_buffers b = stepBuffers(0, false, false);
 	b.debug_current = nullptr;
 	HIP_CHECK(nemo_launch_external_fire(m_stream, &b, flags, m_devToSim.ptr, m_tiles));
-	setBase(s + 1);
-	launchDelivery(m_early, 0, m_stream, false);
-	launchDelivery(m_late, 0, m_stream, false);
+	b.step_offset = 1;
+	if(!m_shape.direct) {
+		launchDelivery(m_early, 1, m_stream, false);
+		launchDelivery(m_late, 1, m_stream, false);
+	}
 	HIP_CHECK(nemo_launch_gather_currents(m_stream, &b, m_devToSim.ptr, m_extE.ptr, m_extI.ptr, m_tiles));
 	m_hostStep = s + 1;
 	HIP_CHECK(hipStreamSynchronize(m_stream));

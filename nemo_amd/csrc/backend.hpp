@@ -161,6 +161,9 @@ struct LaunchShape {
 	                                 branch beside the previous update, 2 as extra blocks of the
 	                                 previous update launch, 3 as in 2 with the previous update's
 	                                 tiles pushing the delay-1 events too (one launch per step) */
+	bool direct = false;          /* no delivery launches: the updates add their firing's events to a ring
+	                                 of input accumulators (nemo_hip_direct); the fields above but the
+	                                 STDP's then only say what a shape set without it would be */
 };
 
 /* The HIP simulation (cuda::Simulation's role, cuda/Simulation.cpp:91-380).
@@ -339,6 +342,14 @@ private:
 	bool m_debug = false;
 	DeviceArray<uint32_t> m_rowptr;
 	DeviceArray<uint2> m_d1Rows;      /* [N] the delay-1 row of each device index: fcm [x, y) */
+	/* direct delivery, where defaultShape chooses it */
+	nemo_hip_direct m_direct;         /* ring NULL: this network cannot be delivered directly */
+	DeviceArray<int64_t> m_ring;
+	DeviceArray<uint2> m_lateRows;    /* [N] the synapses of delay 2.. of each device index: fcm [x, y) */
+	DeviceArray<uint8_t> m_fcmDelay;  /* per fcm entry: its delay - 1 */
+	DeviceArray<uint32_t> m_arrivals;
+	std::vector<uint8_t> m_fcmDelayHost; /* from buildConnectivity to buildDirect */
+	bool m_ringStale = false;         /* the ring must be set up again from the bitmaps before the next step */
 	DeviceArray<int2> m_fcm;
 	DeviceArray<uint32_t> m_rcmPtr, m_rcmSd, m_rcmFwd;
 	DeviceArray<uint32_t> m_rcmOf;    /* per FCM synapse: accumulator index, ~0 if static */
@@ -429,6 +440,10 @@ private:
 	void buildStdp(const Configuration& conf);
 	void allocateStepState();
 	LaunchShape defaultShape() const;
+	bool directPays() const;
+	size_t directCarrier() const;
+	void buildDirect();
+	void ensureRing();
 	void applyShape(const LaunchShape& s);
 	size_t ldsNeeded(const LaunchShape& s) const;
 	void resetStdpBatches();

@@ -96,14 +96,22 @@ hipError_t nemo_launch_apply_stdp(hipStream_t, const nemo_apply_args*);
 hipError_t nemo_launch_invert_rcm(hipStream_t, const uint32_t* rcm_fwd, uint32_t* rcm_of, size_t count,
 		size_t fcm_count);
 
-/* Firing of step base_step given from outside (one flag per neuron in
- * simulation order; dev_to_sim maps device index -> simulation index, ~0
- * for padding): histories and the step's bitmap written as by an update.
- * One block per tile. */
+/* Firing of step base_step + step_offset given from outside (one flag per
+ * neuron in simulation order; dev_to_sim maps device index -> simulation
+ * index, ~0 for padding): histories and the step's bitmap written as by an
+ * update, and, with direct delivery, the events an update would deliver. */
 hipError_t nemo_launch_external_fire(hipStream_t, const nemo_hip_step_buffers* b, const uint32_t* flags,
 		const uint32_t* dev_to_sim, unsigned tiles);
-/* Synaptic input of step base_step gathered per tile (overflow accumulators
- * cleared) and written as floats in simulation order. */
+/* The ring of a directly delivered network set up from the firing of the
+ * steps before t0 (its bitmaps) and the present weights: cleared, then the
+ * events of every firing of the last D steps that arrive from t0 on, without
+ * those that the update of step t0 delivers. */
+hipError_t nemo_launch_direct_rebuild(hipStream_t, const nemo_hip_direct* r, size_t acc_pitch, const uint32_t* rowptr,
+		unsigned D, const uint64_t* fired_bits, size_t fired_words, uint64_t t0);
+/* Synaptic input of step base_step + step_offset gathered per tile (overflow
+ * accumulators cleared; with direct delivery, the slot of the step before it
+ * cleared, which no update has read) and written as floats in simulation
+ * order. */
 hipError_t nemo_launch_gather_currents(hipStream_t, const nemo_hip_step_buffers* b, const uint32_t* dev_to_sim,
 		float* E, float* I, unsigned tiles);
 

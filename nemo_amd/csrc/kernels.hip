@@ -22,6 +22,8 @@
  *                          bins (entries of the blocks whose window holds t)
  *   acc        int64[2][2][N] overflow accumulators (events beyond CAP)
  *   rcm_*      per target, its plastic incoming synapses (STDP only)
+ * and, for a network delivered directly (nemo_hip_direct), the ring of input
+ * accumulators int64[slots][2][N] in place of bins, bin_table and acc.
  */
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
@@ -234,6 +236,14 @@ fired_list_kernel(const uint64_t* bits, size_t words, uint64_t t0, const uint32_
 
 /* ------------------------------------------- externally given firing */
 
+/* All tiles as one group, for the blocks that need no more of it. */
+__device__ inline nemo_hip_neuron_group whole_group(unsigned tiles)
+{
+	nemo_hip_neuron_group g = {};
+	g.count = tiles * NEMO_TILE;
+	return g;
+}
+
 /* The firing of step s given from outside (Brian's propagate,
  * cpu/Simulation.cpp:115-137): neuron ng fired if flags[sim] is nonzero for
  * its simulation index sim = dev_to_sim[ng] (~0 for padding); its history
@@ -241,11 +251,44 @@ fired_list_kernel(const uint64_t* bits, size_t words, uint64_t t0, const uint32_
 __global__ void __launch_bounds__(NEMO_TILE)
 external_fire_kernel(nemo_hip_step_buffers b, const uint32_t* flags, const uint32_t* dev_to_sim)
 {
+	nemo_dev::UpdateLds& L = nemo_dev::update_lds<false>();
+	if(b.direct.ring && nemo_dev::direct_block(b, whole_group(b.direct.tiles), L)) return;
 	const unsigned ng = blockIdx.x * NEMO_TILE + threadIdx.x;
 	const uint32_t sim = dev_to_sim[ng];
 	const bool valid = sim != ~0u;
 	const uint64_t h = nemo_dev::load_history(b, ng, valid);
-	nemo_dev::record_firing(b, ng, valid, valid && flags[sim] != 0u, h);
+	nemo_dev::begin_push(b, L, ng);
+	nemo_dev::record_firing<false>(b, L, ng, valid, valid && flags[sim] != 0u, h);
+}
+
+/* ------------------------------------------------------ direct delivery */
+
+/* The events that arrive from step t0 on of the firing of step t0 - j, j =
+ * 1 .. D (blockIdx.y + 1), of source tile blockIdx.x: of a neuron that fired
+ * then, the rows of delays j .. D, which follow each other in the FCM; of the
+ * last step's firing the delay-1 row only, as the update of step t0 delivers
+ * the others. */
+__global__ void __launch_bounds__(NEMO_TILE)
+direct_rebuild_kernel(nemo_hip_direct r, size_t acc_pitch, const uint32_t* rowptr, unsigned D,
+		const uint64_t* fired_bits, size_t fired_words, uint64_t t0)
+{
+	__shared__ uint2 s_chunk[nemo_dev::DIRECT_CHUNKS];
+	__shared__ uint32_t s_count[64], s_chunks;
+	const unsigned tile = blockIdx.x, j = blockIdx.y + 1, tid = threadIdx.x;
+	if(t0 < j) return;
+	const uint64_t t = t0 - j;
+	const uint64_t word = fired_bits[(t & (NEMO_STEP_RING - 1)) * fired_words + size_t(tile) * (NEMO_TILE / 64) + tid / 64];
+	const bool fired = (word >> (tid & 63)) & 1u;
+	if(tid < 64) s_count[tid] = 0;
+	if(tid == 64) s_chunks = 0;
+	if(!__syncthreads_or(fired)) return;
+	uint2 row = make_uint2(0, 0);
+	if(fired) {
+		const size_t n = size_t(tile) * NEMO_TILE + tid;
+		row.x = rowptr[n * D + j - 1];
+		row.y = rowptr[n * D + (j == 1 ? 1 : D)];
+	}
+	nemo_dev::deliver_direct(r, acc_pitch, row, t, tile, 0, 1, s_chunk, &s_chunks, s_count);
 }
 
 /* The synaptic input of a step, gathered per tile as the neuron updates
@@ -255,17 +298,26 @@ __global__ void __launch_bounds__(NEMO_TILE)
 gather_currents_kernel(nemo_hip_step_buffers b, const uint32_t* dev_to_sim, float* E, float* I)
 {
 	nemo_dev::UpdateLds& L = nemo_dev::update_lds<false>();
-	nemo_hip_neuron_group g;
-	g.start = 0;
-	g.count = gridDim.x * NEMO_TILE;
-	g.pitch = 0;
-	g.param = nullptr;
-	g.state = nullptr;
-	g.rng = nullptr;
-	g.scratch = nullptr;
-	g.incoming = 0;
-	nemo_dev::gather_input(b, g, L);
+	const nemo_hip_neuron_group g = whole_group(gridDim.x);
 	const unsigned ng = blockIdx.x * NEMO_TILE + threadIdx.x;
+	if(b.direct.ring) {
+		/* read, not taken: an update of this step would still find its
+		 * input.  The step before passed without one: its slot is cleared
+		 * for the steps to come. */
+		const nemo_hip_direct& r = b.direct;
+		const uint64_t t = nemo_dev::current_step(b);
+		const size_t slot = size_t(t) & r.mask, before = size_t(t - 1) & r.mask;
+		L.input.E[threadIdx.x] = r.ring[slot * 2 * b.acc_pitch + ng];
+		L.input.I[threadIdx.x] = r.ring[(slot * 2 + 1) * b.acc_pitch + ng];
+		r.ring[before * 2 * b.acc_pitch + ng] = 0;
+		r.ring[(before * 2 + 1) * b.acc_pitch + ng] = 0;
+		if(threadIdx.x == 0) {
+			r.events[ng >> 6] += r.arrivals[slot * r.tiles + blockIdx.x];
+			r.arrivals[before * r.tiles + blockIdx.x] = 0;
+		}
+	} else {
+		nemo_dev::gather_input(b, g, L);
+	}
 	float e, i;
 	nemo_dev::take_current(b, L.input, ng, e, i);
 	const uint32_t sim = dev_to_sim[ng];
@@ -459,7 +511,27 @@ hipError_t nemo_launch_external_fire(hipStream_t st, const nemo_hip_step_buffers
 		const uint32_t* dev_to_sim, unsigned tiles)
 {
 	if(tiles == 0) return hipSuccess;
-	hipLaunchKernelGGL(external_fire_kernel, dim3(tiles), dim3(NEMO_TILE), 0, st, *b, flags, dev_to_sim);
+	if(b->direct.ring && b->direct.tiles != tiles) return hipErrorInvalidValue;
+	const unsigned blocks = tiles + b->direct.late_blocks;
+	hipLaunchKernelGGL(external_fire_kernel, dim3(blocks), dim3(NEMO_TILE), 0, st, *b, flags, dev_to_sim);
+	return hipGetLastError();
+}
+
+hipError_t nemo_launch_direct_rebuild(hipStream_t st, const nemo_hip_direct* r, size_t acc_pitch, const uint32_t* rowptr,
+		unsigned D, const uint64_t* fired_bits, size_t fired_words, uint64_t t0)
+{
+	if(!r->ring || !r->fcm || !r->delay || !r->arrivals || D == 0 || D > NEMO_MAX_DELAY || r->mask < D
+			|| (r->mask & (r->mask + 1)) || fired_words != size_t(r->tiles) * (NEMO_TILE / 64)) {
+		return hipErrorInvalidValue;
+	}
+	if(r->tiles == 0) return hipSuccess;
+	const size_t slots = size_t(r->mask) + 1;
+	hipError_t e = hipMemsetAsync(r->ring, 0, slots * 2 * acc_pitch * sizeof(int64_t), st);
+	if(e != hipSuccess) return e;
+	e = hipMemsetAsync(r->arrivals, 0, slots * r->tiles * sizeof(uint32_t), st);
+	if(e != hipSuccess) return e;
+	hipLaunchKernelGGL(direct_rebuild_kernel, dim3(r->tiles, D), dim3(NEMO_TILE), 0, st, *r, acc_pitch, rowptr, D,
+			fired_bits, fired_words, t0);
 	return hipGetLastError();
 }
 

@@ -4,13 +4,14 @@
  * An update kernel runs one block of NEMO_TILE threads per tile of its neuron
  * type, one neuron per thread, and every thread of a block calls
  *   UpdateLds& L = update_lds<CO>();            (CO: the launch carries propagate blocks)
+ *   if(!CO && b.direct.ring && direct_block(b, g, L)) return;
  *   h = load_history(b, ng, valid);
  *   gather_input(b, g, L);                      (block barriers inside)
  * or, in a launch of NEMO_COLAUNCH_BLOCK-thread blocks whose tile blocks keep
  * their other waves (colaunched_block<true>), those waves help to gather:
  *   if(!gather_input<NEMO_COLAUNCH_BLOCK>(b, g, L)) return;
  *   take_current(b, L.input, ng, E, I);         (valid threads)
- *   record_firing(b, L, ng, valid, fired, h);   (every thread; pushes the delay-1 events when asked)
+ *   record_firing<CO>(b, L, ng, valid, fired, h); (every thread; pushes the delay-1 events when asked)
  *   stdp_tile(b, L, ng, valid, h);              (every thread; barriers inside)
  */
 #ifndef NEMO_AMD_PLUGIN_DEVICE_H
@@ -30,9 +31,18 @@
 
 namespace nemo_dev {
 
+/* The step base.  No kernel that calls this changes the clock, so it is read
+ * as a constant: once per wave, where an ordinary load would be repeated
+ * after every store, each time in the launch's chain of dependent phases. */
+__device__ inline uint64_t clock_base(const nemo_hip_clock* clock)
+{
+	typedef const __attribute__((address_space(4))) nemo_hip_clock* constant_clock;
+	return reinterpret_cast<constant_clock>(reinterpret_cast<uintptr_t>(clock))->base_step;
+}
+
 __device__ inline uint64_t current_step(const nemo_hip_step_buffers& b)
 {
-	return b.clock->base_step + b.step_offset;
+	return clock_base(b.clock) + b.step_offset;
 }
 
 /* Exclusive scan of one value per thread over a block of THREADS threads;
@@ -122,6 +132,10 @@ constexpr unsigned GATHER_BUCKETS_MAX_EVENTS = GATHER_MARKED > GATHER_ILP_WIDE *
 	: GATHER_ILP_WIDE * NEMO_COLAUNCH_BLOCK;
 constexpr unsigned GATHER_BUCKETS = GATHER_BUCKETS_MAX_EVENTS / (1u << GATHER_SHIFT) + 2;
 
+/* Pieces (of up to 64 events) of fired rows that a block delivering directly
+ * lists in LDS at a time. */
+constexpr unsigned DIRECT_CHUNKS = 256;
+
 /* The LDS an update block uses: its tile's input sums, the gather's column
  * prefix, bases and buckets, and the per-tile STDP lists.  A kernel takes it
  * from update_lds<DYNAMIC>(): a static array, or -- in launches that also run
@@ -131,12 +145,21 @@ constexpr unsigned GATHER_BUCKETS = GATHER_BUCKETS_MAX_EVENTS / (1u << GATHER_SH
 struct UpdateLds {
 	TileInput input;
 	uint32_t pre[NEMO_MAX_BIN_BLOCKS + 1];
-	uint32_t base[NEMO_MAX_BIN_BLOCKS];
-	uint32_t bucket[GATHER_BUCKETS];
+	union {
+		uint32_t base[NEMO_MAX_BIN_BLOCKS];
+		uint2 chunk[DIRECT_CHUNKS];      /* direct delivery: pieces of the fired rows */
+	};
+	union {
+		uint32_t bucket[GATHER_BUCKETS];
+		struct {                         /* direct delivery: events per delay, pieces listed */
+			uint32_t count[64];
+			uint32_t chunks;
+		};
+	};
 	int32_t fn[128];
 	uint32_t rb[NEMO_TILE];
 	uint32_t pos[NEMO_TILE + 1];
-	uint2 push_rows[NEMO_TILE]; /* the tile's delay-1 rows, read ahead for push_delay1 */
+	uint2 push_rows[NEMO_TILE]; /* the tile's rows to push, read ahead */
 };
 
 template<bool DYNAMIC>
@@ -161,12 +184,60 @@ struct NoPrefetch {
 	__device__ void operator()() const {}
 };
 
-/* The delay-1 row of device index ng when the launch pushes (co.push), for
- * L.push_rows[threadIdx.x]: gather_input reads it ahead; a kernel that
- * records firing without gathering stores it itself. */
+/* The delay-1 row of device index ng when the launch pushes (co.push, or
+ * direct delivery), for L.push_rows[threadIdx.x]: gather_input reads it
+ * ahead; a kernel that records firing without gathering calls begin_push. */
 __device__ inline uint2 push_row(const nemo_hip_step_buffers& b, unsigned ng)
 {
-	return b.co.push ? b.co.push_rows[ng] : make_uint2(0, 0);
+	return b.direct.ring ? b.direct.first_rows[ng] : b.co.push ? b.co.push_rows[ng] : make_uint2(0, 0);
+}
+
+__device__ inline void begin_push(const nemo_hip_step_buffers& b, UpdateLds& L, unsigned ng)
+{
+	L.push_rows[threadIdx.x] = push_row(b, ng);
+	if(threadIdx.x < 64) L.count[threadIdx.x] = 0;
+	if(threadIdx.x == 64) L.chunks = 0;
+	__syncthreads();
+}
+
+/* The step's slot of the ring of a directly delivered network: the tile's
+ * sums are there already.  One round trip, where the binned gather takes
+ * three (table row, bins, sums).  The neuron's state (prefetch) is requested
+ * first, which needs no clock; the tile's event counter is touched last and
+ * without waiting for it. */
+template<typename Prefetch>
+__device__ inline void gather_direct(const nemo_hip_step_buffers& b, UpdateLds& L, unsigned tile, Prefetch prefetch)
+{
+	const nemo_hip_direct& r = b.direct;
+	const unsigned tid = threadIdx.x;
+	const unsigned ng = tile * NEMO_TILE + tid;
+	/* every argument the launch uses, loaded in one go: where each is used,
+	 * a cold line of the argument block at a time, they cost the chain a
+	 * round trip of the scalar cache each */
+	asm volatile("" ::"s"(r.ring), "s"(r.first_rows), "s"(r.fcm), "s"(r.delay), "s"(r.arrivals), "s"(r.events),
+			"s"(r.mask), "s"(r.tiles), "s"(b.acc_pitch), "s"(b.hist), "s"(b.hist_pitch), "s"(b.fired_bits),
+			"s"(b.fired_words), "s"(b.fbits), "s"(b.ext_current), "s"(b.fstim), "s"(b.debug_current),
+			"s"(b.stdp.rcm_ptr), "s"(clock_base(b.clock)));
+	const uint2 prow = push_row(b, ng);
+	prefetch();
+	const uint32_t slot = uint32_t(current_step(b)) & r.mask;
+	int64_t* acc = r.ring + size_t(slot) * 2 * b.acc_pitch;
+	const int64_t oe = acc[ng];
+	const int64_t oi = acc[b.acc_pitch + ng];
+	uint32_t* arrived = r.arrivals + size_t(slot) * r.tiles + tile;
+	const uint32_t n = tid == 0 ? *arrived : 0;
+	if(tid < 64) L.count[tid] = 0;
+	if(tid == 64) L.chunks = 0;
+	L.input.E[tid] = oe;
+	L.input.I[tid] = oi;
+	L.push_rows[tid] = prow;
+	if(oe) acc[ng] = 0;
+	if(oi) acc[b.acc_pitch + ng] = 0;
+	if(n) {
+		*arrived = 0;
+		atomicAdd(&r.events[ng >> 6], (unsigned long long)n);
+	}
+	__syncthreads(); /* count and chunks, for record_firing */
 }
 
 /* prefetch() is called once the tile's table row and accumulators are
@@ -190,6 +261,13 @@ __device__ inline bool gather_input(const nemo_hip_step_buffers& b, const nemo_h
 	const unsigned tid = threadIdx.x;
 	const bool lead = THREADS == NEMO_TILE || tid < NEMO_TILE; /* uniform per wave */
 	const unsigned tile = g.start / NEMO_TILE + blockIdx.x;
+	if constexpr(THREADS == NEMO_TILE) {
+		/* a launch that carries propagate blocks is never direct */
+		if(b.direct.ring) {
+			gather_direct(b, L, tile, prefetch);
+			return true;
+		}
+	}
 	const size_t parity = current_step(b) & 1;
 	int64_t* acc = b.acc + parity * 2 * b.acc_pitch;
 	const unsigned ng = tile * NEMO_TILE + tid;
@@ -327,7 +405,8 @@ __device__ inline float wfx_to_float(int64_t v, unsigned fbits)
 {
 	v = v > int64_t(INT32_MAX) ? int64_t(INT32_MAX) : v;
 	v = v < int64_t(INT32_MIN) ? int64_t(INT32_MIN) : v;
-	return float(int32_t(v)) / float(1u << fbits);
+	/* the product with the power of two is the quotient, exactly */
+	return float(int32_t(v)) * __uint_as_float((127u - fbits) << 23);
 }
 
 /* Excitatory and inhibitory current of neuron ng (thread threadIdx.x of the
@@ -452,6 +531,111 @@ __device__ inline void push_delay1(const nemo_hip_step_buffers& b, const UpdateL
 	if(lane == 0) atomicAdd(&a.block_events[NEMO_MAX_BIN_BLOCKS + (ng >> 6)], (unsigned long long)total);
 }
 
+/* Direct delivery of the rows (one per thread, [row.x, row.y), empty for
+ * neurons that did not fire) of tile `tile` that fired in step t, this
+ * block's part of them: every thread of a block of NEMO_TILE calls it, with
+ * count (64 entries) and *chunks in LDS cleared and seen by all; chunk is
+ * LDS too.  The chip does 23 G 64-bit atomics a second to random words,
+ * whatever their scope and place, so this pays while a step has few events; a
+ * bin round trip costs a network of any size its chain of dependent phases
+ * instead.
+ *
+ * What counts here is the length of the chain: a thread lists in LDS those
+ * pieces of its row, of 64 events, that are this part's, and after one
+ * barrier each wave takes every fourth of them, a lane an event, with no scan
+ * and no search (which took 1.3 us of a step's launch).  The parts agree on
+ * their pieces by neuron and piece number; the order within a part is free. */
+constexpr int DIRECT_ILP = 8;
+__device__ inline void deliver_direct(const nemo_hip_direct& r, size_t acc_pitch, uint2 row, uint64_t t, unsigned tile,
+		unsigned part, unsigned parts, uint2* chunk, uint32_t* chunks, uint32_t* count)
+{
+	constexpr unsigned WAVES = NEMO_TILE / 64;
+	const unsigned tid = threadIdx.x, lane = tid & 63;
+	/* pieces before, before + parts, ... of the row */
+	const uint32_t pieces = (row.y - row.x + 63) / 64;
+	const uint32_t before = parts == 1 ? 0 : (part + parts - tid % parts) % parts;
+	const uint32_t mine = before < pieces ? (pieces - before + parts - 1) / parts : 0;
+	const uint32_t first = mine ? atomicAdd(chunks, mine) : 0;
+	uint32_t total = 0;
+	for(uint32_t lo = 0;; lo += DIRECT_CHUNKS) {
+		for(uint32_t q = max(first, lo); q < min(first + mine, lo + DIRECT_CHUNKS); ++q) {
+			const uint32_t base = row.x + 64 * (before + (q - first) * parts);
+			chunk[q - lo] = make_uint2(base, min(64u, row.y - base));
+		}
+		__syncthreads();
+		total = *chunks;
+		const uint32_t here = min(total - min(total, lo), DIRECT_CHUNKS);
+		for(uint32_t c0 = tid / 64; c0 < here; c0 += DIRECT_ILP * WAVES) {
+			int2 ev[DIRECT_ILP];
+			unsigned d[DIRECT_ILP];
+			bool live[DIRECT_ILP];
+#pragma unroll
+			for(int u = 0; u < DIRECT_ILP; ++u) {
+				const uint32_t c = c0 + u * WAVES;
+				const uint2 piece = chunk[min(c, here - 1)];
+				live[u] = c < here && lane < piece.y;
+				ev[u] = make_int2(0, 0);
+				d[u] = 0;
+				if(live[u]) {
+					ev[u] = r.fcm[piece.x + lane];
+					d[u] = r.delay[piece.x + lane];
+				}
+			}
+#pragma unroll
+			for(int u = 0; u < DIRECT_ILP; ++u) {
+				if(!live[u]) continue;
+				const uint32_t slot = uint32_t(t + 1 + d[u]) & r.mask;
+				int64_t* dst = r.ring + (size_t(slot) * 2 + (ev[u].y >= 0 ? 0 : 1)) * acc_pitch + uint32_t(ev[u].x);
+				atomicAdd(reinterpret_cast<unsigned long long*>(dst), (unsigned long long)(int64_t)ev[u].y);
+				atomicAdd(&count[d[u]], 1u);
+			}
+		}
+		if(lo + DIRECT_CHUNKS >= total) break;
+		__syncthreads(); /* the list is rewritten */
+	}
+	if(!total) return;
+	__syncthreads();
+	if(tid < 64 && count[tid]) {
+		atomicAdd(&r.arrivals[size_t(uint32_t(t + 1 + tid) & r.mask) * r.tiles + tile], count[tid]);
+	}
+}
+
+/* In an update launch with direct delivery: run this block as one of those
+ * after the group's tiles and return true, or return false in a tile's block.
+ * The block reads a tile's firing of the step before from the bitmap and
+ * delivers its part of the events of delays 2.. (the delay-1 events went out
+ * with that step).  Beside the tiles' work, and split over parts, a tile that
+ * fires a lot does not hold the step up. */
+__device__ inline bool direct_block(const nemo_hip_step_buffers& b, const nemo_hip_neuron_group& g, UpdateLds& L)
+{
+	const unsigned tiles = (g.count + NEMO_TILE - 1) / NEMO_TILE;
+	if(blockIdx.x < tiles) return false;
+	const nemo_hip_direct& r = b.direct;
+	const uint64_t t = current_step(b);
+	if(t == 0) return true;
+	const unsigned k = blockIdx.x - tiles;
+	const unsigned tile = k / r.parts; /* of the network */
+	const unsigned tid = threadIdx.x;
+	const unsigned ng = tile * NEMO_TILE + tid;
+	const uint64_t word = b.fired_bits[((t - 1) & (NEMO_STEP_RING - 1)) * b.fired_words + (ng >> 6)];
+	const uint2 late = r.late_rows[ng];
+	if(tid < 64) L.count[tid] = 0;
+	if(tid == 64) L.chunks = 0;
+	__syncthreads();
+	const bool fired = (word >> (ng & 63)) & 1u;
+	deliver_direct(r, b.acc_pitch, fired ? late : make_uint2(0, 0), t - 1, tile, k % r.parts, r.parts, L.chunk, &L.chunks,
+			L.count);
+	return true;
+}
+
+/* Blocks of an update launch of a group: its tiles, then the propagate blocks
+ * it carries, or the blocks of direct delivery. */
+inline unsigned update_blocks(const nemo_hip_neuron_group* g, const nemo_hip_step_buffers* b)
+{
+	const unsigned tiles = (g->count + NEMO_TILE - 1) / NEMO_TILE;
+	return tiles + b->co.deliver_blocks + b->co.stdp_blocks + b->direct.late_blocks;
+}
+
 /* Store the shifted history (h as from load_history) and write the step's
  * firing bitmap. */
 __device__ inline void record_firing(const nemo_hip_step_buffers& b, unsigned ng, bool valid, bool fired, uint64_t h)
@@ -463,11 +647,20 @@ __device__ inline void record_firing(const nemo_hip_step_buffers& b, unsigned ng
 }
 
 /* The same in an update block whose input gather_input summed into L: with
- * co.push, also deliver the firing's delay-1 events. */
-__device__ inline void record_firing(const nemo_hip_step_buffers& b, const UpdateLds& L, unsigned ng, bool valid,
+ * co.push, or with direct delivery (never in a launch that carries propagate
+ * blocks, CO), also deliver the firing's delay-1 events. */
+template<bool CO>
+__device__ inline void record_firing(const nemo_hip_step_buffers& b, UpdateLds& L, unsigned ng, bool valid,
 		bool fired, uint64_t h)
 {
 	record_firing(b, ng, valid, fired, h);
+	if constexpr(!CO) {
+		if(b.direct.ring) {
+			deliver_direct(b.direct, b.acc_pitch, valid && fired ? L.push_rows[threadIdx.x] : make_uint2(0, 0),
+					current_step(b), ng / NEMO_TILE, 0, 1, L.chunk, &L.chunks, L.count);
+			return;
+		}
+	}
 	if(b.co.push) push_delay1(b, L, ng, valid, fired);
 }
 

@@ -76,6 +76,7 @@ hh_update(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 {
 	if(CO && nemo_dev::colaunched_block<true>(b, g)) return;
 	nemo_dev::UpdateLds& L = nemo_dev::update_lds<CO>();
+	if(!CO && b.direct.ring && nemo_dev::direct_block(b, g, L)) return;
 	if(!nemo_dev::gather_input<CO ? NEMO_COLAUNCH_BLOCK : NEMO_TILE>(b, g, L)) return; /* helpers end here */
 	const unsigned nl = blockIdx.x * NEMO_UPDATE_BLOCK + threadIdx.x;
 	const bool valid = nl < g.count;
@@ -112,7 +113,7 @@ hh_update(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 		s[3 * P + nl] = h;
 		s[4 * P + nl] = dir;
 	}
-	nemo_dev::record_firing(b, L, nn, valid, fired, hist);
+	nemo_dev::record_firing<CO>(b, L, nn, valid, fired, hist);
 	nemo_dev::stdp_tile(b, L, nn, valid, hist);
 }
 
@@ -125,6 +126,7 @@ hh_input(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 {
 	if(CO && nemo_dev::colaunched_block<true>(b, g)) return;
 	nemo_dev::UpdateLds& L = nemo_dev::update_lds<CO>();
+	if(!CO && b.direct.ring && nemo_dev::direct_block(b, g, L)) return;
 	if(!nemo_dev::gather_input<CO ? NEMO_COLAUNCH_BLOCK : NEMO_TILE>(b, g, L)) return; /* helpers end here */
 	const unsigned nl = blockIdx.x * NEMO_UPDATE_BLOCK + threadIdx.x;
 	if(nl < g.count) {
@@ -229,10 +231,10 @@ hh_record(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 	const bool valid = nl < g.count;
 	const unsigned nn = g.start + nl;
 	const uint64_t hist = nemo_dev::load_history(b, nn, valid);
-	L.push_rows[threadIdx.x] = nemo_dev::push_row(b, nn);
+	nemo_dev::begin_push(b, L, nn);
 	bool fired = false;
 	if(valid) fired = g.scratch[SCR_FIRED * g.pitch + nl] != 0.0f || nemo_dev::stimulated(b, nn);
-	nemo_dev::record_firing(b, L, nn, valid, fired, hist);
+	nemo_dev::record_firing<false>(b, L, nn, valid, fired, hist);
 	nemo_dev::stdp_tile(b, L, nn, valid, hist);
 }
 
@@ -243,8 +245,7 @@ hip_update_neurons(hipStream_t stream, const nemo_hip_neuron_group* g, const nem
 {
 	if(g->count == 0) return hipSuccess;
 	const unsigned tiles = (g->count + NEMO_UPDATE_BLOCK - 1) / NEMO_UPDATE_BLOCK;
-	/* the group's tiles, then the propagate blocks the launch carries */
-	const unsigned blocks = tiles + b->co.deliver_blocks + b->co.stdp_blocks;
+	const unsigned blocks = nemo_dev::update_blocks(g, b);
 	if(!g->scratch) {
 		if(b->co.deliver_blocks || b->co.stdp_blocks) {
 			hipExtLaunchKernelGGL(hh_update<true>, dim3(blocks), dim3(NEMO_COLAUNCH_BLOCK), b->co.lds_bytes, stream,

@@ -31,6 +31,7 @@ izhikevich_update(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 {
 	if(CO && nemo_dev::colaunched_block<true>(b, g)) return;
 	nemo_dev::UpdateLds& L = nemo_dev::update_lds<CO>();
+	if(!CO && b.direct.ring && nemo_dev::direct_block(b, g, L)) return;
 	const unsigned nl = blockIdx.x * NEMO_UPDATE_BLOCK + threadIdx.x;
 	const bool valid = nl < g.count;
 	const unsigned ng = g.start + nl;
@@ -86,7 +87,7 @@ izhikevich_update(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 		g.state[STATE_U * P + nl] = u;
 		g.state[STATE_V * P + nl] = v;
 	}
-	nemo_dev::record_firing(b, L, ng, valid, fired, h);
+	nemo_dev::record_firing<CO>(b, L, ng, valid, fired, h);
 	nemo_dev::stdp_tile(b, L, ng, valid, h);
 }
 
@@ -96,9 +97,7 @@ extern "C" hipError_t
 hip_update_neurons(hipStream_t stream, const nemo_hip_neuron_group* g, const nemo_hip_step_buffers* b)
 {
 	if(g->count == 0) return hipSuccess;
-	/* the group's tiles, then the propagate blocks the launch carries */
-	const unsigned blocks = (g->count + NEMO_UPDATE_BLOCK - 1) / NEMO_UPDATE_BLOCK + b->co.deliver_blocks
-		+ b->co.stdp_blocks;
+	const unsigned blocks = nemo_dev::update_blocks(g, b);
 	if(b->co.deliver_blocks || b->co.stdp_blocks) {
 		hipExtLaunchKernelGGL(izhikevich_update<true>, dim3(blocks), dim3(NEMO_COLAUNCH_BLOCK), b->co.lds_bytes, stream,
 				b->time_start, b->time_stop, 0, *g, *b);

@@ -218,7 +218,7 @@ __global__ void NEMO_UPDATE_BOUNDS(CO)
 kuramoto_update(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 {
 	const unsigned before = (g.count + NEMO_UPDATE_BLOCK - 1) / NEMO_UPDATE_BLOCK + b.co.deliver_blocks
-		+ b.co.stdp_blocks;
+		+ b.co.stdp_blocks + b.direct.late_blocks;
 	if(blockIdx.x >= before) {
 		const unsigned nl = group_index<L>(blockIdx.x - before);
 		if(nl < g.count) kuramoto_group<L>(g, b, nl, false);
@@ -226,11 +226,12 @@ kuramoto_update(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 	}
 	if(CO && nemo_dev::colaunched_block(b, g)) return;
 	nemo_dev::UpdateLds& U = nemo_dev::update_lds<CO>();
+	if(!CO && b.direct.ring && nemo_dev::direct_block(b, g, U)) return;
 	const unsigned nl = blockIdx.x * NEMO_UPDATE_BLOCK + threadIdx.x;
 	const bool valid = nl < g.count;
 	const unsigned ng = g.start + nl;
 	const uint64_t hist = nemo_dev::load_history(b, ng, valid);
-	nemo_dev::record_firing(b, U, ng, valid, false, hist);
+	nemo_dev::record_firing(b, ng, valid, false, hist); /* nothing to push */
 	nemo_dev::stdp_tile(b, U, ng, valid, hist);
 }
 
@@ -258,11 +259,12 @@ kuramoto_record(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 {
 	if(CO && nemo_dev::colaunched_block(b, g)) return;
 	nemo_dev::UpdateLds& L = nemo_dev::update_lds<CO>();
+	if(!CO && b.direct.ring && nemo_dev::direct_block(b, g, L)) return;
 	const unsigned nl = blockIdx.x * NEMO_UPDATE_BLOCK + threadIdx.x;
 	const bool valid = nl < g.count;
 	const unsigned ng = g.start + nl;
 	const uint64_t hist = nemo_dev::load_history(b, ng, valid);
-	nemo_dev::record_firing(b, L, ng, valid, false, hist);
+	nemo_dev::record_firing(b, ng, valid, false, hist);
 	nemo_dev::stdp_tile(b, L, ng, valid, hist);
 }
 
@@ -310,10 +312,9 @@ static unsigned lanes_for(const nemo_hip_neuron_group* g, unsigned n)
 template<unsigned L>
 static hipError_t launch_update(hipStream_t stream, const nemo_hip_neuron_group* g, const nemo_hip_step_buffers* b)
 {
-	const unsigned tiles = (g->count + NEMO_UPDATE_BLOCK - 1) / NEMO_UPDATE_BLOCK;
-	/* the group's tiles, then the propagate blocks the launch carries, then
-	 * the oscillators */
-	const unsigned before = tiles + b->co.deliver_blocks + b->co.stdp_blocks;
+	/* the group's tiles and the blocks the launch carries, then the
+	 * oscillators */
+	const unsigned before = nemo_dev::update_blocks(g, b);
 	if(b->co.deliver_blocks || b->co.stdp_blocks) {
 		const unsigned per = NEMO_COLAUNCH_BLOCK / L;
 		hipExtLaunchKernelGGL((kuramoto_update<true, L>), dim3(before + (g->count + per - 1) / per),
@@ -348,7 +349,7 @@ hip_update_neurons(hipStream_t stream, const nemo_hip_neuron_group* g, const nem
 	}
 	if(!g->scratch || !g->level_idx || g->levels < 1) return hipErrorInvalidValue;
 	const unsigned tiles = (g->count + NEMO_UPDATE_BLOCK - 1) / NEMO_UPDATE_BLOCK;
-	const unsigned blocks = tiles + b->co.deliver_blocks + b->co.stdp_blocks;
+	const unsigned blocks = nemo_dev::update_blocks(g, b);
 	const bool co = b->co.deliver_blocks || b->co.stdp_blocks;
 	hipExtLaunchKernelGGL(kuramoto_keep_next, dim3(tiles), dim3(NEMO_UPDATE_BLOCK), 0, stream, b->time_start,
 			nullptr, 0, *g, *b);

@@ -627,7 +627,7 @@ __device__ inline bool colaunched_block(const nemo_hip_step_buffers& b, const ne
 	unsigned char* lds = reinterpret_cast<unsigned char*>(colaunch_lds);
 	const unsigned k = blockIdx.x - tiles;
 	const nemo_propagate_args& a = b.co.args;
-	const uint64_t t = a.clock->base_step + a.step_offset;
+	const uint64_t t = clock_base(a.clock) + a.step_offset;
 	if(k < b.co.deliver_blocks) {
 		deliver_block<NEMO_COLAUNCH_BLOCK, CARRIED_EVENT_ILP>(a, t, k, lds);
 	} else {

@@ -59,3 +59,84 @@ def test_kuramoto_lane_groups_match_oracle(n, degrees, dmax):
     for t in range(12):
         assert ref.step() == hip.step() == []
         assert same_f32(ref.neuron_states(0), hip.neuron_states(0)), t
+
+
+# --------------------------------------------------- direct delivery
+def stdp(conf):
+    pre, post = gen.stdp_exp_function(0.1, -0.12, 20.0, 20)
+    conf.set_stdp_function(pre, post, 0.0, 10.0, 0.0, -10.0)
+    return conf
+
+
+def pair(spec, with_stdp):
+    sims = []
+    for api in (oa, nemo_amd):
+        net = api.Network()
+        spec.load(net)
+        conf = api.Configuration()
+        sims.append(api.Simulation(net, stdp(conf) if with_stdp else conf))
+    return sims
+
+
+@pytest.mark.parametrize("binned", [False, True])
+@pytest.mark.parametrize("n,m,dmax", [
+    (1, 3, 1),        # a ring of two slots, self synapses
+    (255, 40, 1),
+    (257, 60, 31),    # 32 slots, every delay of them used
+    (700, 30, 32),    # 64 slots
+    (513, 300, 43),   # rows of one neuron longer than a block's threads
+])
+def test_small_network_delivery_matches_oracle(n, m, dmax, binned):
+    """Rasters, events, potentials and learned weights against the oracle over
+    runs, single steps, a step in which every neuron fires (each block delivers
+    thousands of events), applyStdp with events under way, and a shape set and
+    left in between."""
+    spec = gen.random_izhikevich(n, m, dmax=dmax, seed=n + dmax, stdp=True)
+    ref, hip = pair(spec, True)
+    if binned:
+        hip.launch_shape = hip.launch_shape
+
+    def advance(steps):
+        before = ref.delivered_events()
+        want = [ref.step() for _ in range(steps)]
+        counts, fired, events = hip.run(steps)
+        assert counts.tolist() == [len(f) for f in want]
+        assert fired.tolist() == [i for f in want for i in f]
+        assert events == ref.delivered_events() - before
+
+    everyone = list(range(n))
+    advance(70)
+    assert ref.step(everyone) == hip.step(everyone)
+    advance(3)
+    for sim in (ref, hip):
+        sim.apply_stdp(1.0)
+    advance(dmax + 5)
+    if not binned:
+        hip.launch_shape = hip.launch_shape  # the binned delivery from here on, with events under way
+    assert ref.step(everyone) == hip.step(everyone)
+    advance(66)
+    ref.apply_stdp(-0.5)
+    hip.apply_stdp(-0.5)
+    assert np.array_equal(ref.fixed_weights(spec.synapse_count), hip.fixed_weights())
+    for var in (0, 1):
+        assert same_f32(ref.neuron_states(var), hip.neuron_states(var))
+
+
+def test_maximum_delay_and_propagate_with_steps_in_between():
+    """Delays up to 64 (a ring of 128 slots), and Brian's propagate before,
+    between and after steps: its events stay under way for the steps, and the
+    input of a step it passed over is not left for a later one."""
+    spec = gen.random_izhikevich(600, 80, dmax=64, seed=9)
+    ref, hip = pair(spec, False)
+    rng = np.random.default_rng(2)
+    for block in range(4):
+        for _ in range(5 if block else 150):
+            f = sorted(rng.choice(600, 40, replace=False).tolist())
+            (er, ir), (eh, ih) = ref.propagate(f), hip.propagate(f)
+            assert same_f32(er, eh) and same_f32(ir, ih)
+        for _ in range(7):
+            assert ref.step() == hip.step()
+        want = [ref.step() for _ in range(130)]
+        counts, fired, _ = hip.run(130)
+        assert counts.tolist() == [len(f) for f in want]
+        assert fired.tolist() == [i for f in want for i in f]
