@@ -53,21 +53,37 @@ NEMO_HD double fma_d(double a, double b, double c) { return __builtin_fma(a, b, 
 
 /* ---------------------------------------------------------------- logf */
 
+/* (1/c, log c) for the 16 subintervals of [0x3f330000, 2*0x3f330000) */
+#define NEMO_LOGF_INVC { \
+		0x1.661ec79f8f3bep+0, 0x1.571ed4aaf883dp+0, 0x1.49539f0f010bp+0, 0x1.3c995b0b80385p+0, \
+		0x1.30d190c8864a5p+0, 0x1.25e227b0b8eap+0, 0x1.1bb4a4a1a343fp+0, 0x1.12358f08ae5bap+0, \
+		0x1.0953f419900a7p+0, 0x1p+0, 0x1.e608cfd9a47acp-1, 0x1.ca4b31f026aap-1, \
+		0x1.b2036576afce6p-1, 0x1.9c2d163a1aa2dp-1, 0x1.886e6037841edp-1, 0x1.767dcf5534862p-1, \
+}
+#define NEMO_LOGF_LOGC { \
+		-0x1.57bf7808caadep-2, -0x1.2bef0a7c06ddbp-2, -0x1.01eae7f513a67p-2, -0x1.b31d8a68224e9p-3, \
+		-0x1.6574f0ac07758p-3, -0x1.1aa2bc79c81p-3, -0x1.a4e76ce8c0e5ep-4, -0x1.1973c5a611cccp-4, \
+		-0x1.252f438e10c1ep-5, 0x0p+0, 0x1.aa5aa5df25984p-5, 0x1.c5e53aa362eb4p-4, \
+		0x1.526e57720db08p-3, 0x1.bc2860d22477p-3, 0x1.1058bc8a07ee1p-2, 0x1.4043057b6ee09p-2, \
+}
+
+/* Entry i (i < 16) of the tables. */
+NEMO_HD double logf_invc(unsigned i)
+{
+	const double T[16] = NEMO_LOGF_INVC;
+	return T[i % 16];
+}
+
+NEMO_HD double logf_logc(unsigned i)
+{
+	const double T[16] = NEMO_LOGF_LOGC;
+	return T[i % 16];
+}
+
 NEMO_HD float logf_exact(float x)
 {
-	/* (1/c, log c) for the 16 subintervals of [0x3f330000, 2*0x3f330000) */
-	const double invc[16] = {
-		0x1.661ec79f8f3bep+0, 0x1.571ed4aaf883dp+0, 0x1.49539f0f010bp+0, 0x1.3c995b0b80385p+0,
-		0x1.30d190c8864a5p+0, 0x1.25e227b0b8eap+0, 0x1.1bb4a4a1a343fp+0, 0x1.12358f08ae5bap+0,
-		0x1.0953f419900a7p+0, 0x1p+0, 0x1.e608cfd9a47acp-1, 0x1.ca4b31f026aap-1,
-		0x1.b2036576afce6p-1, 0x1.9c2d163a1aa2dp-1, 0x1.886e6037841edp-1, 0x1.767dcf5534862p-1,
-	};
-	const double logc[16] = {
-		-0x1.57bf7808caadep-2, -0x1.2bef0a7c06ddbp-2, -0x1.01eae7f513a67p-2, -0x1.b31d8a68224e9p-3,
-		-0x1.6574f0ac07758p-3, -0x1.1aa2bc79c81p-3, -0x1.a4e76ce8c0e5ep-4, -0x1.1973c5a611cccp-4,
-		-0x1.252f438e10c1ep-5, 0x0p+0, 0x1.aa5aa5df25984p-5, 0x1.c5e53aa362eb4p-4,
-		0x1.526e57720db08p-3, 0x1.bc2860d22477p-3, 0x1.1058bc8a07ee1p-2, 0x1.4043057b6ee09p-2,
-	};
+	const double invc[16] = NEMO_LOGF_INVC;
+	const double logc[16] = NEMO_LOGF_LOGC;
 	const double A0 = -0x1.00ea348b88334p-2, A1 = 0x1.5575b0be00b6ap-2, A2 = -0x1.ffffef20a4123p-2;
 	const double Ln2 = 0x1.62e42fefa39efp-1;
 
@@ -95,6 +111,33 @@ NEMO_HD float logf_exact(float x)
 	y = fma_d(A0, r2, y);
 	y = fma_d(y, r2, y0 + r);
 	return float(y);
+}
+
+/* logf of x = 0 or 2^-24 <= x <= 1, what the Box-Muller transform passes it
+ * (1 minus a multiple of 2^-32 rounded to float, in [0, 1]), without a branch:
+ * no subnormal, infinite or negative argument needs normalising, and the two
+ * special values are selected at the end.  The table entries come from
+ * entry(i, &invc, &logc), i < 16: device code keeps them in the lanes of the
+ * wave, where a load would add a round trip to the neuron update's chain. */
+template<typename Entry>
+NEMO_HD float logf_unit(float x, Entry entry)
+{
+	const double A0 = -0x1.00ea348b88334p-2, A1 = 0x1.5575b0be00b6ap-2, A2 = -0x1.ffffef20a4123p-2;
+	const double Ln2 = 0x1.62e42fefa39efp-1;
+	const uint32_t ix = asuint(x);
+	const uint32_t tmp = ix - 0x3f330000u;
+	double invc, logc;
+	entry((tmp >> (23 - 4)) % 16, &invc, &logc);
+	const int k = int32_t(tmp) >> 23;
+	const double z = double(asfloat(ix - (tmp & 0xff800000u)));
+	const double r = fma_d(z, invc, -1.0);
+	const double y0 = fma_d(double(k), Ln2, logc);
+	const double r2 = r * r;
+	double y = fma_d(A1, r, A2);
+	y = fma_d(A0, r2, y);
+	y = fma_d(y, r2, y0 + r);
+	const float main = x == 1.0f ? 0.0f : float(y);
+	return x == 0.0f ? -__builtin_inff() : main;
 }
 
 /* ---------------------------------------------------------------- sinf */
@@ -143,6 +186,34 @@ NEMO_HD float sinf_exact(float y)
 		return sinf_poly(x * s, x * x, (n & 2) ? 1 : 0, n);
 	}
 	return __builtin_nanf("");
+}
+
+/* sinf of 0 <= y < 8 without a branch: every such y takes the route of the
+ * arguments from 0.75 up (below, n is 0 and the reduction leaves y as it is;
+ * the polynomial rounds to y itself where the routine returns it untouched),
+ * and the sine and cosine polynomials, which have the same shape, share their
+ * operations with the coefficients selected by quadrant. */
+NEMO_HD float sinf_turn(float y)
+{
+	const double hpi_inv = 0x1.45F306DC9C883p+23; /* 2/pi * 2^24 */
+	const double hpi = 0x1.921FB54442D18p0;       /* pi/2 */
+	const double S1 = -0x1.555545995a603p-3, S2 = 0x1.1107605230bc4p-7, S3 = -0x1.994eb3774cf24p-13;
+	const double C0 = 0x1p0, C1 = -0x1.ffffffd0c621cp-2, C2 = 0x1.55553e1068f19p-5, C3 = -0x1.6c087e89a359dp-10,
+			C4 = 0x1.99343027bf8c3p-16;
+	const double yd = double(y);
+	const int n = (int32_t(yd * hpi_inv) + 0x800000) >> 24;
+	double x = fma_d(-double(n), hpi, yd);
+	const double x2 = x * x;
+	const bool cosine = n & 1;
+	/* the sign of {1, -1, -1, 1} on the sine's argument, of {1, 1, -1, -1} on
+	 * the cosine's coefficients */
+	x = (n & 3) == 1 || (n & 3) == 2 ? -x : x;
+	const double sg = n & 2 ? -1.0 : 1.0;
+	const double base = cosine ? fma_d(x2, sg * C1, sg * C0) : x;
+	const double high = fma_d(x2, cosine ? sg * C4 : S3, cosine ? sg * C3 : S2);
+	const double x3 = cosine ? x2 * x2 : x * x2; /* x^4, x^3 */
+	const double x5 = x3 * x2;                   /* x^6, x^5 */
+	return float(fma_d(x5, high, fma_d(x3, cosine ? sg * C2 : S1, base)));
 }
 
 /* ---------------------------------------------------------------- expf */

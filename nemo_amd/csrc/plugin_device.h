@@ -180,7 +180,7 @@ __device__ inline UpdateLds& update_lds()
  * atomics does not matter).  The whole table row is read: columns whose
  * window does not hold the tile keep a zero count, and reading them costs
  * less than a dependent load of the tile's column range. */
-struct NoPrefetch {
+struct Nothing {
 	__device__ void operator()() const {}
 };
 
@@ -205,8 +205,9 @@ __device__ inline void begin_push(const nemo_hip_step_buffers& b, UpdateLds& L, 
  * three (table row, bins, sums).  The neuron's state (prefetch) is requested
  * first, which needs no clock; the tile's event counter is touched last and
  * without waiting for it. */
-template<typename Prefetch>
-__device__ inline void gather_direct(const nemo_hip_step_buffers& b, UpdateLds& L, unsigned tile, Prefetch prefetch)
+template<typename Prefetch, typename Meanwhile>
+__device__ inline void gather_direct(const nemo_hip_step_buffers& b, UpdateLds& L, unsigned tile, Prefetch prefetch,
+		Meanwhile meanwhile)
 {
 	const nemo_hip_direct& r = b.direct;
 	const unsigned tid = threadIdx.x;
@@ -228,6 +229,7 @@ __device__ inline void gather_direct(const nemo_hip_step_buffers& b, UpdateLds& 
 	const uint32_t n = tid == 0 ? *arrived : 0;
 	if(tid < 64) L.count[tid] = 0;
 	if(tid == 64) L.chunks = 0;
+	meanwhile();
 	L.input.E[tid] = oe;
 	L.input.I[tid] = oi;
 	L.push_rows[tid] = prow;
@@ -242,7 +244,12 @@ __device__ inline void gather_direct(const nemo_hip_step_buffers& b, UpdateLds& 
 
 /* prefetch() is called once the tile's table row and accumulators are
  * requested: the loads it issues (the model's state, say) queue behind them,
- * so that waiting for the table does not wait for them too.
+ * so that waiting for the table does not wait for them too.  meanwhile()
+ * runs in the tile's own threads, all of them, while the ring's slot is on
+ * its way (direct delivery) or the block's other waves still sum events: work
+ * on what prefetch loaded that needs no input, such as a neuron's noise.
+ * Beside the events' loads its registers would take the update from 58 VGPRs
+ * to 72, before them it would hold the gather up.
  *
  * THREADS threads of the block take part: the tile's NEMO_TILE (one per
  * neuron, which alone read the table row, the accumulators and, through
@@ -250,9 +257,9 @@ __device__ inline void gather_direct(const nemo_hip_step_buffers& b, UpdateLds& 
  * threads, helpers that only load and sum events, so that a tile of up to
  * 3072 events (GATHER_ILP_WIDE per thread) takes one round of loads.  Returns false for
  * the helpers, which take no further part in the step. */
-template<unsigned THREADS = NEMO_TILE, typename Prefetch = NoPrefetch>
+template<unsigned THREADS = NEMO_TILE, typename Prefetch = Nothing, typename Meanwhile = Nothing>
 __device__ inline bool gather_input(const nemo_hip_step_buffers& b, const nemo_hip_neuron_group& g, UpdateLds& L,
-		Prefetch prefetch = Prefetch())
+		Prefetch prefetch = Prefetch(), Meanwhile meanwhile = Meanwhile())
 {
 	static_assert(THREADS % 64 == 0 && THREADS >= NEMO_TILE, "whole waves beyond the tile");
 	TileInput& in = L.input;
@@ -264,7 +271,7 @@ __device__ inline bool gather_input(const nemo_hip_step_buffers& b, const nemo_h
 	if constexpr(THREADS == NEMO_TILE) {
 		/* a launch that carries propagate blocks is never direct */
 		if(b.direct.ring) {
-			gather_direct(b, L, tile, prefetch);
+			gather_direct(b, L, tile, prefetch, meanwhile);
 			return true;
 		}
 	}
@@ -308,6 +315,7 @@ __device__ inline bool gather_input(const nemo_hip_step_buffers& b, const nemo_h
 		if(oi) acc[b.acc_pitch + ng] = 0;
 	}
 	if(B == 0) {
+		if(lead) meanwhile();
 		__syncthreads();
 		return lead;
 	}
@@ -395,6 +403,7 @@ __device__ inline bool gather_input(const nemo_hip_step_buffers& b, const nemo_h
 		}
 		if(!marked) __syncthreads(); /* the buckets are rewritten by the next batch */
 	}
+	if(lead) meanwhile();
 	__syncthreads();
 	return lead;
 }
@@ -453,6 +462,34 @@ __device__ inline float nrand(uint4& s)
 	float b = float(urand(s)) * 0.00000000023283064365386962890625f;
 	float r = __builtin_sqrtf(-2.0f * nemo_math::logf_exact(1.0f - b));
 	return nemo_math::sinf_exact(a) * r;
+}
+
+/* The same for every lane of a wave at once, all of them active, without a
+ * branch or a load: lane i holds entry i % 16 of logf's tables (noise_table,
+ * loaded ahead with the neuron's state), which the lanes look up by shuffle.
+ * As a chain of branches over both routes of sinf and logf's special cases,
+ * with the table in memory, the deviate took 0.9 us of a step's launch. */
+struct NoiseTable {
+	double invc, logc;
+};
+
+__device__ inline NoiseTable noise_table()
+{
+	NoiseTable t;
+	t.invc = nemo_math::logf_invc(threadIdx.x & 15);
+	t.logc = nemo_math::logf_logc(threadIdx.x & 15);
+	return t;
+}
+
+__device__ inline float nrand_wave(uint4& s, const NoiseTable& t)
+{
+	const float a = float(urand(s)) * 1.4629180792671596810513378043098e-9f;
+	const float b = float(urand(s)) * 0.00000000023283064365386962890625f;
+	const float l = nemo_math::logf_unit(1.0f - b, [&t](unsigned i, double* invc, double* logc) {
+		*invc = __shfl(t.invc, int(i));
+		*logc = __shfl(t.logc, int(i));
+	});
+	return nemo_math::sinf_turn(a) * __builtin_sqrtf(-2.0f * l);
 }
 
 /* Write the tile's words of the step's firing bitmap (one ballot per wave;

@@ -42,6 +42,9 @@ izhikevich_update(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 	float sigma = 0.0f, a = 0.0f, bb = 0.0f, c = 0.0f, d = 0.0f, u = 0.0f, v = 0.0f;
 	uint4 s = make_uint4(0, 0, 0, 0);
 	uint64_t h = 0;
+	nemo_dev::NoiseTable table;
+	bool noisy = false;
+	float noise = 0.0f;
 	/* in a carrying launch the block's other waves help with the gather */
 	if(!nemo_dev::gather_input<CO ? NEMO_COLAUNCH_BLOCK : NEMO_TILE>(b, g, L, [&]() {
 		if(valid) {
@@ -52,8 +55,16 @@ izhikevich_update(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 			d = g.param[PARAM_D * P + nl];
 			u = g.state[STATE_U * P + nl];
 			v = g.state[STATE_V * P + nl];
-			if(g.rng) s = reinterpret_cast<const uint4*>(g.rng)[nl];
+			s = reinterpret_cast<const uint4*>(g.rng)[nl]; /* Izhikevich.ini: rng.normal */
 			h = nemo_dev::load_history(b, ng, true);
+		}
+		table = nemo_dev::noise_table();
+	}, [&]() {
+		/* the step's noise needs no input: drawn while that is gathered */
+		noisy = valid && sigma != 0.0f;
+		if(__any(noisy)) {
+			noise = sigma * nemo_dev::nrand_wave(s, table);
+			if(noisy) reinterpret_cast<uint4*>(g.rng)[nl] = s;
 		}
 	}))
 		return;
@@ -64,10 +75,7 @@ izhikevich_update(nemo_hip_neuron_group g, nemo_hip_step_buffers b)
 		nemo_dev::take_current(b, L.input, ng, E, In);
 		float I = E + In + nemo_dev::take_external(b, ng);
 
-		if(sigma != 0.0f) {
-			I += sigma * nemo_dev::nrand(s);
-			reinterpret_cast<uint4*>(g.rng)[nl] = s;
-		}
+		if(noisy) I += noise;
 
 #pragma unroll
 		for(int t = 0; t < 4; ++t) {
