@@ -406,7 +406,7 @@ hipError_t nemo_launch_stdp_snapshot(hipStream_t st, const nemo_propagate_args* 
 size_t nemo_colaunch_lds_bytes(unsigned max_window, unsigned bin_capacity, int delivery)
 {
 	/* the update blocks of the launch take their LDS from the same buffer */
-	return std::max(nemo_dev::PropagateLds<NEMO_COLAUNCH_BLOCK, nemo_dev::CARRIED_EVENT_ILP>::bytes(delivery != 0,
+	return std::max(nemo_dev::PropagateLds<NEMO_COLAUNCH_BLOCK>::bytes(delivery != 0,
 					bin_capacity, max_window),
 			sizeof(nemo_dev::UpdateLds));
 }

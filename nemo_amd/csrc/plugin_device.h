@@ -45,6 +45,37 @@ __device__ inline uint64_t current_step(const nemo_hip_step_buffers& b)
 	return clock_base(b.clock) + b.step_offset;
 }
 
+/* Inclusive sum over the lanes of a wave, all of them active: within rows of
+ * 16 by DPP shifts, then each row's last lane broadcast into the rows after
+ * it (row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3).  Six
+ * additions, where shuffles take six round trips of the LDS crossbar. */
+__device__ inline uint32_t wave_inclusive_sum(uint32_t x)
+{
+	int v = int(x);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+	return uint32_t(v);
+}
+
+/* Room for x entries per lane in a list that the block's waves fill in
+ * whatever order they come: *counter (LDS) grows by the wave's total, the
+ * lane's entries start where returned.  Every lane of the wave calls it. */
+__device__ inline uint32_t wave_append(uint32_t* counter, uint32_t x)
+{
+	const uint32_t upto = wave_inclusive_sum(x);
+	const uint32_t all = uint32_t(__builtin_amdgcn_readlane(int(upto), 63));
+	uint32_t base = 0;
+	if(all) {
+		if((threadIdx.x & 63) == 0) base = atomicAdd(counter, all);
+		base = uint32_t(__builtin_amdgcn_readfirstlane(int(base)));
+	}
+	return base + upto - x;
+}
+
 /* Exclusive scan of one value per thread over a block of THREADS threads;
  * returns the thread's prefix and sets *total. */
 template<unsigned THREADS = NEMO_TILE>
@@ -53,12 +84,7 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t x, uint32_t* total)
 	__shared__ uint32_t s_wave[THREADS / 64];
 	const unsigned lane = threadIdx.x & 63;
 	const unsigned wave = threadIdx.x >> 6;
-	uint32_t v = x;
-#pragma unroll
-	for(int o = 1; o < 64; o <<= 1) {
-		const uint32_t y = __shfl_up(v, o);
-		if(int(lane) >= o) v += y;
-	}
+	const uint32_t v = wave_inclusive_sum(x);
 	if(lane == 63) s_wave[wave] = v;
 	__syncthreads();
 	uint32_t before = 0, all = 0;
@@ -530,13 +556,8 @@ __device__ inline void push_delay1(const nemo_hip_step_buffers& b, const UpdateL
 		rb = r.x;
 		len = r.y - r.x;
 	}
-	uint32_t incl = len;
-#pragma unroll
-	for(int o = 1; o < 64; o <<= 1) {
-		const uint32_t y = __shfl_up(incl, o);
-		if(int(lane) >= o) incl += y;
-	}
-	const uint32_t total = __shfl(incl, 63);
+	const uint32_t incl = wave_inclusive_sum(len);
+	const uint32_t total = uint32_t(__builtin_amdgcn_readlane(int(incl), 63));
 	const uint32_t excl = incl - len;
 	int64_t* acc = a.acc + ((current_step(b) + 1) & 1) * 2 * a.acc_pitch;
 	for(uint32_t e0 = 0; e0 < total; e0 += 64 * PUSH_ILP) {

@@ -30,9 +30,8 @@ constexpr int EVENT_ILP = 8;
 /* The delivery blocks an update launch carries (overlap 3) keep 6: that
  * launch is held to 72 VGPRs (NEMO_COLAUNCH_WAVES), so that beside three of
  * its blocks a CU's SIMDs still hold one wave each of an STDP batch block
- * (NEMO_STDP_BATCH_BLOCK threads, 80 VGPRs); with 8 the launch needs 78, and
- * a batch block beside it leaves a CU room for one of its blocks instead of
- * three, so that the blocks of the steps beside a batch wait for each other */
+ * (NEMO_STDP_BATCH_BLOCK threads, 80 VGPRs).  8 would take all 72 and gains
+ * nothing (19.62 against 19.65 us a step at 100k x 1000 with STDP) */
 constexpr int CARRIED_EVENT_ILP = 6;
 /* independent global loads per thread in the synapse loop of the STDP batch
  * beside the steps, held to 80 VGPRs (NEMO_STDP_BATCH_WAVES waves per SIMD),
@@ -43,44 +42,38 @@ constexpr int STDP_FLUSH_ILP = 8;
 constexpr unsigned SORT_REGS = 8;
 
 /* LDS of a propagate block of THREADS threads, carved from one buffer:
- * staged events (bin capacity), per-window-tile counts and cursors, the
- * bitmap words of a batch with their prefix, and the fired rows of a chunk
- * with their event prefix.  An STDP block uses the start of the same buffer
- * for its weight-change table, row bases and prefix. */
-template<unsigned THREADS, int EV_ILP = EVENT_ILP>
+ * staged events (bin capacity), the fired rows of a batch (ROWS at a time)
+ * and the pieces of their events (PIECES at a time: first event, and count <<
+ * 25 | place in the stage), the counters of the three, and per-window-tile
+ * counts and cursors.  An STDP block uses the start of the same buffer for
+ * its weight-change table, row bases and prefix. */
+template<unsigned THREADS>
 struct PropagateLds {
-	/* fired rows a delivery block lists at a time */
-	static constexpr unsigned ROWS = THREADS < 512 ? 512 : THREADS;
+	static constexpr unsigned PIECE = 16;
+	static constexpr unsigned ROWS = THREADS;
+	static constexpr unsigned PIECES = 2 * THREADS;
 	int2* stage;
-	uint64_t* word;
-	uint32_t* wpre;
-	uint32_t* rb;
-	uint32_t* rpre;
+	uint2* piece;
+	uint32_t* row;
+	uint32_t* rows;   /* fired rows of the batch */
+	uint32_t* pieces; /* pieces of the chunk of rows */
+	uint32_t* fill;   /* events staged, or delivered beyond the stage */
 	uint32_t* cnt;
 	uint32_t* cur;
-	uint32_t* bucket;
-	/* events of a batch of the event loop, events per row bucket, and the
-	 * most events of a chunk whose buckets the rows mark (buckets hold the
-	 * larger of a batch and that) */
-	static constexpr unsigned BATCH = EV_ILP * THREADS;
-	static constexpr unsigned BUCKET_SHIFT = 5;
-	static constexpr unsigned MARKED = 16384;
-	static constexpr unsigned BUCKETS = (BATCH > MARKED ? BATCH : MARKED) >> BUCKET_SHIFT;
 	__device__ PropagateLds(unsigned char* p, unsigned cap, unsigned max_window)
 	{
 		stage = reinterpret_cast<int2*>(p);
-		word = reinterpret_cast<uint64_t*>(stage + cap);
-		wpre = reinterpret_cast<uint32_t*>(word + THREADS);
-		rb = wpre + THREADS + 2;
-		rpre = rb + ROWS;
-		bucket = rpre + ROWS + 2;
-		cnt = bucket + BUCKETS + 2;
+		piece = reinterpret_cast<uint2*>(stage + cap);
+		row = reinterpret_cast<uint32_t*>(piece + PIECES);
+		rows = row + ROWS;
+		pieces = rows + 1;
+		fill = rows + 2;
+		cnt = rows + 4;
 		cur = cnt + max_window;
 	}
 	static constexpr size_t delivery_bytes(unsigned cap, unsigned max_window)
 	{
-		return size_t(cap) * 8 + size_t(THREADS) * 8 + 4 * (size_t(THREADS) + 2) + 4 * (2 * size_t(ROWS) + 2)
-			+ 4 * (size_t(BUCKETS) + 2) + 8 * size_t(max_window);
+		return size_t(cap) * 8 + size_t(PIECES) * 8 + 4 * (size_t(ROWS) + 4) + 8 * size_t(max_window);
 	}
 	static constexpr size_t stdp_bytes() { return 128 * 4 + 4 * (2 * size_t(THREADS) + 2) + 8 * size_t(THREADS); }
 	static constexpr size_t bytes(bool delivery, unsigned cap, unsigned max_window)
@@ -90,200 +83,141 @@ struct PropagateLds {
 	}
 };
 
-__device__ inline unsigned kth_set_bit(uint64_t w, unsigned k)
-{
-	for(unsigned i = 0; i < k; ++i) w &= w - 1;
-	return unsigned(__builtin_ctzll(w));
-}
-
 /* ------------------------------------------------------------ delivery */
 
 /* A delivery block: list the fired rows of its (source tile, delay) pairs,
- * read their row pointers in parallel, then spread all their events evenly
- * over the block (four loads in flight per thread), staging them in LDS;
- * finally counting-sort the staged events by target tile (relative to the
- * block's window) into the block's bins. */
+ * read their row pointers in parallel, list the rows' events in pieces of up
+ * to 16, then spread the pieces over groups of 16 lanes, a lane an event and
+ * EV_ILP pieces in flight, staging the events in LDS; finally counting-sort the
+ * staged events by target tile (relative to the block's window) into the
+ * block's bins.
+ *
+ * The block is a chain of dependent phases (bitmap words, row pointers,
+ * events, sort, copy-out), and its length bounds the launch that carries it.
+ * So the lists are built with LDS counters in whatever order the waves come
+ * (the sums are integer, any order gives the same), where scans over the block
+ * took two barriers each and an event its search for the row it belongs to;
+ * and a pair is divided into tile and delay once, in 32
+ * bits (a pair's number is below tiles * D, at most 2^24).  Measured with the
+ * wave sums by DPP (us a step, graphs): 100k neurons x 1000 synapses 18.07 ->
+ * 17.14 without STDP, 20.65 -> 19.65 with it; 100k x 400 13.4 -> 12.0; 60k x
+ * 600 12.9 -> 11.2.  Pieces of 64, a wave each, were slower than the scans
+ * (20.8): rows of 20 to 50 events leave too many lanes idle. */
 template<unsigned THREADS, int EV_ILP = EVENT_ILP>
 __device__ inline void deliver_block(const nemo_propagate_args& a, uint64_t t, unsigned b, unsigned char* lds)
 {
-	using Lds = PropagateLds<THREADS, EV_ILP>;
+	using Lds = PropagateLds<THREADS>;
 	constexpr unsigned ROWS = Lds::ROWS;
-	constexpr unsigned ROWS_PER_THREAD = ROWS / THREADS;
+	constexpr unsigned PIECES = Lds::PIECES;
+	constexpr uint32_t PIECE = Lds::PIECE;
+	constexpr unsigned GROUPS = THREADS / PIECE;
+	constexpr uint32_t PLACES = (1u << 25) - 1; /* beyond any stage */
 	const Lds L(lds, a.bin_capacity, a.max_window);
 	int2* stage = L.stage;
 	uint32_t* cnt = L.cnt;
 	uint32_t* cur = L.cur;
-	uint64_t* s_word = L.word;
-	uint32_t* s_wpre = L.wpre;
-	uint32_t* s_rb = L.rb;
-	uint32_t* s_rpre = L.rpre;
 
 	const unsigned CAP = a.bin_capacity;
 	const unsigned D = a.D;
 	const unsigned DC = a.d_count;
 	const unsigned tid = threadIdx.x;
+	const unsigned lane = tid % PIECE;
 	const unsigned col = a.block_base + b;
 	const size_t parity = t & 1;
 	int64_t* acc = a.acc + parity * 2 * a.acc_pitch;
 	const uint2 win = a.windows[b];
 	const unsigned tlo = win.x;
 	const unsigned W = win.y - win.x; /* tiles in the window */
+	const uint32_t q0 = a.pair_bounds[b];
+	const uint32_t nwords = (a.pair_bounds[b + 1] - q0) * 4;
 	for(unsigned p = tid; p < W; p += THREADS) cnt[p] = 0;
+	if(tid == 0) *L.fill = 0;
 
-	const uint64_t q0 = a.pair_bounds[b];
-	const uint64_t q1 = a.pair_bounds[b + 1];
-	const uint64_t nwords = (q1 - q0) * 4;
-	uint32_t fill = 0;
-	unsigned long long events = 0;
+	/* staging of an event at its place: with a count for its tile, or (beyond
+	 * capacity or, defensively, outside the window) straight into the
+	 * accumulators */
+	auto stage_event = [&](int2 ev, uint32_t pos) {
+		const uint32_t rel = uint32_t(ev.x) / NEMO_TILE - tlo;
+		if(pos < CAP && rel < W) {
+			stage[pos] = ev;
+			atomicAdd(&cnt[rel], 1u);
+		} else {
+			if(pos < CAP) stage[pos] = make_int2(-1, 0);
+			int64_t* dst = acc + (ev.y >= 0 ? size_t(0) : a.acc_pitch) + uint32_t(ev.x);
+			atomicAdd(reinterpret_cast<unsigned long long*>(dst), (unsigned long long)(int64_t)ev.y);
+		}
+	};
 
-	for(uint64_t wb = 0; wb < nwords; wb += THREADS) {
+	for(uint32_t wb = 0; wb < nwords; wb += THREADS) {
 		/* the bitmap words of this batch, one per thread */
 		uint64_t word = 0;
-		const uint64_t w = wb + tid;
+		uint32_t row0 = 0; /* row of the word's first neuron */
+		const uint32_t w = wb + tid;
 		if(w < nwords) {
-			const uint64_t q = q0 + w / 4;
-			const unsigned p = unsigned(q / DC);
-			const unsigned d = unsigned(q % DC) + a.d_first;
+			const uint32_t q = q0 + w / 4;
+			const uint32_t p = q / DC;
+			const uint32_t d = q - p * DC + a.d_first;
+			row0 = (p * NEMO_TILE + (w & 3) * 64) * D + (d - 1);
 			if(t >= d) word = a.fired_bits[((t - d) & PROPAGATE_RING_MASK) * a.fired_words + size_t(p) * 4 + (w & 3)];
 		}
-		__syncthreads(); /* previous batch done with s_word */
-		s_word[tid] = word;
-		uint32_t R;
-		const uint32_t wpre = block_exclusive_scan<THREADS>(uint32_t(__popcll(word)), &R);
-		s_wpre[tid] = wpre;
-		if(tid == 0) s_wpre[THREADS] = R;
+		if(tid == 0) *L.rows = 0;
 		__syncthreads();
-
-		for(uint32_t r0 = 0; r0 < R; r0 += ROWS) {
-			const uint32_t nr = min(ROWS, R - r0);
-			/* row pointers of up to ROWS fired rows, ROWS_PER_THREAD per thread */
-			uint32_t lens[ROWS_PER_THREAD];
-			uint32_t mine = 0;
-			uint32_t rr[ROWS_PER_THREAD];
-			unsigned wl[ROWS_PER_THREAD];
-#pragma unroll
-			for(unsigned k = 0; k < ROWS_PER_THREAD; ++k) rr[k] = r0 + tid * ROWS_PER_THREAD + k;
-			last_not_above_k<THREADS>(s_wpre, THREADS, rr, wl);
-			uint32_t rbv[ROWS_PER_THREAD], rev[ROWS_PER_THREAD];
-#pragma unroll
-			for(unsigned k = 0; k < ROWS_PER_THREAD; ++k) {
-				const uint32_t ri = tid * ROWS_PER_THREAD + k;
-				rbv[k] = 0;
-				rev[k] = 0;
-				if(ri < nr) {
-					const unsigned lo = wl[k];
-					const uint64_t wg = wb + lo;
-					const uint64_t q = q0 + wg / 4;
-					const unsigned p = unsigned(q / DC);
-					const unsigned d = unsigned(q % DC) + a.d_first;
-					const unsigned bit = kth_set_bit(s_word[lo], rr[k] - s_wpre[lo]);
-					const uint32_t n = p * NEMO_TILE + unsigned(wg & 3) * 64 + bit;
-					const size_t row = size_t(n) * D + (d - 1);
-					rbv[k] = a.rowptr[row];
-					rev[k] = a.rowptr[row + 1];
-				}
+		const uint32_t fired = uint32_t(__popcll(word));
+		const uint32_t mine = wave_append(L.rows, fired);
+		for(uint32_t r0 = 0;; r0 += ROWS) {
+			/* this chunk's rows */
+			uint32_t at = mine;
+			for(uint64_t x = word; x; x &= x - 1, ++at) {
+				if(at - r0 < ROWS) L.row[at - r0] = row0 + uint32_t(__builtin_ctzll(x)) * D;
 			}
-#pragma unroll
-			for(unsigned k = 0; k < ROWS_PER_THREAD; ++k) {
-				const uint32_t ri = tid * ROWS_PER_THREAD + k;
-				lens[k] = rev[k] - rbv[k];
-				if(ri < nr) s_rb[ri] = rbv[k];
-				mine += lens[k];
-			}
-			uint32_t M;
-			uint32_t pre = block_exclusive_scan<THREADS>(mine, &M);
-#pragma unroll
-			for(unsigned k = 0; k < ROWS_PER_THREAD; ++k) {
-				const uint32_t ri = tid * ROWS_PER_THREAD + k;
-				if(ri < nr) s_rpre[ri] = pre;
-				pre += lens[k];
-			}
-			if(tid == 0) s_rpre[nr] = M;
+			if(tid == 0) *L.pieces = 0;
 			__syncthreads();
-
-			/* staging of event number e of this chunk: into the stage with a
-			 * count for its tile, or (beyond capacity or, defensively,
-			 * outside the window) straight into the accumulators */
-			auto stage_event = [&](int2 ev, uint32_t e) {
-				const uint32_t pos = fill + e;
-				const uint32_t rel = uint32_t(ev.x) / NEMO_TILE - tlo;
-				if(pos < CAP && rel < W) {
-					stage[pos] = ev;
-					atomicAdd(&cnt[rel], 1u);
-				} else {
-					if(pos < CAP) stage[pos] = make_int2(-1, 0);
-					int64_t* dst = acc + (ev.y >= 0 ? size_t(0) : a.acc_pitch) + uint32_t(ev.x);
-					atomicAdd(reinterpret_cast<unsigned long long*>(dst), (unsigned long long)(int64_t)ev.y);
-				}
-			};
-			/* the events of these rows evenly over the block, in batches of
-			 * EV_ILP per thread.  An event's row lies between the rows of
-			 * the bucket bounds around it (every 32nd event), which each row
-			 * marks when the chunk has at most MARKED events, or which are
-			 * searched per batch; it is refined between them. */
-			constexpr unsigned BATCH = Lds::BATCH;
-			constexpr unsigned SHIFT = Lds::BUCKET_SHIFT;
-			const bool marked = M <= Lds::MARKED;
-			if(marked) {
-#pragma unroll
-				for(unsigned k = 0; k < ROWS_PER_THREAD; ++k) {
-					const uint32_t ri = tid * ROWS_PER_THREAD + k;
-					if(ri < nr) {
-						const uint32_t p0 = s_rpre[ri], p1 = s_rpre[ri + 1];
-						for(uint32_t j = (p0 + (1u << SHIFT) - 1) >> SHIFT; (j << SHIFT) < p1; ++j) L.bucket[j] = ri;
-					}
-				}
-				if(tid == 0 && M) L.bucket[((M - 1) >> SHIFT) + 1] = nr - 1;
-				__syncthreads();
+			const uint32_t R = *L.rows;
+			/* a row per thread: its events' pieces and their place */
+			uint32_t rb = 0, len = 0;
+			if(r0 + tid < R) {
+				const size_t row = L.row[tid];
+				rb = a.rowptr[row];
+				len = a.rowptr[row + 1] - rb;
 			}
-			for(uint32_t base = 0; base < M; base += BATCH) {
-				const uint32_t b0 = marked ? 0u : base; /* first event of the buckets */
-				if(!marked) {
-					for(unsigned j = tid; j <= (BATCH >> SHIFT); j += THREADS) {
-						L.bucket[j] = last_not_above<ROWS>(s_rpre, nr, min(base + (j << SHIFT), M - 1));
-					}
-					__syncthreads();
+			const uint32_t np = (len + PIECE - 1) / PIECE;
+			const uint32_t first = wave_append(L.pieces, np);
+			const uint32_t place = wave_append(L.fill, len);
+			for(uint32_t p0 = 0;; p0 += PIECES) {
+				/* this round's pieces */
+				for(uint32_t i = max(first, p0); i < min(first + np, p0 + PIECES); ++i) {
+					const uint32_t e = PIECE * (i - first);
+					L.piece[i - p0] = make_uint2(rb + e, (min(PIECE, len - e) << 25) | min(PLACES, place + e));
 				}
-				uint32_t ee[EV_ILP];
-				unsigned lo[EV_ILP], hi[EV_ILP];
-#pragma unroll
-				for(int u = 0; u < EV_ILP; ++u) {
-					/* buckets past the last event may be unset: only the
-					 * events of the chunk read theirs */
-					ee[u] = base + u * THREADS + tid;
-					const unsigned j = (ee[u] - b0) >> SHIFT;
-					lo[u] = ee[u] < M ? L.bucket[j] : 0u;
-					hi[u] = ee[u] < M ? L.bucket[j + 1] : 0u;
-				}
-				bool open = true;
-				while(open) {
-					open = false;
+				__syncthreads();
+				const uint32_t P = *L.pieces;
+				const uint32_t here = min(P - min(P, p0), PIECES);
+				for(uint32_t c0 = tid / PIECE; c0 < here; c0 += EV_ILP * GROUPS) {
+					int2 ev[EV_ILP];
+					uint32_t pos[EV_ILP];
 #pragma unroll
 					for(int u = 0; u < EV_ILP; ++u) {
-						if(lo[u] < hi[u]) {
-							const unsigned mid = lo[u] + ((hi[u] - lo[u] + 1) >> 1);
-							if(s_rpre[mid] <= ee[u]) lo[u] = mid; else hi[u] = mid - 1;
-							open = open || lo[u] < hi[u];
-						}
+						const uint32_t c = c0 + u * GROUPS;
+						const uint2 pc = L.piece[min(c, here - 1)];
+						const bool live = c < here && lane < (pc.y >> 25);
+						pos[u] = live ? (pc.y & PLACES) + lane : ~0u;
+						ev[u] = make_int2(0, 0);
+						if(live) ev[u] = a.fcm[pc.x + lane];
+					}
+#pragma unroll
+					for(int u = 0; u < EV_ILP; ++u) {
+						if(pos[u] != ~0u) stage_event(ev[u], pos[u]);
 					}
 				}
-				int2 ev[EV_ILP];
-#pragma unroll
-				for(int u = 0; u < EV_ILP; ++u) {
-					ev[u] = make_int2(0, 0);
-					if(ee[u] < M) ev[u] = a.fcm[s_rb[lo[u]] + (ee[u] - s_rpre[lo[u]])];
-				}
-#pragma unroll
-				for(int u = 0; u < EV_ILP; ++u) {
-					if(ee[u] < M) stage_event(ev[u], ee[u]);
-				}
-				if(!marked) __syncthreads(); /* the buckets are rewritten by the next batch */
+				if(p0 + PIECES >= P) break;
+				__syncthreads(); /* the list is rewritten */
 			}
-			fill += M;
-			events += M;
-			__syncthreads(); /* s_rb / s_rpre are rewritten by the next chunk */
+			__syncthreads(); /* the lists are rewritten by the next chunk or batch */
+			if(r0 + ROWS >= R) break;
 		}
 	}
+	if(nwords == 0) __syncthreads();
+	const uint32_t fill = *L.fill;
 
 	/* counting sort of the staged events by target tile */
 	const uint32_t staged = min(fill, CAP);
@@ -351,7 +285,7 @@ __device__ inline void deliver_block(const nemo_propagate_args& a, uint64_t t, u
 			}
 		}
 	}
-	if(tid == 0 && events) a.block_events[col] += events;
+	if(tid == 0 && fill) a.block_events[col] += fill;
 }
 
 /* ---------------------------------------------------------------- STDP */
