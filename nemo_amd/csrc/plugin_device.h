@@ -99,23 +99,10 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t x, uint32_t* total)
 	return before + v - x;
 }
 
-/* The largest i < n with arr[i] <= x, for a non-decreasing arr with
- * arr[0] <= x and n <= MAXN (a power of two): a fixed number of unrolled
- * steps, so that searches of independent items interleave. */
-template<unsigned MAXN>
-__device__ inline unsigned last_not_above(const uint32_t* arr, unsigned n, uint32_t x)
-{
-	unsigned lo = 0;
-#pragma unroll
-	for(unsigned step = MAXN / 2; step >= 1; step >>= 1) {
-		const unsigned probe = lo + step;
-		if(probe < n && arr[probe] <= x) lo = probe;
-	}
-	return lo;
-}
-
-/* last_not_above for K items at once, step by step in lock-step, so that
- * the K LDS reads of a step are in flight together.  Requires n >= 1. */
+/* For each of K items x, the largest i < n with arr[i] <= x, for a
+ * non-decreasing arr with arr[0] <= x and 1 <= n <= MAXN (a power of two): a
+ * fixed number of steps, in lock-step, so that the K LDS reads of a step are
+ * in flight together. */
 template<unsigned MAXN, int K>
 __device__ inline void last_not_above_k(const uint32_t* arr, unsigned n, const uint32_t (&x)[K], unsigned (&lo)[K])
 {
@@ -143,45 +130,25 @@ struct TileInput {
 	long long I[NEMO_TILE];
 };
 
-/* Gather batches: GATHER_ILP events per thread in flight (6 when the tile's
- * block has NEMO_COLAUNCH_BLOCK threads, all of which gather: 3072 events per
- * batch, and 0.25 us per step faster than 8 at 100k x 1000); an event's column
- * is found from buckets of 2^GATHER_SHIFT events, marked per column when the
- * tile has at most GATHER_MARKED events. */
-constexpr int GATHER_ILP = 8;
-constexpr int GATHER_ILP_WIDE = 6;
-constexpr unsigned GATHER_SHIFT = 3;
-constexpr unsigned GATHER_MARKED = 4096;
-/* events of the largest batch or marked gather */
-constexpr unsigned GATHER_BUCKETS_MAX_EVENTS = GATHER_MARKED > GATHER_ILP_WIDE * NEMO_COLAUNCH_BLOCK
-	? (GATHER_MARKED > GATHER_ILP * NEMO_TILE ? GATHER_MARKED : GATHER_ILP * NEMO_TILE)
-	: GATHER_ILP_WIDE * NEMO_COLAUNCH_BLOCK;
-constexpr unsigned GATHER_BUCKETS = GATHER_BUCKETS_MAX_EVENTS / (1u << GATHER_SHIFT) + 2;
+/* Columns of the bin table a group of lanes gathers at a time, an event per
+ * lane each in flight. */
+constexpr int GATHER_ILP = 4;
 
 /* Pieces (of up to 64 events) of fired rows that a block delivering directly
  * lists in LDS at a time. */
 constexpr unsigned DIRECT_CHUNKS = 256;
 
-/* The LDS an update block uses: its tile's input sums, the gather's column
- * prefix, bases and buckets, and the per-tile STDP lists.  A kernel takes it
+/* The LDS an update block uses: its tile's input sums, the lists of direct
+ * delivery, and the per-tile STDP lists.  A kernel takes it
  * from update_lds<DYNAMIC>(): a static array, or -- in launches that also run
  * propagate blocks -- the start of the launch's dynamic LDS, which those
  * blocks use for their own purposes, so that a block of either kind needs
  * only the larger of the two. */
 struct UpdateLds {
 	TileInput input;
-	uint32_t pre[NEMO_MAX_BIN_BLOCKS + 1];
-	union {
-		uint32_t base[NEMO_MAX_BIN_BLOCKS];
-		uint2 chunk[DIRECT_CHUNKS];      /* direct delivery: pieces of the fired rows */
-	};
-	union {
-		uint32_t bucket[GATHER_BUCKETS];
-		struct {                         /* direct delivery: events per delay, pieces listed */
-			uint32_t count[64];
-			uint32_t chunks;
-		};
-	};
+	uint2 chunk[DIRECT_CHUNKS]; /* direct delivery: pieces of the fired rows, events per delay, pieces listed */
+	uint32_t count[64];
+	uint32_t chunks;
 	int32_t fn[128];
 	uint32_t rb[NEMO_TILE];
 	uint32_t pos[NEMO_TILE + 1];
@@ -200,12 +167,6 @@ __device__ inline UpdateLds& update_lds()
 	}
 }
 
-/* Sum the tile's input of this step into LDS: the overflow accumulators of
- * its neurons (cleared here, cpu/Simulation.cpp:279-288) and the binned events
- * of every delivery column (integer sums, so the order of the 64-bit LDS
- * atomics does not matter).  The whole table row is read: columns whose
- * window does not hold the tile keep a zero count, and reading them costs
- * less than a dependent load of the tile's column range. */
 struct Nothing {
 	__device__ void operator()() const {}
 };
@@ -268,29 +229,42 @@ __device__ inline void gather_direct(const nemo_hip_step_buffers& b, UpdateLds& 
 	__syncthreads(); /* count and chunks, for record_firing */
 }
 
-/* prefetch() is called once the tile's table row and accumulators are
+/* Sum the tile's input of this step into LDS: the overflow accumulators of
+ * its neurons (cleared here, cpu/Simulation.cpp:279-288) and the binned events
+ * of every delivery column (integer sums, so the order of the 64-bit LDS
+ * atomics does not matter).  The whole table row is read (or, bin_ranged, the
+ * tile's two ranges of it): columns whose window does not hold the tile keep
+ * a zero count, and reading them costs less than a dependent load of the
+ * tile's column range.
+ *
+ * A group of lanes takes a column: its entry, then its events, a lane each,
+ * four columns in flight per group.  Two round trips and no barrier between
+ * them, where one event per thread needs the columns' prefix (a block scan)
+ * and a search for each event's column.  The lanes per group are what a block
+ * has for two rounds of four columns: 16 at 100k neurons x 1000 synapses (245
+ * columns of about 8 of the tile's events).  Measured (us a step, graphs, scan
+ * and search before): 100k x 1000 17.06 -> 16.14 without STDP, 19.7 -> 19.3
+ * with it, a batch of 32 networks 19.1 -> 17.9; one round of six columns 16.5
+ * and 19.3, of eight spills (72 VGPRs) and gains nothing.
+ *
+ * prefetch() is called once the row's entries and the accumulators are
  * requested: the loads it issues (the model's state, say) queue behind them,
- * so that waiting for the table does not wait for them too.  meanwhile()
+ * so that waiting for the entries does not wait for them too.  meanwhile()
  * runs in the tile's own threads, all of them, while the ring's slot is on
  * its way (direct delivery) or the block's other waves still sum events: work
  * on what prefetch loaded that needs no input, such as a neuron's noise.
- * Beside the events' loads its registers would take the update from 58 VGPRs
- * to 72, before them it would hold the gather up.
  *
  * THREADS threads of the block take part: the tile's NEMO_TILE (one per
- * neuron, which alone read the table row, the accumulators and, through
- * prefetch, their neuron's state) and, in a block of NEMO_COLAUNCH_BLOCK
- * threads, helpers that only load and sum events, so that a tile of up to
- * 3072 events (GATHER_ILP_WIDE per thread) takes one round of loads.  Returns false for
- * the helpers, which take no further part in the step. */
+ * neuron, which alone read the accumulators and, through prefetch, their
+ * neuron's state) and, in a block of NEMO_COLAUNCH_BLOCK threads, helpers that
+ * only load and sum events.  Returns false for the helpers, which take no
+ * further part in the step. */
 template<unsigned THREADS = NEMO_TILE, typename Prefetch = Nothing, typename Meanwhile = Nothing>
 __device__ inline bool gather_input(const nemo_hip_step_buffers& b, const nemo_hip_neuron_group& g, UpdateLds& L,
 		Prefetch prefetch = Prefetch(), Meanwhile meanwhile = Meanwhile())
 {
 	static_assert(THREADS % 64 == 0 && THREADS >= NEMO_TILE, "whole waves beyond the tile");
 	TileInput& in = L.input;
-	uint32_t* s_pre = L.pre;
-	uint32_t* s_base = L.base;
 	const unsigned tid = threadIdx.x;
 	const bool lead = THREADS == NEMO_TILE || tid < NEMO_TILE; /* uniform per wave */
 	const unsigned tile = g.start / NEMO_TILE + blockIdx.x;
@@ -305,9 +279,9 @@ __device__ inline bool gather_input(const nemo_hip_step_buffers& b, const nemo_h
 	int64_t* acc = b.acc + parity * 2 * b.acc_pitch;
 	const unsigned ng = tile * NEMO_TILE + tid;
 	const unsigned BB = b.bin_blocks;
-	const uint32_t* row = b.bin_table + (parity * b.tiles + tile) * BB;
-	const size_t cap = b.bin_capacity;
-	const int2* bins = b.bins + parity * BB * cap;
+	const char* row = reinterpret_cast<const char*>(b.bin_table + (parity * b.tiles + tile) * BB);
+	const uint32_t cap = b.bin_capacity;
+	const char* bins = reinterpret_cast<const char*>(b.bins + parity * BB * size_t(cap));
 	/* the columns read: the whole row, or (bin_ranged) the tile's two ranges,
 	 * column first0 + i for i < n0, then first1 + i - n0 */
 	const unsigned BR = b.bin_first_set ? b.bin_first_set : BB; /* columns holding events */
@@ -319,118 +293,74 @@ __device__ inline bool gather_input(const nemo_hip_step_buffers& b, const nemo_h
 		first1 = r1 & 0xffffu;
 		B = n0 + (b.bin_first_set ? 0u : (r1 >> 16) - first1);
 	}
-	constexpr unsigned PER = NEMO_MAX_BIN_BLOCKS / NEMO_TILE;
-	uint32_t ent[PER];
-	unsigned col[PER];
-	/* a helper's i is at least NEMO_TILE * PER = NEMO_MAX_BIN_BLOCKS >= B */
-#pragma unroll
-	for(unsigned k = 0; k < PER; ++k) {
-		const unsigned i = tid * PER + k;
-		col[k] = i < n0 ? first0 + i : first1 + (i - n0);
-		ent[k] = i < B ? row[col[k]] : 0u;
-	}
-	if(lead) {
-		const int64_t oe = acc[ng];
-		const int64_t oi = acc[b.acc_pitch + ng];
-		const uint2 prow = push_row(b, ng);
-		prefetch();
-		in.E[tid] = oe;
-		in.I[tid] = oi;
-		L.push_rows[tid] = prow;
-		if(oe) acc[ng] = 0;
-		if(oi) acc[b.acc_pitch + ng] = 0;
-	}
-	if(B == 0) {
-		if(lead) meanwhile();
-		__syncthreads();
-		return lead;
-	}
-	uint32_t mine = 0;
-#pragma unroll
-	for(unsigned k = 0; k < PER; ++k) {
-		const unsigned i = tid * PER + k;
-		if(i < B) s_base[i] = uint32_t(col[k] * cap + (ent[k] & 0xffffu));
-		mine += ent[k] >> 16;
-	}
-	/* batches of ILP events per thread, ILP independent loads in flight per
-	 * thread before the LDS atomics.  An event's column lies
-	 * between the columns of the bucket bounds around it (every 8th event),
-	 * which each column marks when the tile has at most MARKED events, or
-	 * which are searched per batch; it is refined between them. */
-	constexpr int ILP = THREADS > NEMO_TILE ? GATHER_ILP_WIDE : GATHER_ILP;
-	constexpr unsigned BATCH = ILP * THREADS;
-	constexpr unsigned SHIFT = GATHER_SHIFT;
-	constexpr unsigned MARKED = GATHER_MARKED;
-	static_assert(BATCH <= GATHER_BUCKETS_MAX_EVENTS, "the bucket array holds a batch");
-	uint32_t* s_bucket = L.bucket;
-	uint32_t total;
-	uint32_t pre = block_exclusive_scan<THREADS>(mine, &total);
-	const bool marked = total <= MARKED;
-#pragma unroll
-	for(unsigned k = 0; k < PER; ++k) {
-		const unsigned i = tid * PER + k;
-		const uint32_t c = ent[k] >> 16;
-		if(i < B) {
-			s_pre[i] = pre;
-			if(marked) {
-				for(uint32_t j = (pre + (1u << SHIFT) - 1) >> SHIFT; (j << SHIFT) < pre + c; ++j) s_bucket[j] = i;
-			}
-		}
-		pre += c;
-	}
-	if(tid == 0) {
-		s_pre[B] = total;
-		if(marked && total) s_bucket[((total - 1) >> SHIFT) + 1] = B - 1;
-	}
-	__syncthreads();
-	for(uint32_t base = 0; base < total; base += BATCH) {
-		const uint32_t b0 = marked ? 0u : base; /* first event of the buckets */
-		if(!marked) {
-			for(unsigned j = tid; j <= (BATCH >> SHIFT); j += THREADS) {
-				s_bucket[j] = last_not_above<NEMO_MAX_BIN_BLOCKS>(s_pre, B, min(base + (j << SHIFT), total - 1));
-			}
-			__syncthreads();
-		}
-		uint32_t jj[ILP];
-		unsigned lo[ILP], hi[ILP];
+	/* groups of 1 << shift lanes take a column each, as many lanes as two
+	 * rounds of GATHER_ILP columns per group leave them */
+	constexpr int ILP = GATHER_ILP;
+	unsigned shift = 6;
+	while(shift > 2 && (B << shift) > 2 * ILP * THREADS) --shift;
+	const unsigned lanes = 1u << shift, lane = tid & (lanes - 1);
+	const unsigned groups = THREADS >> shift, group = tid >> shift;
+	uint32_t ent[ILP]; /* count << 16 | offset */
+	auto column = [&](unsigned i) { return i < n0 ? first0 + i : first1 + (i - n0); };
+	auto read_row = [&](unsigned c0) {
 #pragma unroll
 		for(int u = 0; u < ILP; ++u) {
-			/* buckets past the last event may be unset: only the events of
-			 * the tile read theirs */
-			jj[u] = base + u * THREADS + tid;
-			const unsigned j = (jj[u] - b0) >> SHIFT;
-			lo[u] = jj[u] < total ? s_bucket[j] : 0u;
-			hi[u] = jj[u] < total ? s_bucket[j + 1] : 0u;
+			const unsigned i = c0 + u * groups + group;
+			ent[u] = i < B ? *reinterpret_cast<const uint32_t*>(row + column(i) * uint32_t(sizeof(uint32_t))) : 0u;
 		}
-		bool open = true;
-		while(open) {
-			open = false;
+	};
+	read_row(0);
+	int64_t oe = 0, oi = 0;
+	if(lead) {
+		oe = acc[ng];
+		oi = acc[b.acc_pitch + ng];
+		const uint2 prow = push_row(b, ng);
+		prefetch();
+		in.E[tid] = 0;
+		in.I[tid] = 0;
+		L.push_rows[tid] = prow;
+	}
+	__syncthreads(); /* the sums are cleared; the loads stay on their way */
+	for(unsigned c0 = 0; c0 < B; c0 += ILP * groups) {
+		if(c0) read_row(c0);
+		uint32_t at[ILP]; /* byte offset of the lane's next event: below 2^28 */
+#pragma unroll
+		for(int u = 0; u < ILP; ++u) {
+			at[u] = (column(c0 + u * groups + group) * cap + (ent[u] & 0xffffu) + lane) * uint32_t(sizeof(int2));
+			ent[u] >>= 16;
+		}
+		/* events lane, lane + lanes, ... of every column: one round while no
+		 * column holds more events than its group has lanes */
+		bool more = true;
+		for(uint32_t e = lane; __any(more); e += lanes) {
+			int2 ev[ILP];
+			more = false;
 #pragma unroll
 			for(int u = 0; u < ILP; ++u) {
-				if(lo[u] < hi[u]) {
-					const unsigned mid = lo[u] + ((hi[u] - lo[u] + 1) >> 1);
-					if(s_pre[mid] <= jj[u]) lo[u] = mid; else hi[u] = mid - 1;
-					open = open || lo[u] < hi[u];
+				ev[u] = make_int2(-1, 0);
+				if(e < ent[u]) ev[u] = *reinterpret_cast<const int2*>(bins + at[u]);
+				at[u] += lanes * uint32_t(sizeof(int2));
+				more = more || e - lane + lanes < ent[u];
+			}
+#pragma unroll
+			for(int u = 0; u < ILP; ++u) {
+				if(ev[u].x >= 0) {
+					long long* dst = ev[u].y >= 0 ? &in.E[ev[u].x] : &in.I[ev[u].x];
+					atomicAdd(reinterpret_cast<unsigned long long*>(dst), (unsigned long long)(long long)ev[u].y);
 				}
 			}
 		}
-		int2 ev[ILP];
-#pragma unroll
-		for(int u = 0; u < ILP; ++u) {
-			ev[u] = make_int2(0, 0);
-			if(jj[u] < total) ev[u] = bins[s_base[lo[u]] + (jj[u] - s_pre[lo[u]])];
-		}
-#pragma unroll
-		for(int u = 0; u < ILP; ++u) {
-			if(jj[u] < total) {
-				long long* dst = ev[u].y >= 0 ? &in.E[ev[u].x] : &in.I[ev[u].x];
-				atomicAdd(reinterpret_cast<unsigned long long*>(dst), (unsigned long long)(long long)ev[u].y);
-			}
-		}
-		if(!marked) __syncthreads(); /* the buckets are rewritten by the next batch */
 	}
-	if(lead) meanwhile();
+	if(lead) {
+		if(oe) acc[ng] = 0;
+		if(oi) acc[b.acc_pitch + ng] = 0;
+		meanwhile();
+	}
 	__syncthreads();
+	if(lead) {
+		in.E[tid] += oe;
+		in.I[tid] += oi;
+	}
 	return lead;
 }
 
