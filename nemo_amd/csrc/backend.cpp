@@ -599,6 +599,7 @@ Simulation::~Simulation()
 	}
 	if(m_pinnedScalars) (void) hipHostFree(m_pinnedScalars);
 	if(m_pinnedBits) (void) hipHostFree(m_pinnedBits);
+	if(m_pinnedStage) (void) hipHostFree(m_pinnedStage);
 	if(m_pinnedCounters) (void) hipHostFree(m_pinnedCounters);
 	if(m_pinnedListCounts) (void) hipHostFree(m_pinnedListCounts);
 	for(uint32_t* p : m_pinnedList) {
@@ -1894,6 +1895,7 @@ void Simulation::enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, 
 		}
 	}
 	if(lagged && k) HIP_CHECK(hipStreamWaitEvent(m_stream, m_stdpLag[(k - 1) & 1], 0));
+	if(advanceBase && k && !batched) HIP_CHECK(nemo_launch_advance_clock(m_stream, m_clock.ptr, first + k));
 }
 
 /* k steps with neuron updates were enqueued after m_hostStep */
@@ -2096,44 +2098,49 @@ const std::vector<unsigned>& Simulation::step(const unsigned* fstim, size_t nf,
 	std::vector<uint32_t> fIdx(nf);
 	for(size_t i = 0; i < nf; ++i) fIdx[i] = localIdx(fstim[i]);
 
-	const size_t nstim = std::max(iIdx.size(), fIdx.size());
-	if(nstim > m_stimIdx.n) {
-		HIP_CHECK(hipStreamSynchronize(m_stream));
-		m_stimIdx.allocate(nstim);
-		m_stimVal.allocate(nstim);
-	}
-	if(!iIdx.empty()) {
-		HIP_CHECK(hipMemcpyAsync(m_stimIdx.ptr, iIdx.data(), iIdx.size() * 4, hipMemcpyHostToDevice, m_stream));
-		HIP_CHECK(hipMemcpyAsync(m_stimVal.ptr, iVal.data(), iVal.size() * 4, hipMemcpyHostToDevice, m_stream));
-		HIP_CHECK(nemo_launch_istim(m_stream, m_ext.ptr, m_stimIdx.ptr, m_stimVal.ptr, iIdx.size()));
-		/* the index buffer is reused for the firing stimulus below */
-		HIP_CHECK(hipStreamSynchronize(m_stream));
-	}
-	if(!fIdx.empty()) {
-		HIP_CHECK(hipMemcpyAsync(m_stimIdx.ptr, fIdx.data(), fIdx.size() * 4, hipMemcpyHostToDevice, m_stream));
-		HIP_CHECK(nemo_launch_fstim(m_stream, m_fstim.ptr, m_stimIdx.ptr, fIdx.size(), 1));
-	}
+	/* the lists go to the device in pinned memory that the kernels read, and
+	 * the step's number as an offset from the base that the device has: a
+	 * copy each (and a synchronisation between the two lists) took 90 us a
+	 * step of a 1000-neuron network, whose kernels take 8 */
+	uint32_t* fList = static_cast<uint32_t*>(stageRoom((nf + 2 * iIdx.size()) * sizeof(uint32_t)));
+	uint32_t* iList = fList + nf;
+	float* vList = reinterpret_cast<float*>(iList + iIdx.size());
+	std::copy(fIdx.begin(), fIdx.end(), fList);
+	std::copy(iIdx.begin(), iIdx.end(), iList);
+	std::copy(iVal.begin(), iVal.end(), vList);
+	m_stageBusy = true;
+	HIP_CHECK(nemo_launch_stimulus(m_stream, m_fstim.ptr, fList, nf, m_ext.ptr, iList, vList, iIdx.size()));
 	const uint64_t t = m_hostStep;
 	ensureRing();
-	setBase(t);
-	enqueueSteps(0, 1, !iIdx.empty(), !fIdx.empty());
+	enqueueSteps(t - m_base, 1, !iIdx.empty(), !fIdx.empty());
 	advanceSteps(1);
-	if(!fIdx.empty()) {
-		HIP_CHECK(nemo_launch_fstim(m_stream, m_fstim.ptr, m_stimIdx.ptr, fIdx.size(), 0));
-	}
-	readBitmaps(t, 1);
+	HIP_CHECK(nemo_launch_step_readout(m_stream, m_firedBits.ptr + (t & (NEMO_STEP_RING - 1)) * m_firedWords, m_pinnedBits,
+				m_firedWords, m_fstim.ptr, fList, nf));
 	waitStream(m_stream);
+	m_stageBusy = false;
 	checkStatus();
 	m_firedOut.clear();
 	decodeFiring(m_pinnedBits, m_firedOut);
 	return m_firedOut;
 }
 
-/* With batched STDP every graph of steps ends with a snapshot, which then
- * moves the step base on (the other placements set it from the host). */
-bool Simulation::graphsAdvanceBase() const
+/* Pinned room for a call's lists, and for what its kernels give back. */
+void* Simulation::stageRoom(size_t bytes)
 {
-	return m_shape.stdpMode == 4 && m_stdpBlocks;
+	if(m_stageBusy) {
+		/* a call before ended in an error with kernels under way */
+		HIP_CHECK(hipStreamSynchronize(m_stream));
+		m_stageBusy = false;
+	}
+	if(bytes > m_pinnedStageCap) {
+		const size_t cap = std::max<size_t>(65536, 2 * bytes);
+		unsigned char* p = nullptr;
+		HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&p), cap, hipHostMallocDefault));
+		if(m_pinnedStage) HIP_CHECK(hipHostFree(m_pinnedStage));
+		m_pinnedStage = p;
+		m_pinnedStageCap = cap;
+	}
+	return m_pinnedStage;
 }
 
 hipGraphExec_t Simulation::graphFor(unsigned k, bool forkPending)
@@ -2146,7 +2153,7 @@ hipGraphExec_t Simulation::graphFor(unsigned k, bool forkPending)
 	const bool debug = m_debug;
 	m_debug = false;
 	try {
-		enqueueSteps(0, k, false, false, nullptr, forkPending, graphsAdvanceBase());
+		enqueueSteps(0, k, false, false, nullptr, forkPending, true);
 	} catch(...) {
 		m_debug = debug;
 		m_stdpPending = false;
@@ -2301,13 +2308,12 @@ void Simulation::run(unsigned nsteps, unsigned stdpPeriod, float reward, bool re
 			const uint64_t t0 = m_hostStep;
 			hipGraphExec_t g = graphFor(k, batchPending);
 			batchPending = true; /* each chunk leaves its steps pending */
-			const bool advances = graphsAdvanceBase();
 			ensureRing();
-			if(!advances || m_base != t0) setBase(t0);
+			if(m_base != t0) setBase(t0);
 			/* the ring slots this chunk overwrites were copied out */
 			if(inFlight[half]) HIP_CHECK(hipStreamWaitEvent(m_stream, copied[half], 0));
 			HIP_CHECK(hipGraphLaunch(g, m_stream));
-			if(advances) m_base = t0 + k;
+			m_base = t0 + k;
 			advanceSteps(k);
 			if(readRaster) {
 				uint32_t* listDev = devList ? m_listDev.ptr + size_t(half) * CHUNK * m_npad : nullptr;
@@ -2524,11 +2530,10 @@ double Simulation::timeSteps(unsigned nsteps)
 	while(done < nsteps) {
 		const unsigned k = std::min(64u, nsteps - done);
 		hipGraphExec_t g = graphFor(k, true);
-		const bool advances = graphsAdvanceBase();
 		ensureRing();
-		if(!advances || m_base != m_hostStep) setBase(m_hostStep);
+		if(m_base != m_hostStep) setBase(m_hostStep);
 		HIP_CHECK(hipGraphLaunch(g, m_stream));
-		if(advances) m_base = m_hostStep + k;
+		m_base = m_hostStep + k;
 		advanceSteps(k);
 		done += k;
 	}
@@ -2712,9 +2717,8 @@ void Simulation::applyStdp(float reward)
  * written from it, the spikes arriving at step s + 1 are delivered and
  * gathered, and the timer advances by one step.  Defined only without STDP,
  * as in the CUDA backend. */
-void Simulation::propagateDevice(const uint32_t* flags, float** E, float** I)
+void Simulation::propagateStep(const uint32_t* flags, float* E, float* I)
 {
-	activate();
 	if(m_nets > 1) {
 		throw Error(NEMO_API_UNSUPPORTED, "propagate drives a single network");
 	}
@@ -2726,45 +2730,56 @@ void Simulation::propagateDevice(const uint32_t* flags, float** E, float** I)
 		for(size_t i = 0; i < m_ncount; ++i) d2s[m_order[i]] = uint32_t(i);
 		m_devToSim.allocate(m_npad);
 		HIP_CHECK(hipMemcpy(m_devToSim.ptr, d2s.data(), m_devToSim.bytes(), hipMemcpyHostToDevice));
+	}
+	joinStdp();
+	const uint64_t s = m_hostStep, off = s - m_base;
+	ensureRing();
+	nemo_hip_step_buffers b = stepBuffers(off, false, false);
+	b.debug_current = nullptr;
+	HIP_CHECK(nemo_launch_external_fire(m_stream, &b, flags, m_fstim.ptr, m_devToSim.ptr, m_tiles));
+	b.step_offset = off + 1;
+	if(!m_shape.direct) {
+		launchDelivery(m_early, off + 1, m_stream, false);
+		launchDelivery(m_late, off + 1, m_stream, false);
+	}
+	HIP_CHECK(nemo_launch_gather_currents(m_stream, &b, m_devToSim.ptr, E, I, m_tiles));
+	m_hostStep = s + 1;
+	waitStream(m_stream);
+}
+
+void Simulation::propagateDevice(const uint32_t* flags, float** E, float** I)
+{
+	activate();
+	if(!m_extE.ptr) {
 		m_extE.allocate(std::max<size_t>(1, m_ncount));
 		m_extI.allocate(std::max<size_t>(1, m_ncount));
 	}
-	joinStdp();
-	const uint64_t s = m_hostStep;
-	ensureRing();
-	setBase(s);
-	nemo_hip_step_buffers b = stepBuffers(0, false, false);
-	b.debug_current = nullptr;
-	HIP_CHECK(nemo_launch_external_fire(m_stream, &b, flags, m_devToSim.ptr, m_tiles));
-	b.step_offset = 1;
-	if(!m_shape.direct) {
-		launchDelivery(m_early, 1, m_stream, false);
-		launchDelivery(m_late, 1, m_stream, false);
-	}
-	HIP_CHECK(nemo_launch_gather_currents(m_stream, &b, m_devToSim.ptr, m_extE.ptr, m_extI.ptr, m_tiles));
-	m_hostStep = s + 1;
-	HIP_CHECK(hipStreamSynchronize(m_stream));
+	propagateStep(flags, m_extE.ptr, m_extI.ptr);
 	*E = m_extE.ptr;
 	*I = m_extI.ptr;
 }
 
+/* The firing goes to the device as a pinned list of neurons and the input
+ * comes back in pinned memory that the gather writes: flags for every neuron,
+ * two scalars and two arrays copied from pageable memory took 50 us of the 75
+ * a call on 20,000 neurons took. */
 void Simulation::propagate(const unsigned* fired, size_t nfired, float* E, float* I, size_t n)
 {
 	activate();
 	if(n != m_ncount) throw Error(NEMO_INVALID_INPUT, "current arrays must hold one entry per neuron");
-	std::vector<uint32_t> flags(std::max<size_t>(1, m_ncount), 0u);
-	if(nfired) {
-		std::vector<uint32_t> d2s(m_npad, ~0u);
-		for(size_t i = 0; i < m_ncount; ++i) d2s[m_order[i]] = uint32_t(i);
-		for(size_t k = 0; k < nfired; ++k) flags[d2s[localIdx(fired[k])]] = 1u;
+	unsigned char* room = static_cast<unsigned char*>(stageRoom(2 * n * sizeof(float) + nfired * sizeof(uint32_t)));
+	float* hE = reinterpret_cast<float*>(room);
+	float* hI = hE + n;
+	uint32_t* list = reinterpret_cast<uint32_t*>(hI + n);
+	for(size_t k = 0; k < nfired; ++k) list[k] = localIdx(fired[k]);
+	if(m_nets == 1 && !m_stdp) {
+		m_stageBusy = true;
+		HIP_CHECK(nemo_launch_stimulus(m_stream, m_fstim.ptr, list, nfired, nullptr, nullptr, nullptr, 0));
 	}
-	if(m_extFlags.n < flags.size()) m_extFlags.allocate(flags.size());
-	HIP_CHECK(hipMemcpy(m_extFlags.ptr, flags.data(), flags.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-	float* dE = nullptr;
-	float* dI = nullptr;
-	propagateDevice(m_extFlags.ptr, &dE, &dI);
-	HIP_CHECK(hipMemcpy(E, dE, n * sizeof(float), hipMemcpyDeviceToHost));
-	HIP_CHECK(hipMemcpy(I, dI, n * sizeof(float), hipMemcpyDeviceToHost));
+	propagateStep(nullptr, hE, hI);
+	m_stageBusy = false;
+	std::copy(hE, hE + n, E);
+	std::copy(hI, hI + n, I);
 }
 
 /* --------------------------------------------------------- neuron access */
@@ -2845,10 +2860,12 @@ void Simulation::setNeuronParameter(unsigned idx, unsigned param, float val)
 }
 
 /* Vector forms of the neuron getters and setters (the Python binding's list
- * arguments, src/api/python/nemo_py.cpp): a few neurons are read or written
- * element by element; more, plane by plane (each plane of a model that the
- * call touches is copied to the host once, and written back once). */
+ * arguments, src/api/python/nemo_py.cpp): up to GATHERED_MAX neurons are read
+ * by one kernel into pinned memory (a copy each took about 10 us), a few are
+ * written element by element; more, plane by plane (each plane of a model that
+ * the call touches is copied to the host once, and written back once). */
 static const size_t ELEMENTWISE_MAX = 16;
+static const size_t GATHERED_MAX = 4096;
 
 void Simulation::getNeuronValues(bool param, unsigned var, size_t n, const unsigned* idx, float* out)
 {
@@ -2862,16 +2879,27 @@ void Simulation::getNeuronValues(bool param, unsigned var, size_t n, const unsig
 					+ std::to_string(var));
 		}
 	}
+	if(n <= GATHERED_MAX) {
+		unsigned char* room = static_cast<unsigned char*>(stageRoom(n * (sizeof(float*) + sizeof(float))));
+		const float** src = reinterpret_cast<const float**>(room);
+		float* val = reinterpret_cast<float*>(src + n);
+		for(size_t i = 0; i < n; ++i) {
+			const Group& g = groupOf(loc[i]);
+			src[i] = (param ? g.param.ptr + size_t(var) * g.count : statePlane(g, var)) + (loc[i] - g.start);
+		}
+		m_stageBusy = true;
+		HIP_CHECK(nemo_launch_read_values(m_stream, src, val, n));
+		waitStream(m_stream);
+		m_stageBusy = false;
+		std::copy(val, val + n, out);
+		return;
+	}
 	HIP_CHECK(hipStreamSynchronize(m_stream));
 	std::vector<std::vector<float> > planes(m_groups.size());
 	for(size_t i = 0; i < n; ++i) {
 		const int gi = m_typeOfLocal[loc[i]];
 		Group& g = m_groups[gi];
 		const float* plane = (param ? g.param.ptr + size_t(var) * g.count : statePlane(g, var));
-		if(n <= ELEMENTWISE_MAX) {
-			HIP_CHECK(hipMemcpy(out + i, plane + (loc[i] - g.start), 4, hipMemcpyDeviceToHost));
-			continue;
-		}
 		if(planes[gi].empty()) {
 			planes[gi].resize(g.count);
 			HIP_CHECK(hipMemcpy(planes[gi].data(), plane, g.count * sizeof(float), hipMemcpyDeviceToHost));

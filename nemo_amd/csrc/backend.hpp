@@ -192,6 +192,9 @@ public:
 	 * arrays valid until the next call).  Neuron state is not updated. */
 	void propagate(const unsigned* fired, size_t nfired, float* E, float* I, size_t n);
 	void propagateDevice(const uint32_t* flags, float** E, float** I);
+	/* the step of either: the firing from flags, or (NULL) from the stimulus
+	 * bits; the input into E and I, which the device can write */
+	void propagateStep(const uint32_t* flags, float* E, float* I);
 	/* Where run() writes fired neurons: a caller's buffer while it has room,
 	 * then a vector. */
 	struct FiredSink {
@@ -359,8 +362,6 @@ private:
 	DeviceArray<unsigned> m_status;   /* NEMO_HIP_STATUS_* bits set by the kernels */
 	bool m_checkStatus = false;       /* some model may set status bits */
 	DeviceArray<int32_t> m_rcmAcc;
-	DeviceArray<uint32_t> m_stimIdx;
-	DeviceArray<float> m_stimVal;
 	DeviceArray<int2> m_bins;
 	DeviceArray<uint32_t> m_binTable;
 	DeviceArray<uint32_t> m_pairBounds, m_binRange;
@@ -368,7 +369,7 @@ private:
 	DeviceArray<unsigned long long> m_blockEvents, m_blockExamined;
 	/* propagate: device index -> simulation index (~0 for padding), the
 	 * given firing, and the input it produces */
-	DeviceArray<uint32_t> m_devToSim, m_extFlags;
+	DeviceArray<uint32_t> m_devToSim;
 	DeviceArray<float> m_extE, m_extI;
 	std::vector<uint2> m_srcWindow;       /* per source tile: target tiles [x, y) of its synapses */
 	std::vector<uint64_t> m_pairWeight;   /* synapses per (source tile, delay) pair */
@@ -411,6 +412,13 @@ private:
 	uint64_t* m_pinnedScalars = nullptr; /* ring of sources for host-to-device scalars */
 	unsigned m_scalarNext = 0;
 	uint64_t* m_pinnedBits = nullptr;  /* firing bitmaps read back */
+	/* pinned memory that a call hands to its kernels (stimulus lists, values
+	 * asked for and given back): free when no call is under way, as each
+	 * waits for its kernels */
+	unsigned char* m_pinnedStage = nullptr;
+	size_t m_pinnedStageCap = 0;
+	bool m_stageBusy = false;
+	void* stageRoom(size_t bytes);
 	/* run()'s firing readout of a single network, compacted on the device:
 	 * per half (chunks alternate), the steps' counts and fired lists */
 	DeviceArray<uint32_t> m_l2gDev;       /* m_l2g on the device */
@@ -453,8 +461,6 @@ private:
 	void setBase(uint64_t base);
 	void enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, hipEvent_t* ev = nullptr,
 			bool forkPending = true, bool advanceBase = false);
-	/* whether the graphs of steps move the device's step base on themselves */
-	bool graphsAdvanceBase() const;
 	void launchDelivery(const nemo_propagate_args& set, uint64_t offset, hipStream_t st, bool withStdp,
 			hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 	void flushStdp();

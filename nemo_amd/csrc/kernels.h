@@ -97,10 +97,11 @@ hipError_t nemo_launch_invert_rcm(hipStream_t, const uint32_t* rcm_fwd, uint32_t
 		size_t fcm_count);
 
 /* Firing of step base_step + step_offset given from outside (one flag per
- * neuron in simulation order; dev_to_sim maps device index -> simulation
- * index, ~0 for padding): histories and the step's bitmap written as by an
+ * neuron in simulation order, or, flags NULL, a bit per device index, cleared
+ * afterwards; dev_to_sim maps device index -> simulation index, ~0 for
+ * padding): histories and the step's bitmap written as by an
  * update, and, with direct delivery, the events an update would deliver. */
-hipError_t nemo_launch_external_fire(hipStream_t, const nemo_hip_step_buffers* b, const uint32_t* flags,
+hipError_t nemo_launch_external_fire(hipStream_t, const nemo_hip_step_buffers* b, const uint32_t* flags, uint32_t* bits,
 		const uint32_t* dev_to_sim, unsigned tiles);
 /* The ring of a directly delivered network set up from the firing of the
  * steps before t0 (its bitmaps) and the present weights: cleared, then the
@@ -122,11 +123,18 @@ hipError_t nemo_launch_gather_currents(hipStream_t, const nemo_hip_step_buffers*
 hipError_t nemo_launch_fired_list(hipStream_t, const uint64_t* bits, size_t words, uint64_t t0, unsigned k,
 		const uint32_t* l2g, uint32_t* counts, uint32_t* list);
 
-/* Firing stimulus: set (or clear) the bits of the n given device indices. */
-hipError_t nemo_launch_fstim(hipStream_t, uint32_t* bits, const uint32_t* idx, size_t n, int set);
-
-/* Current stimulus: ext[idx[i]] = val[i] (indices must be distinct). */
-hipError_t nemo_launch_istim(hipStream_t, float* ext, const uint32_t* idx, const float* val, size_t n);
+/* The stimulus of a step: bits set for the nf device indices fidx, ext[iidx[i]]
+ * = ival[i] (distinct indices); the lists may be pinned host memory. */
+hipError_t nemo_launch_stimulus(hipStream_t, uint32_t* bits, const uint32_t* fidx, size_t nf, float* ext,
+		const uint32_t* iidx, const float* ival, size_t ni);
+/* After the step: its firing bitmap copied to out (pinned host memory), and
+ * the words of the firing stimulus cleared. */
+hipError_t nemo_launch_step_readout(hipStream_t, const uint64_t* fired, uint64_t* out, size_t words, uint32_t* bits,
+		const uint32_t* fidx, size_t nf);
+/* out[i] = *src[i] (src and out pinned host memory) */
+hipError_t nemo_launch_read_values(hipStream_t, const float* const* src, float* out, size_t n);
+/* clock->base_step += steps */
+hipError_t nemo_launch_advance_clock(hipStream_t, nemo_hip_clock* clock, uint64_t steps);
 
 /* Device logf (fn 0), sinf (fn 1) or expf (fn 2) of n inputs (diagnostics). */
 hipError_t nemo_launch_eval_math(hipStream_t, int fn, const float* in, float* out, size_t n);

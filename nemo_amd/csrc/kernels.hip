@@ -246,10 +246,11 @@ __device__ inline nemo_hip_neuron_group whole_group(unsigned tiles)
 
 /* The firing of step s given from outside (Brian's propagate,
  * cpu/Simulation.cpp:115-137): neuron ng fired if flags[sim] is nonzero for
- * its simulation index sim = dev_to_sim[ng] (~0 for padding); its history
+ * its simulation index sim = dev_to_sim[ng] (~0 for padding), or, without
+ * flags, if its bit in bits is set, which is cleared; its history
  * and the step's bitmap word are written as an update would. */
 __global__ void __launch_bounds__(NEMO_TILE)
-external_fire_kernel(nemo_hip_step_buffers b, const uint32_t* flags, const uint32_t* dev_to_sim)
+external_fire_kernel(nemo_hip_step_buffers b, const uint32_t* flags, uint32_t* bits, const uint32_t* dev_to_sim)
 {
 	nemo_dev::UpdateLds& L = nemo_dev::update_lds<false>();
 	if(b.direct.ring && nemo_dev::direct_block(b, whole_group(b.direct.tiles), L)) return;
@@ -258,7 +259,10 @@ external_fire_kernel(nemo_hip_step_buffers b, const uint32_t* flags, const uint3
 	const bool valid = sim != ~0u;
 	const uint64_t h = nemo_dev::load_history(b, ng, valid);
 	nemo_dev::begin_push(b, L, ng);
-	nemo_dev::record_firing<false>(b, L, ng, valid, valid && flags[sim] != 0u, h);
+	const bool fired = valid && (flags ? flags[sim] != 0u : ((bits[ng >> 5] >> (ng & 31)) & 1u) != 0u);
+	nemo_dev::record_firing<false>(b, L, ng, valid, fired, h);
+	/* the wave has read its two words */
+	if(!flags && (threadIdx.x & 31) == 0) bits[ng >> 5] = 0;
 }
 
 /* ------------------------------------------------------ direct delivery */
@@ -329,20 +333,41 @@ gather_currents_kernel(nemo_hip_step_buffers b, const uint32_t* dev_to_sim, floa
 
 /* ------------------------------------------------------------ stimulus */
 
-__global__ void fstim_kernel(uint32_t* bits, const uint32_t* idx, size_t n, int set)
+/* The stimulus of a step, read from the host's pinned lists: firing bits set,
+ * external currents written (distinct neurons). */
+__global__ void __launch_bounds__(NEMO_BLOCK)
+stimulus_kernel(uint32_t* bits, const uint32_t* fidx, size_t nf, float* ext, const uint32_t* iidx, const float* ival,
+		size_t ni)
 {
 	const size_t i = size_t(blockIdx.x) * NEMO_BLOCK + threadIdx.x;
-	if(i < n) {
-		const uint32_t v = idx[i];
-		if(set) atomicOr(&bits[v >> 5], 1u << (v & 31));
-		else atomicAnd(&bits[v >> 5], ~(1u << (v & 31)));
-	}
+	if(i < nf) atomicOr(&bits[fidx[i] >> 5], 1u << (fidx[i] & 31));
+	if(i < ni) ext[iidx[i]] = ival[i];
 }
 
-__global__ void istim_kernel(float* ext, const uint32_t* idx, const float* val, size_t n)
+/* ... and its end: the step's firing bitmap written to pinned host memory,
+ * the firing stimulus cleared (its words hold no other bits). */
+__global__ void __launch_bounds__(NEMO_BLOCK)
+step_readout_kernel(const uint64_t* fired, uint64_t* out, size_t words, uint32_t* bits, const uint32_t* fidx, size_t nf)
 {
 	const size_t i = size_t(blockIdx.x) * NEMO_BLOCK + threadIdx.x;
-	if(i < n) ext[idx[i]] = val[i];
+	if(i < words) out[i] = fired[i];
+	if(i < nf) bits[fidx[i] >> 5] = 0;
+}
+
+/* out[i] = *src[i], from and to pinned host memory */
+__global__ void __launch_bounds__(NEMO_BLOCK)
+read_values_kernel(const float* const* src, float* out, size_t n)
+{
+	const size_t i = size_t(blockIdx.x) * NEMO_BLOCK + threadIdx.x;
+	if(i < n) out[i] = *src[i];
+}
+
+/* The step base moved on by the last node of a graph of steps, so that the
+ * next graph needs no copy of its base from the host: that copy starts 5 to
+ * 15 us after the last kernel, and the next graph 15 to 20 us after it. */
+__global__ void advance_clock_kernel(nemo_hip_clock* clock, uint64_t steps)
+{
+	clock->base_step += steps;
 }
 
 __global__ void eval_math_kernel(int fn, const float* in, float* out, size_t n)
@@ -507,13 +532,13 @@ hipError_t nemo_launch_invert_rcm(hipStream_t st, const uint32_t* rcm_fwd, uint3
 	return hipGetLastError();
 }
 
-hipError_t nemo_launch_external_fire(hipStream_t st, const nemo_hip_step_buffers* b, const uint32_t* flags,
+hipError_t nemo_launch_external_fire(hipStream_t st, const nemo_hip_step_buffers* b, const uint32_t* flags, uint32_t* bits,
 		const uint32_t* dev_to_sim, unsigned tiles)
 {
 	if(tiles == 0) return hipSuccess;
 	if(b->direct.ring && b->direct.tiles != tiles) return hipErrorInvalidValue;
 	const unsigned blocks = tiles + b->direct.late_blocks;
-	hipLaunchKernelGGL(external_fire_kernel, dim3(blocks), dim3(NEMO_TILE), 0, st, *b, flags, dev_to_sim);
+	hipLaunchKernelGGL(external_fire_kernel, dim3(blocks), dim3(NEMO_TILE), 0, st, *b, flags, bits, dev_to_sim);
 	return hipGetLastError();
 }
 
@@ -555,19 +580,37 @@ hipError_t nemo_launch_fired_list(hipStream_t st, const uint64_t* bits, size_t w
 	return hipGetLastError();
 }
 
-hipError_t nemo_launch_fstim(hipStream_t st, uint32_t* bits, const uint32_t* idx, size_t n, int set)
+hipError_t nemo_launch_stimulus(hipStream_t st, uint32_t* bits, const uint32_t* fidx, size_t nf, float* ext,
+		const uint32_t* iidx, const float* ival, size_t ni)
 {
+	const size_t n = std::max(nf, ni);
 	if(n == 0) return hipSuccess;
-	hipLaunchKernelGGL(fstim_kernel, dim3(unsigned((n + NEMO_BLOCK - 1) / NEMO_BLOCK)), dim3(NEMO_BLOCK), 0, st,
-			bits, idx, n, set);
+	hipLaunchKernelGGL(stimulus_kernel, dim3(unsigned((n + NEMO_BLOCK - 1) / NEMO_BLOCK)), dim3(NEMO_BLOCK), 0, st, bits,
+			fidx, nf, ext, iidx, ival, ni);
 	return hipGetLastError();
 }
 
-hipError_t nemo_launch_istim(hipStream_t st, float* ext, const uint32_t* idx, const float* val, size_t n)
+hipError_t nemo_launch_step_readout(hipStream_t st, const uint64_t* fired, uint64_t* out, size_t words, uint32_t* bits,
+		const uint32_t* fidx, size_t nf)
+{
+	const size_t n = std::max(words, nf);
+	if(n == 0) return hipSuccess;
+	hipLaunchKernelGGL(step_readout_kernel, dim3(unsigned((n + NEMO_BLOCK - 1) / NEMO_BLOCK)), dim3(NEMO_BLOCK), 0, st,
+			fired, out, words, bits, fidx, nf);
+	return hipGetLastError();
+}
+
+hipError_t nemo_launch_read_values(hipStream_t st, const float* const* src, float* out, size_t n)
 {
 	if(n == 0) return hipSuccess;
-	hipLaunchKernelGGL(istim_kernel, dim3(unsigned((n + NEMO_BLOCK - 1) / NEMO_BLOCK)), dim3(NEMO_BLOCK), 0, st,
-			ext, idx, val, n);
+	hipLaunchKernelGGL(read_values_kernel, dim3(unsigned((n + NEMO_BLOCK - 1) / NEMO_BLOCK)), dim3(NEMO_BLOCK), 0, st,
+			src, out, n);
+	return hipGetLastError();
+}
+
+hipError_t nemo_launch_advance_clock(hipStream_t st, nemo_hip_clock* clock, uint64_t steps)
+{
+	hipLaunchKernelGGL(advance_clock_kernel, dim3(1), dim3(1), 0, st, clock, steps);
 	return hipGetLastError();
 }
 
