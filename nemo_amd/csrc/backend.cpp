@@ -600,6 +600,7 @@ Simulation::~Simulation()
 	if(m_pinnedScalars) (void) hipHostFree(m_pinnedScalars);
 	if(m_pinnedBits) (void) hipHostFree(m_pinnedBits);
 	if(m_pinnedStage) (void) hipHostFree(m_pinnedStage);
+	if(m_pinnedFlag) (void) hipHostFree(m_pinnedFlag);
 	if(m_pinnedCounters) (void) hipHostFree(m_pinnedCounters);
 	if(m_pinnedListCounts) (void) hipHostFree(m_pinnedListCounts);
 	for(uint32_t* p : m_pinnedList) {
@@ -1549,6 +1550,10 @@ void Simulation::allocateStepState()
 	HIP_CHECK(hipMemset(m_ext.ptr, 0, m_ext.bytes()));
 	m_fstim.allocate((N + 31) / 32);
 	HIP_CHECK(hipMemset(m_fstim.ptr, 0, m_fstim.bytes()));
+	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&m_pinnedFlag), sizeof(uint64_t), hipHostMallocDefault));
+	*m_pinnedFlag = 0;
+	m_signalBlocks.allocate(1);
+	HIP_CHECK(hipMemset(m_signalBlocks.ptr, 0, m_signalBlocks.bytes()));
 	m_status.allocate(1);
 	HIP_CHECK(hipMemset(m_status.ptr, 0, m_status.bytes()));
 	m_debugCurrent.allocate(2 * m_accPitch);
@@ -2114,14 +2119,49 @@ const std::vector<unsigned>& Simulation::step(const unsigned* fstim, size_t nf,
 	ensureRing();
 	enqueueSteps(t - m_base, 1, !iIdx.empty(), !fIdx.empty());
 	advanceSteps(1);
+	const nemo_host_signal done = nextSignal();
 	HIP_CHECK(nemo_launch_step_readout(m_stream, m_firedBits.ptr + (t & (NEMO_STEP_RING - 1)) * m_firedWords, m_pinnedBits,
-				m_firedWords, m_fstim.ptr, fList, nf));
-	waitStream(m_stream);
+				m_firedWords, m_fstim.ptr, fList, nf, &done));
+	waitSignal(done);
 	m_stageBusy = false;
 	checkStatus();
 	m_firedOut.clear();
 	decodeFiring(m_pinnedBits, m_firedOut);
 	return m_firedOut;
+}
+
+nemo_host_signal Simulation::nextSignal()
+{
+	nemo_host_signal s;
+	s.flag = m_pinnedFlag;
+	s.value = ++m_signalled;
+	s.blocks = m_signalBlocks.ptr;
+	return s;
+}
+
+/* Poll the flag of the stream's last signal.  What was queued before it has
+ * run then; an error on the way shows in the stream's state, which is asked
+ * for every now and then (it costs more than the wait). */
+void Simulation::waitSignal(const nemo_host_signal& done)
+{
+	auto asked = std::chrono::steady_clock::now();
+	for(;;) {
+		for(int i = 0; i < 64; ++i) {
+			if(__atomic_load_n(done.flag, __ATOMIC_ACQUIRE) >= done.value) return;
+#if defined(__x86_64__)
+			__builtin_ia32_pause();
+#endif
+		}
+		const auto t = std::chrono::steady_clock::now();
+		if(t - asked > std::chrono::milliseconds(2)) {
+			const hipError_t e = hipStreamQuery(m_stream);
+			if(e != hipErrorNotReady) HIP_CHECK(e);
+			if(e == hipSuccess && __atomic_load_n(done.flag, __ATOMIC_ACQUIRE) < done.value) {
+				throw Error(NEMO_CUDA_INVOCATION_ERROR, "a kernel ended without its signal");
+			}
+			asked = t;
+		}
+	}
 }
 
 /* Pinned room for a call's lists, and for what its kernels give back. */
@@ -2742,9 +2782,10 @@ void Simulation::propagateStep(const uint32_t* flags, float* E, float* I)
 		launchDelivery(m_early, off + 1, m_stream, false);
 		launchDelivery(m_late, off + 1, m_stream, false);
 	}
-	HIP_CHECK(nemo_launch_gather_currents(m_stream, &b, m_devToSim.ptr, E, I, m_tiles));
+	const nemo_host_signal done = nextSignal();
+	HIP_CHECK(nemo_launch_gather_currents(m_stream, &b, m_devToSim.ptr, E, I, m_tiles, &done));
 	m_hostStep = s + 1;
-	waitStream(m_stream);
+	waitSignal(done);
 }
 
 void Simulation::propagateDevice(const uint32_t* flags, float** E, float** I)
@@ -2755,6 +2796,7 @@ void Simulation::propagateDevice(const uint32_t* flags, float** E, float** I)
 		m_extI.allocate(std::max<size_t>(1, m_ncount));
 	}
 	propagateStep(flags, m_extE.ptr, m_extI.ptr);
+	HIP_CHECK(hipStreamSynchronize(m_stream)); /* for the caller's own streams */
 	*E = m_extE.ptr;
 	*I = m_extI.ptr;
 }
@@ -2888,8 +2930,9 @@ void Simulation::getNeuronValues(bool param, unsigned var, size_t n, const unsig
 			src[i] = (param ? g.param.ptr + size_t(var) * g.count : statePlane(g, var)) + (loc[i] - g.start);
 		}
 		m_stageBusy = true;
-		HIP_CHECK(nemo_launch_read_values(m_stream, src, val, n));
-		waitStream(m_stream);
+		const nemo_host_signal done = nextSignal();
+		HIP_CHECK(nemo_launch_read_values(m_stream, src, val, n, &done));
+		waitSignal(done);
 		m_stageBusy = false;
 		std::copy(val, val + n, out);
 		return;

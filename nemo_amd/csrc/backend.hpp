@@ -419,6 +419,13 @@ private:
 	size_t m_pinnedStageCap = 0;
 	bool m_stageBusy = false;
 	void* stageRoom(size_t bytes);
+	/* the flag that a call's last kernel sets in pinned memory when its
+	 * results are there, and the value of the last signal handed out */
+	uint64_t* m_pinnedFlag = nullptr;
+	uint64_t m_signalled = 0;
+	DeviceArray<unsigned> m_signalBlocks;
+	nemo_host_signal nextSignal();
+	void waitSignal(const nemo_host_signal& done);
 	/* run()'s firing readout of a single network, compacted on the device:
 	 * per half (chunks alternate), the steps' counts and fired lists */
 	DeviceArray<uint32_t> m_l2gDev;       /* m_l2g on the device */

@@ -42,6 +42,17 @@ extern "C" {
 #define NEMO_STDP_BATCH_WORDS 6
 
 
+/* A kernel's word to the host that what it wrote to pinned memory is there:
+ * value into flag (pinned), by the last of its blocks; blocks (device memory,
+ * 0 before and after) counts them.  The host sees it 7 us after a launch on an
+ * idle stream, where hipStreamSynchronize returns after 13 and a polled
+ * hipStreamQuery after 24. */
+typedef struct nemo_host_signal {
+	uint64_t* flag; /* NULL: no signal (where a kernel allows it) */
+	uint64_t value;
+	unsigned* blocks;
+} nemo_host_signal;
+
 /* dynamic LDS bytes a delivery block needs */
 size_t nemo_propagate_lds_bytes(unsigned max_window, unsigned bin_capacity);
 /* The pending STDP accumulation (clock->stdp_first, stdp_count) in one launch
@@ -114,7 +125,7 @@ hipError_t nemo_launch_direct_rebuild(hipStream_t, const nemo_hip_direct* r, siz
  * cleared, which no update has read) and written as floats in simulation
  * order. */
 hipError_t nemo_launch_gather_currents(hipStream_t, const nemo_hip_step_buffers* b, const uint32_t* dev_to_sim,
-		float* E, float* I, unsigned tiles);
+		float* E, float* I, unsigned tiles, const nemo_host_signal* done);
 
 /* Firing readout of k steps from step t0 (their firing-bitmap ring slots,
  * words words each): counts[s] the neurons fired in step t0 + s, and list
@@ -130,9 +141,10 @@ hipError_t nemo_launch_stimulus(hipStream_t, uint32_t* bits, const uint32_t* fid
 /* After the step: its firing bitmap copied to out (pinned host memory), and
  * the words of the firing stimulus cleared. */
 hipError_t nemo_launch_step_readout(hipStream_t, const uint64_t* fired, uint64_t* out, size_t words, uint32_t* bits,
-		const uint32_t* fidx, size_t nf);
+		const uint32_t* fidx, size_t nf, const nemo_host_signal* done);
 /* out[i] = *src[i] (src and out pinned host memory) */
-hipError_t nemo_launch_read_values(hipStream_t, const float* const* src, float* out, size_t n);
+hipError_t nemo_launch_read_values(hipStream_t, const float* const* src, float* out, size_t n,
+		const nemo_host_signal* done);
 /* clock->base_step += steps */
 hipError_t nemo_launch_advance_clock(hipStream_t, nemo_hip_clock* clock, uint64_t steps);
 

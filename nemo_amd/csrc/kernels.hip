@@ -234,6 +234,22 @@ fired_list_kernel(const uint64_t* bits, size_t words, uint64_t t0, const uint32_
 	}
 }
 
+/* Tells the host, which polls done->flag in pinned memory, that the kernel's
+ * writes to pinned memory are there: by the last of its blocks to get here,
+ * every thread of which calls it (done->blocks counts them, and ends at 0). */
+__device__ inline void signal_done(const nemo_host_signal& done)
+{
+	__threadfence_system();
+	__syncthreads();
+	if(threadIdx.x != 0) return;
+	if(gridDim.x > 1) {
+		if(atomicAdd(done.blocks, 1u) + 1 < gridDim.x) return;
+		*done.blocks = 0;
+		__threadfence_system();
+	}
+	__hip_atomic_store(done.flag, done.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 /* ------------------------------------------- externally given firing */
 
 /* All tiles as one group, for the blocks that need no more of it. */
@@ -299,7 +315,7 @@ direct_rebuild_kernel(nemo_hip_direct r, size_t acc_pitch, const uint32_t* rowpt
  * gather it (overflow accumulators cleared), converted to float and written
  * in simulation order: E[sim], I[sim]. */
 __global__ void __launch_bounds__(NEMO_TILE)
-gather_currents_kernel(nemo_hip_step_buffers b, const uint32_t* dev_to_sim, float* E, float* I)
+gather_currents_kernel(nemo_hip_step_buffers b, const uint32_t* dev_to_sim, float* E, float* I, nemo_host_signal done)
 {
 	nemo_dev::UpdateLds& L = nemo_dev::update_lds<false>();
 	const nemo_hip_neuron_group g = whole_group(gridDim.x);
@@ -329,6 +345,7 @@ gather_currents_kernel(nemo_hip_step_buffers b, const uint32_t* dev_to_sim, floa
 		E[sim] = e;
 		I[sim] = i;
 	}
+	if(done.flag) signal_done(done);
 }
 
 /* ------------------------------------------------------------ stimulus */
@@ -345,21 +362,23 @@ stimulus_kernel(uint32_t* bits, const uint32_t* fidx, size_t nf, float* ext, con
 }
 
 /* ... and its end: the step's firing bitmap written to pinned host memory,
- * the firing stimulus cleared (its words hold no other bits). */
+ * the firing stimulus cleared (its words hold no other bits).  One block. */
 __global__ void __launch_bounds__(NEMO_BLOCK)
-step_readout_kernel(const uint64_t* fired, uint64_t* out, size_t words, uint32_t* bits, const uint32_t* fidx, size_t nf)
+step_readout_kernel(const uint64_t* fired, uint64_t* out, size_t words, uint32_t* bits, const uint32_t* fidx, size_t nf,
+		nemo_host_signal done)
 {
-	const size_t i = size_t(blockIdx.x) * NEMO_BLOCK + threadIdx.x;
-	if(i < words) out[i] = fired[i];
-	if(i < nf) bits[fidx[i] >> 5] = 0;
+	for(size_t i = threadIdx.x; i < words; i += NEMO_BLOCK) out[i] = fired[i];
+	for(size_t i = threadIdx.x; i < nf; i += NEMO_BLOCK) bits[fidx[i] >> 5] = 0;
+	signal_done(done);
 }
 
 /* out[i] = *src[i], from and to pinned host memory */
 __global__ void __launch_bounds__(NEMO_BLOCK)
-read_values_kernel(const float* const* src, float* out, size_t n)
+read_values_kernel(const float* const* src, float* out, size_t n, nemo_host_signal done)
 {
 	const size_t i = size_t(blockIdx.x) * NEMO_BLOCK + threadIdx.x;
 	if(i < n) out[i] = *src[i];
+	signal_done(done);
 }
 
 /* The step base moved on by the last node of a graph of steps, so that the
@@ -561,10 +580,10 @@ hipError_t nemo_launch_direct_rebuild(hipStream_t st, const nemo_hip_direct* r, 
 }
 
 hipError_t nemo_launch_gather_currents(hipStream_t st, const nemo_hip_step_buffers* b, const uint32_t* dev_to_sim,
-		float* E, float* I, unsigned tiles)
+		float* E, float* I, unsigned tiles, const nemo_host_signal* done)
 {
-	if(tiles == 0) return hipSuccess;
-	hipLaunchKernelGGL(gather_currents_kernel, dim3(tiles), dim3(NEMO_TILE), 0, st, *b, dev_to_sim, E, I);
+	if(tiles == 0) return hipErrorInvalidValue; /* no block to signal */
+	hipLaunchKernelGGL(gather_currents_kernel, dim3(tiles), dim3(NEMO_TILE), 0, st, *b, dev_to_sim, E, I, *done);
 	return hipGetLastError();
 }
 
@@ -591,20 +610,17 @@ hipError_t nemo_launch_stimulus(hipStream_t st, uint32_t* bits, const uint32_t* 
 }
 
 hipError_t nemo_launch_step_readout(hipStream_t st, const uint64_t* fired, uint64_t* out, size_t words, uint32_t* bits,
-		const uint32_t* fidx, size_t nf)
+		const uint32_t* fidx, size_t nf, const nemo_host_signal* done)
 {
-	const size_t n = std::max(words, nf);
-	if(n == 0) return hipSuccess;
-	hipLaunchKernelGGL(step_readout_kernel, dim3(unsigned((n + NEMO_BLOCK - 1) / NEMO_BLOCK)), dim3(NEMO_BLOCK), 0, st,
-			fired, out, words, bits, fidx, nf);
+	hipLaunchKernelGGL(step_readout_kernel, dim3(1), dim3(NEMO_BLOCK), 0, st, fired, out, words, bits, fidx, nf, *done);
 	return hipGetLastError();
 }
 
-hipError_t nemo_launch_read_values(hipStream_t st, const float* const* src, float* out, size_t n)
+hipError_t nemo_launch_read_values(hipStream_t st, const float* const* src, float* out, size_t n,
+		const nemo_host_signal* done)
 {
-	if(n == 0) return hipSuccess;
-	hipLaunchKernelGGL(read_values_kernel, dim3(unsigned((n + NEMO_BLOCK - 1) / NEMO_BLOCK)), dim3(NEMO_BLOCK), 0, st,
-			src, out, n);
+	const size_t blocks = std::max<size_t>(1, (n + NEMO_BLOCK - 1) / NEMO_BLOCK);
+	hipLaunchKernelGGL(read_values_kernel, dim3(unsigned(blocks)), dim3(NEMO_BLOCK), 0, st, src, out, n, *done);
 	return hipGetLastError();
 }
 
