@@ -505,15 +505,11 @@ void Simulation::construct(const std::vector<const Network*>& nets, const Config
 	HIP_CHECK(hipEventCreateWithFlags(&m_stdpLag[0], hipEventDisableTiming));
 	HIP_CHECK(hipEventCreateWithFlags(&m_stdpLag[1], hipEventDisableTiming));
 	HIP_CHECK(hipStreamCreateWithFlags(&m_earlyStream, hipStreamNonBlocking));
-	HIP_CHECK(hipStreamCreateWithFlags(&m_copyStream, hipStreamNonBlocking));
 	HIP_CHECK(hipStreamCreateWithFlags(&m_restStream, hipStreamNonBlocking));
+	HIP_CHECK(hipEventCreateWithFlags(&m_waitEvent, hipEventDisableTiming));
 	HIP_CHECK(hipEventCreateWithFlags(&m_earlyFork, hipEventDisableTiming));
 	HIP_CHECK(hipEventCreateWithFlags(&m_earlyDone[0], hipEventDisableTiming));
 	HIP_CHECK(hipEventCreateWithFlags(&m_earlyDone[1], hipEventDisableTiming));
-	for(int i = 0; i < 2; ++i) {
-		HIP_CHECK(hipEventCreateWithFlags(&m_readoutReady[i], hipEventDisableTiming));
-		HIP_CHECK(hipEventCreateWithFlags(&m_readoutCopied[i], hipEventDisableTiming));
-	}
 	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&m_pinnedScalars), SCALAR_SLOTS * sizeof(uint64_t),
 				hipHostMallocDefault));
 
@@ -565,14 +561,13 @@ Simulation::~Simulation()
 	if(m_stream) (void) hipStreamSynchronize(m_stream);
 	if(m_stdpStream) (void) hipStreamSynchronize(m_stdpStream);
 	if(m_earlyStream) (void) hipStreamSynchronize(m_earlyStream);
-	if(m_copyStream) (void) hipStreamSynchronize(m_copyStream);
 	if(m_restStream) (void) hipStreamSynchronize(m_restStream);
 	for(hipStream_t q : m_groupStreams) {
 		if(q) (void) hipStreamSynchronize(q);
 	}
 	clearGraphs();
-	if(m_copyStream) (void) hipStreamDestroy(m_copyStream);
 	if(m_restStream) (void) hipStreamDestroy(m_restStream);
+	if(m_waitEvent) (void) hipEventDestroy(m_waitEvent);
 	for(hipStream_t q : m_groupStreams) {
 		if(q) (void) hipStreamDestroy(q);
 	}
@@ -580,9 +575,6 @@ Simulation::~Simulation()
 		if(e) (void) hipEventDestroy(e);
 	}
 	if(m_groupFork) (void) hipEventDestroy(m_groupFork);
-	for(hipEvent_t e : {m_readoutReady[0], m_readoutReady[1], m_readoutCopied[0], m_readoutCopied[1]}) {
-		if(e) (void) hipEventDestroy(e);
-	}
 	if(m_earlyStream) {
 		(void) hipStreamDestroy(m_earlyStream);
 		(void) hipEventDestroy(m_earlyFork);
@@ -601,9 +593,8 @@ Simulation::~Simulation()
 	if(m_pinnedBits) (void) hipHostFree(m_pinnedBits);
 	if(m_pinnedStage) (void) hipHostFree(m_pinnedStage);
 	if(m_pinnedFlag) (void) hipHostFree(m_pinnedFlag);
-	if(m_pinnedCounters) (void) hipHostFree(m_pinnedCounters);
-	if(m_pinnedListCounts) (void) hipHostFree(m_pinnedListCounts);
-	for(uint32_t* p : m_pinnedList) {
+	for(void* p : {static_cast<void*>(m_pinnedCounts), static_cast<void*>(m_pinnedLists),
+			static_cast<void*>(m_pinnedStepFlag), static_cast<void*>(m_pinnedEvents)}) {
 		if(p) (void) hipHostFree(p);
 	}
 }
@@ -1552,7 +1543,7 @@ void Simulation::allocateStepState()
 	HIP_CHECK(hipMemset(m_fstim.ptr, 0, m_fstim.bytes()));
 	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&m_pinnedFlag), sizeof(uint64_t), hipHostMallocDefault));
 	*m_pinnedFlag = 0;
-	m_signalBlocks.allocate(1);
+	m_signalBlocks.allocate(2); /* nextSignal's kernels, the readout */
 	HIP_CHECK(hipMemset(m_signalBlocks.ptr, 0, m_signalBlocks.bytes()));
 	m_status.allocate(1);
 	HIP_CHECK(hipMemset(m_status.ptr, 0, m_status.bytes()));
@@ -1567,9 +1558,9 @@ void Simulation::allocateStepState()
 	/* per table column, then per 64 device indices (events pushed by updates) */
 	m_blockEvents.allocate(NEMO_MAX_BIN_BLOCKS + m_npad / 64);
 	HIP_CHECK(hipMemset(m_blockEvents.ptr, 0, m_blockEvents.bytes()));
-	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&m_pinnedCounters), 2 * m_blockEvents.bytes(),
-				hipHostMallocDefault));
-	std::memset(m_pinnedCounters, 0, 2 * m_blockEvents.bytes());
+	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&m_pinnedEvents), 2 * sizeof(uint64_t), hipHostMallocDefault));
+	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&m_pinnedStepFlag), sizeof(uint64_t), hipHostMallocDefault));
+	*m_pinnedStepFlag = 0;
 	m_blockExamined.allocate(std::max<size_t>(1, m_firedWords));
 	HIP_CHECK(hipMemset(m_blockExamined.ptr, 0, m_blockExamined.bytes()));
 
@@ -1657,15 +1648,16 @@ void Simulation::copyScalar(uint64_t* dst, uint64_t value)
 	HIP_CHECK(hipMemcpyAsync(dst, slot, sizeof(uint64_t), hipMemcpyHostToDevice, m_stream));
 }
 
-/* Wait for an event (or a stream) by polling it for up to 50 ms before the
+/* Wait for a stream by polling an event on it for up to 50 ms before the
  * blocking wait: a blocking wait can put the thread to sleep and wake it
- * milliseconds after the work ended, which costs more than a whole short
- * run of steps. */
-static void pollThenWait(hipError_t (*query)(void*), hipError_t (*wait)(void*), void* x)
+ * milliseconds after the work ended, which costs more than a whole short run
+ * of steps. */
+void Simulation::waitStream(hipStream_t st)
 {
+	HIP_CHECK(hipEventRecord(m_waitEvent, st));
 	const auto t0 = std::chrono::steady_clock::now();
 	for(;;) {
-		const hipError_t e = query(x);
+		const hipError_t e = hipEventQuery(m_waitEvent);
 		if(e == hipSuccess) return;
 		if(e != hipErrorNotReady) HIP_CHECK(e);
 		if(std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(50)) break;
@@ -1673,19 +1665,7 @@ static void pollThenWait(hipError_t (*query)(void*), hipError_t (*wait)(void*), 
 		__builtin_ia32_pause();
 #endif
 	}
-	HIP_CHECK(wait(x));
-}
-
-void Simulation::waitEvent(hipEvent_t e)
-{
-	pollThenWait([](void* x) { return hipEventQuery(static_cast<hipEvent_t>(x)); },
-			[](void* x) { return hipEventSynchronize(static_cast<hipEvent_t>(x)); }, e);
-}
-
-void Simulation::waitStream(hipStream_t s)
-{
-	pollThenWait([](void* x) { return hipStreamQuery(static_cast<hipStream_t>(x)); },
-			[](void* x) { return hipStreamSynchronize(static_cast<hipStream_t>(x)); }, s);
+	HIP_CHECK(hipStreamSynchronize(st));
 }
 
 /* The step base used by the next launches: step = base + launch offset. */
@@ -1734,7 +1714,7 @@ void Simulation::launchDelivery(const nemo_propagate_args& set, uint64_t offset,
  * step), the kernels record the start and end of the step's delivery on this
  * stream and of its neuron updates. */
 void Simulation::enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, hipEvent_t* ev, bool forkPending,
-		bool advanceBase)
+		bool advanceBase, bool readout)
 {
 	/* direct delivery: the updates are the whole step */
 	const bool direct = m_shape.direct;
@@ -1888,6 +1868,15 @@ void Simulation::enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, 
 			if(ev) HIP_CHECK(hipEventRecord(ev[4 * i + 3], m_stream));
 		}
 		if(overlap && i + 2 < k) forkEarly(i + 2);
+		if(readout && i + 1 == k) {
+			/* before the snapshot, which may wait for the STDP batch */
+			nemo_host_signal done;
+			done.flag = m_pinnedStepFlag;
+			done.value = k;
+			done.blocks = m_signalBlocks.ptr + 1;
+			HIP_CHECK(nemo_launch_fired_readout(m_stream, m_clock.ptr, first, k, m_firedBits.ptr, m_firedWords,
+						m_nets == 1 ? m_l2gDev.ptr : nullptr, m_pinnedCounts, m_pinnedLists, m_readoutRoom, &done));
+		}
 		if(batched && (i + 1 == k || (i + 1) % 64 == 0)) {
 			/* snapshot after this step: the steps since the last one are
 			 * pending for the next batch */
@@ -2017,43 +2006,25 @@ void Simulation::decodeFiring(const uint64_t* bits, Out& out) const
 	appendFired(out, d, pos);
 }
 
-/* Fired neurons of every network of a batch for one step: out gets each
- * network's user indices in turn, in that network's simulation order, and
- * counts one entry per network. */
+/* Fired neurons of every network of a batch for one step, from its list of
+ * device indices: out gets each network's user indices in turn, in that
+ * network's simulation order, and counts one entry per network. */
 template<typename Out>
-void Simulation::decodeFiringBatch(const uint64_t* bits, Out& out, std::vector<unsigned>& counts) const
+void Simulation::decodeListBatch(const uint32_t* fired, size_t n, Out& out, std::vector<unsigned>& counts) const
 {
-	if(m_nets == 1) {
-		const size_t before = out.size();
-		decodeFiring(bits, out);
-		counts.push_back(unsigned(out.size() - before));
-		return;
-	}
 	if(m_decodeInOrder) {
 		const size_t c0 = counts.size();
 		counts.resize(c0 + m_nets, 0u);
-		for(size_t w = 0; w < m_firedWords; ++w) {
-			uint64_t word = bits[w];
-			while(word) {
-				const unsigned l = unsigned(w * 64 + unsigned(__builtin_ctzll(word)));
-				word &= word - 1;
-				out.push_back(m_l2g[l]);
-				++counts[c0 + m_netOf[l]];
-			}
+		for(size_t i = 0; i < n; ++i) {
+			out.push_back(m_l2g[fired[i]]);
+			++counts[c0 + m_netOf[fired[i]]];
 		}
 		return;
 	}
 	std::vector<std::vector<unsigned> >& per = m_decodePer; /* kept between steps: no allocation per step */
 	per.resize(m_nets);
 	for(std::vector<unsigned>& v : per) v.clear();
-	for(size_t w = 0; w < m_firedWords; ++w) {
-		uint64_t word = bits[w];
-		while(word) {
-			const unsigned bit = unsigned(__builtin_ctzll(word));
-			word &= word - 1;
-			per[m_netOf[w * 64 + bit]].push_back(unsigned(w * 64 + bit));
-		}
-	}
+	for(size_t i = 0; i < n; ++i) per[m_netOf[fired[i]]].push_back(fired[i]);
 	for(unsigned k = 0; k < m_nets; ++k) {
 		std::vector<unsigned>& v = per[k];
 		if(m_reorder[k]) {
@@ -2139,15 +2110,15 @@ nemo_host_signal Simulation::nextSignal()
 	return s;
 }
 
-/* Poll the flag of the stream's last signal.  What was queued before it has
- * run then; an error on the way shows in the stream's state, which is asked
- * for every now and then (it costs more than the wait). */
-void Simulation::waitSignal(const nemo_host_signal& done)
+/* Poll a flag that a kernel queued on the stream sets.  What was queued before
+ * that kernel has run then; an error on the way shows in the stream's state,
+ * which is asked for every now and then (it costs more than the wait). */
+void Simulation::waitFlag(const uint64_t* flag, uint64_t value)
 {
 	auto asked = std::chrono::steady_clock::now();
 	for(;;) {
 		for(int i = 0; i < 64; ++i) {
-			if(__atomic_load_n(done.flag, __ATOMIC_ACQUIRE) >= done.value) return;
+			if(__atomic_load_n(flag, __ATOMIC_ACQUIRE) >= value) return;
 #if defined(__x86_64__)
 			__builtin_ia32_pause();
 #endif
@@ -2156,12 +2127,17 @@ void Simulation::waitSignal(const nemo_host_signal& done)
 		if(t - asked > std::chrono::milliseconds(2)) {
 			const hipError_t e = hipStreamQuery(m_stream);
 			if(e != hipErrorNotReady) HIP_CHECK(e);
-			if(e == hipSuccess && __atomic_load_n(done.flag, __ATOMIC_ACQUIRE) < done.value) {
+			if(e == hipSuccess && __atomic_load_n(flag, __ATOMIC_ACQUIRE) < value) {
 				throw Error(NEMO_CUDA_INVOCATION_ERROR, "a kernel ended without its signal");
 			}
 			asked = t;
 		}
 	}
+}
+
+void Simulation::waitSignal(const nemo_host_signal& done)
+{
+	waitFlag(done.flag, done.value);
 }
 
 /* Pinned room for a call's lists, and for what its kernels give back. */
@@ -2183,9 +2159,10 @@ void* Simulation::stageRoom(size_t bytes)
 	return m_pinnedStage;
 }
 
-hipGraphExec_t Simulation::graphFor(unsigned k, bool forkPending)
+hipGraphExec_t Simulation::graphFor(unsigned k, bool forkPending, bool readout)
 {
-	const unsigned key = 2 * k + (forkPending ? 1u : 0u);
+	if(readout) ensureReadout();
+	const unsigned key = 4 * k + (forkPending ? 2u : 0u) + (readout ? 1u : 0u);
 	auto it = m_graphs.find(key);
 	if(it != m_graphs.end()) return it->second;
 	hipGraph_t graph;
@@ -2193,7 +2170,7 @@ hipGraphExec_t Simulation::graphFor(unsigned k, bool forkPending)
 	const bool debug = m_debug;
 	m_debug = false;
 	try {
-		enqueueSteps(0, k, false, false, nullptr, forkPending, true);
+		enqueueSteps(0, k, false, false, nullptr, forkPending, true, readout);
 	} catch(...) {
 		m_debug = debug;
 		m_stdpPending = false;
@@ -2226,45 +2203,27 @@ uint64_t Simulation::sumCounters(const DeviceArray<unsigned long long>& a)
 	return s;
 }
 
-/* The device-compacted firing readout of run() for a single network, set
- * up on first use; false (bitmaps decoded on the host instead) for batches
- * or when its lists would take more than 1 GiB. */
-bool Simulation::ensureListReadout()
+/* The pinned memory of the firing readout, set up on first use: room for all
+ * neurons of a small network, for one in 16 of a large one (a step that fires
+ * more has its bitmap copied). */
+void Simulation::ensureReadout()
 {
-	if(m_nets != 1) return false;
-	const size_t CHUNK = NEMO_STEP_RING / 2;
-	if(m_listDev.n) return true;
-	if(2 * CHUNK * m_npad * sizeof(uint32_t) > (size_t(1) << 30)) return false;
-	m_l2gDev.allocate(m_npad);
-	HIP_CHECK(hipMemcpy(m_l2gDev.ptr, m_l2g.data(), m_l2gDev.bytes(), hipMemcpyHostToDevice));
-	m_listDev.allocate(2 * CHUNK * m_npad);
-	m_listCountsDev.allocate(2 * CHUNK);
-	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&m_pinnedListCounts), 2 * CHUNK * sizeof(uint32_t),
+	if(m_pinnedLists) return;
+	m_readoutRoom = unsigned(std::min<size_t>(m_npad, std::min<size_t>(262144, std::max<size_t>(4096, m_npad / 16))));
+	if(m_nets == 1) {
+		m_l2gDev.allocate(m_npad);
+		HIP_CHECK(hipMemcpy(m_l2gDev.ptr, m_l2g.data(), m_l2gDev.bytes(), hipMemcpyHostToDevice));
+	}
+	const size_t bytes = size_t(NEMO_STEP_RING) * m_readoutRoom * sizeof(uint32_t);
+	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&m_pinnedCounts), NEMO_STEP_RING * sizeof(uint32_t),
 				hipHostMallocDefault));
-	std::memset(m_pinnedListCounts, 0, 2 * CHUNK * sizeof(uint32_t));
-	for(int h = 0; h < 2; ++h) growPinnedList(h, std::max<size_t>(65536, CHUNK * m_npad / 32), 0);
-	return true;
+	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&m_pinnedLists), bytes, hipHostMallocDefault));
+	std::memset(m_pinnedLists, 0, bytes); /* its pages faulted in now, not by the readout */
 }
 
-/* Room for need entries in half h's pinned list, keeping its first keep. */
-void Simulation::growPinnedList(int h, size_t need, size_t keep)
-{
-	if(need <= m_pinnedListCap[h]) return;
-	const size_t cap = std::max(need, 2 * m_pinnedListCap[h]);
-	uint32_t* p = nullptr;
-	HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&p), cap * sizeof(uint32_t), hipHostMallocDefault));
-	std::memset(p, 0, cap * sizeof(uint32_t)); /* its pages faulted in now, not by the readout */
-	if(keep) std::memcpy(p, m_pinnedList[h], keep * sizeof(uint32_t));
-	if(m_pinnedList[h]) HIP_CHECK(hipHostFree(m_pinnedList[h]));
-	m_pinnedList[h] = p;
-	m_pinnedListCap[h] = cap;
-}
-
-/* Steps without stimulus, captured in graphs of up to 64 steps; the firing
- * of each graph's steps is read back after it: for a single network as
- * per-step counts and a fired list compacted on the device (the list's
- * expected length copied with the counts, any rest once they are known),
- * for a batch as bitmaps decoded on the host. */
+/* Steps without stimulus, captured in graphs of up to 64 steps; each graph
+ * ends by writing its steps' fired neurons into pinned memory and a flag for
+ * the host, which takes them from there beside the next graph. */
 void Simulation::run(unsigned nsteps, unsigned stdpPeriod, float reward, bool readRaster,
 		std::vector<unsigned>* counts, FiredSink* fired, uint64_t* events)
 {
@@ -2272,17 +2231,12 @@ void Simulation::run(unsigned nsteps, unsigned stdpPeriod, float reward, bool re
 	if(stdpPeriod && !m_stdp) {
 		throw Error(NEMO_LOGIC_ERROR, "applyStdp called, but no STDP model specified");
 	}
-	waitStream(m_stream);
-	/* the event counters before and after the run's work, copied on its
-	 * stream (no blocking copy at either end) */
-	/* The counters are copied even when the caller does not ask for the
-	 * events: a run whose graph was the first work queued on the stream
-	 * after the synchronisation above started it about 5 ms late on the
-	 * MI355X in every 20-step run measured (with the copy queued first: 22-23
-	 * us per step; without: 250 us). */
-	const size_t nCounters = m_blockEvents.n;
-	HIP_CHECK(hipMemcpyAsync(m_pinnedCounters, m_blockEvents.ptr, m_blockEvents.bytes(), hipMemcpyDeviceToHost,
-				m_stream));
+	/* The event total before and after the run's work, by a kernel on its
+	 * stream.  The first is summed even when the caller does not ask for the
+	 * events: a run whose graph was the first work queued on an idle stream
+	 * started it about 5 ms late on the MI355X in every 20-step run measured. */
+	const nemo_host_signal none = {nullptr, 0, nullptr};
+	HIP_CHECK(nemo_launch_sum_counters(m_stream, m_blockEvents.ptr, m_blockEvents.n, m_pinnedEvents, &none));
 	/* a run begins with no STDP batch pending when the last thing before it
 	 * was a run (which ends with its flush) */
 	bool batchPending = m_stdpBlocks && m_hostStep > 0 && m_flushed != m_hostStep - 1;
@@ -2295,97 +2249,56 @@ void Simulation::run(unsigned nsteps, unsigned stdpPeriod, float reward, bool re
 		if(fired->cap == 0) fired->spill->reserve(fired->spill->size() + size_t(1.25 * m_firedPerStep * nsteps) + 1024);
 		counts->reserve(counts->size() + size_t(nsteps) * m_nets);
 	}
-	/* Chunks alternate between the two halves of the readout buffers (pinned
-	 * bitmaps, or device and pinned lists): chunk i+1 is queued before chunk
-	 * i's firing is decoded on the host, so the device does not wait for the
-	 * host between chunks.  The copy of chunk i runs on its own stream beside
-	 * chunk i+1; the device ring holds 128 steps, so chunk i's bitmaps (and
-	 * its half's device list) are intact until chunk i+2, which waits for
-	 * that copy (the copy of chunk i is the last use of its half's event
-	 * before chunk i+2 records it again). */
-	hipEvent_t* copied = m_readoutCopied;
-	hipEvent_t* ready = m_readoutReady;
-	bool inFlight[2] = {false, false};
-	unsigned pendingSteps = 0; /* steps of the chunk waiting to be decoded */
-	int pendingHalf = -1;
-	const bool devList = readRaster && ensureListReadout();
-	size_t listCopied[2] = {0, 0}; /* entries of each half's list copied with its counts */
-	auto decodePending = [&]() {
-		if(pendingHalf < 0) return;
-		waitEvent(copied[pendingHalf]);
-		if(devList) {
-			const int h = pendingHalf;
-			const uint32_t* cnt = m_pinnedListCounts + size_t(h) * CHUNK;
-			size_t total = 0;
-			for(unsigned s = 0; s < pendingSteps; ++s) {
-				counts->push_back(cnt[s]);
-				total += cnt[s];
+	/* Chunk i's firing is taken after chunk i+1 is queued, so that the device
+	 * does not wait for the host, and before chunk i+2 is, which writes the
+	 * same ring slots. */
+	uint64_t takeFrom = m_hostStep; /* first step whose firing is not taken */
+	auto take = [&](uint64_t upto) {
+		if(!readRaster || takeFrom == upto) return;
+		waitFlag(m_pinnedStepFlag, upto);
+		for(; takeFrom < upto; ++takeFrom) {
+			const size_t slot = takeFrom & (NEMO_STEP_RING - 1);
+			const size_t n = m_pinnedCounts[slot];
+			const uint32_t* list = m_pinnedLists + slot * m_readoutRoom;
+			if(n <= m_readoutRoom && m_nets == 1) {
+				counts->push_back(unsigned(n));
+				fired->append(list, n);
+				continue;
 			}
-			if(total > listCopied[h]) {
-				/* the rest, on a stream of its own: the copy stream may
-				 * already wait for the next chunk */
-				growPinnedList(h, total, listCopied[h]);
-				HIP_CHECK(hipMemcpyAsync(m_pinnedList[h] + listCopied[h],
-							m_listDev.ptr + size_t(h) * CHUNK * m_npad + listCopied[h],
-							(total - listCopied[h]) * sizeof(uint32_t), hipMemcpyDeviceToHost, m_restStream));
+			std::vector<uint32_t> all;
+			if(n > m_readoutRoom) {
+				/* the bitmap, beside the next chunk */
+				readBitmaps(takeFrom, 1, m_pinnedBits + slot * m_firedWords, m_restStream);
 				waitStream(m_restStream);
+				const uint64_t* bits = m_pinnedBits + slot * m_firedWords;
+				if(m_nets == 1) {
+					counts->push_back(unsigned(n));
+					decodeFiring(bits, *fired);
+					continue;
+				}
+				all.reserve(n);
+				for(size_t w = 0; w < m_firedWords; ++w) {
+					for(uint64_t x = bits[w]; x; x &= x - 1) all.push_back(uint32_t(w * 64 + lowestBit(x)));
+				}
+				list = all.data();
 			}
-			fired->append(m_pinnedList[h], total);
-		} else {
-			const uint64_t* bits = m_pinnedBits + size_t(pendingHalf) * CHUNK * m_firedWords;
-			for(unsigned s = 0; s < pendingSteps; ++s) {
-				decodeFiringBatch(bits + size_t(s) * m_firedWords, *fired, *counts);
-			}
+			decodeListBatch(list, n, *fired, *counts);
 		}
-		pendingHalf = -1;
 	};
 	try {
 		unsigned done = 0;
-		int half = 0;
 		while(done < nsteps) {
 			unsigned k = std::min(CHUNK, nsteps - done);
 			if(stdpPeriod) k = unsigned(std::min<uint64_t>(k, stdpPeriod - stepsSinceApply));
 			const uint64_t t0 = m_hostStep;
-			hipGraphExec_t g = graphFor(k, batchPending);
+			hipGraphExec_t g = graphFor(k, batchPending, readRaster);
 			batchPending = true; /* each chunk leaves its steps pending */
 			ensureRing();
 			if(m_base != t0) setBase(t0);
-			/* the ring slots this chunk overwrites were copied out */
-			if(inFlight[half]) HIP_CHECK(hipStreamWaitEvent(m_stream, copied[half], 0));
 			HIP_CHECK(hipGraphLaunch(g, m_stream));
 			m_base = t0 + k;
 			advanceSteps(k);
-			if(readRaster) {
-				uint32_t* listDev = devList ? m_listDev.ptr + size_t(half) * CHUNK * m_npad : nullptr;
-				uint32_t* countsDev = devList ? m_listCountsDev.ptr + size_t(half) * CHUNK : nullptr;
-				HIP_CHECK(hipEventRecord(ready[half], m_stream));
-				HIP_CHECK(hipStreamWaitEvent(m_copyStream, ready[half], 0));
-				if(devList) {
-					/* compacted on the copy stream too, beside the next chunk (or
-					 * the run's closing STDP batch) */
-					HIP_CHECK(nemo_launch_fired_list(m_copyStream, m_firedBits.ptr, m_firedWords, t0, k,
-								m_l2gDev.ptr, countsDev, listDev));
-					/* the counts and as much of the list as recent rates suggest,
-					 * at least 1/64 of the neurons per step (half the bytes of
-					 * the bitmaps) */
-					const size_t expect = std::max(size_t(1.5 * m_firedPerStep * k), size_t(k) * m_npad / 64) + 4096;
-					listCopied[half] = std::min({expect, m_pinnedListCap[half], size_t(k) * m_npad});
-					HIP_CHECK(hipMemcpyAsync(m_pinnedListCounts + size_t(half) * CHUNK, countsDev, k * sizeof(uint32_t),
-								hipMemcpyDeviceToHost, m_copyStream));
-					HIP_CHECK(hipMemcpyAsync(m_pinnedList[half], listDev, listCopied[half] * sizeof(uint32_t),
-								hipMemcpyDeviceToHost, m_copyStream));
-				} else {
-					readBitmaps(t0, k, m_pinnedBits + size_t(half) * CHUNK * m_firedWords, m_copyStream);
-				}
-				HIP_CHECK(hipEventRecord(copied[half], m_copyStream));
-				inFlight[half] = true;
-			}
-			decodePending();
-			if(readRaster) {
-				pendingHalf = half;
-				pendingSteps = k;
-				half ^= 1;
-			}
+			take(t0);
 			done += k;
 			stepsSinceApply += k;
 			if(stdpPeriod && stepsSinceApply == stdpPeriod) {
@@ -2396,27 +2309,17 @@ void Simulation::run(unsigned nsteps, unsigned stdpPeriod, float reward, bool re
 		/* a run returns with the STDP accumulation of all its steps done
 		 * (the last batch, or the last step's in the per-step placements) */
 		enqueueFlush();
-		if(events) {
-			HIP_CHECK(hipMemcpyAsync(m_pinnedCounters + nCounters, m_blockEvents.ptr, m_blockEvents.bytes(),
-						hipMemcpyDeviceToHost, m_stream));
-		}
-		decodePending();
+		const nemo_host_signal end = nextSignal();
+		HIP_CHECK(nemo_launch_sum_counters(m_stream, m_blockEvents.ptr, m_blockEvents.n, m_pinnedEvents + 1, &end));
+		take(m_hostStep);
+		waitSignal(end);
 	} catch(...) {
 		(void) hipStreamSynchronize(m_stream);
-		(void) hipStreamSynchronize(m_copyStream);
+		(void) hipStreamSynchronize(m_restStream);
 		throw;
 	}
-	waitStream(m_copyStream);
-	waitStream(m_stream);
 	if(readRaster && fired && nsteps) m_firedPerStep = double(fired->size() - firedBefore) / nsteps;
-	if(events) {
-		uint64_t before = 0, after = 0;
-		for(size_t i = 0; i < nCounters; ++i) {
-			before += m_pinnedCounters[i];
-			after += m_pinnedCounters[nCounters + i];
-		}
-		*events = after - before;
-	}
+	if(events) *events = m_pinnedEvents[1] - m_pinnedEvents[0];
 	m_firedOut.clear();
 	checkStatus();
 }
@@ -2485,8 +2388,10 @@ void Simulation::prepare(unsigned nsteps, unsigned stdpPeriod)
 	while(done < nsteps) {
 		unsigned k = std::min(64u, nsteps - done);
 		if(stdpPeriod) k = unsigned(std::min<uint64_t>(k, stdpPeriod - since));
-		graphFor(k, true);
-		if(done == 0) graphFor(k, false); /* a run's first chunk with nothing pending */
+		for(bool readout : {true, false}) {
+			graphFor(k, true, readout);
+			if(done == 0) graphFor(k, false, readout); /* a run's first chunk with nothing pending */
+		}
 		done += k;
 		since += k;
 		if(stdpPeriod && since == stdpPeriod) since = 0;
@@ -2555,6 +2460,7 @@ void Simulation::restoreSnapshot(const Snapshot& s)
 	m_lastCycle = s.lastCycle;
 	m_updated = s.updated;
 	m_ringStale = true;
+	*m_pinnedStepFlag = 0; /* the steps to come may be ones it has counted */
 }
 
 /* Advance nsteps steps in graphs of up to 64 steps, then their pending STDP
@@ -2569,7 +2475,7 @@ double Simulation::timeSteps(unsigned nsteps)
 	unsigned done = 0;
 	while(done < nsteps) {
 		const unsigned k = std::min(64u, nsteps - done);
-		hipGraphExec_t g = graphFor(k, true);
+		hipGraphExec_t g = graphFor(k, true, false);
 		ensureRing();
 		if(m_base != m_hostStep) setBase(m_hostStep);
 		HIP_CHECK(hipGraphLaunch(g, m_stream));
@@ -2732,7 +2638,7 @@ void Simulation::applyStdp(float reward)
 		msg << "STDP reward rounded down to zero. The smallest valid reward is " << fxToFloat(1, m_fbits);
 		throw Error(NEMO_INVALID_INPUT, msg.str());
 	}
-	flushStdp();
+	enqueueFlush();
 	nemo_apply_args a;
 	a.rcm_of = m_rcmOf.ptr;
 	a.fcm_count = m_fcm.n;

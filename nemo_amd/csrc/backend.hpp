@@ -290,8 +290,8 @@ private:
 	hipEvent_t m_stdpFork = nullptr, m_stdpDone = nullptr;
 	hipEvent_t m_stdpLag[2] = {nullptr, nullptr}; /* mode 3: branch of step parity i done */
 	hipStream_t m_earlyStream = nullptr; /* branch for the delays 2..D of the next step */
-	hipStream_t m_copyStream = nullptr;  /* firing-bitmap readout of run(), beside the next steps */
-	hipStream_t m_restStream = nullptr;  /* the rest of a fired list longer than expected */
+	hipEvent_t m_waitEvent = nullptr;    /* waitStream's */
+	hipStream_t m_restStream = nullptr;  /* bitmaps of steps that fired more than the readout has room for */
 	/* with several neuron models, every model's update after the first runs
 	 * on a branch of its own, so a step waits for the slowest model */
 	std::vector<hipStream_t> m_groupStreams;
@@ -303,10 +303,6 @@ private:
 	bool m_decodeInOrder = false;         /* batch whose device order lists each network in turn, in order */
 	bool m_binRanged = false;             /* updates read only their tiles' column ranges */
 	hipEvent_t m_earlyFork = nullptr, m_earlyDone[2] = {nullptr, nullptr};
-	/* run(): a chunk's steps are done (ready) and its firing is copied out
-	 * (copied), per half of the readout buffers; created once, as creating
-	 * them per run delays a short run's first work */
-	hipEvent_t m_readoutReady[2] = {nullptr, nullptr}, m_readoutCopied[2] = {nullptr, nullptr};
 	bool m_stdpPending = false;          /* the STDP branch has not been joined yet */
 	unsigned m_nets = 1;   /* networks in the batch */
 	size_t m_ncount = 0;   /* neurons */
@@ -426,20 +422,18 @@ private:
 	DeviceArray<unsigned> m_signalBlocks;
 	nemo_host_signal nextSignal();
 	void waitSignal(const nemo_host_signal& done);
-	/* run()'s firing readout of a single network, compacted on the device:
-	 * per half (chunks alternate), the steps' counts and fired lists */
-	DeviceArray<uint32_t> m_l2gDev;       /* m_l2g on the device */
-	DeviceArray<uint32_t> m_listDev;      /* [2][CHUNK * m_npad] fired lists */
-	DeviceArray<uint32_t> m_listCountsDev; /* [2][CHUNK] */
-	uint32_t* m_pinnedListCounts = nullptr; /* [2][CHUNK] */
-	uint32_t* m_pinnedList[2] = {nullptr, nullptr};
-	size_t m_pinnedListCap[2] = {0, 0};
-	bool ensureListReadout();
-	void waitEvent(hipEvent_t);
+	/* run()'s firing readout, compacted by the last kernel of a graph of steps
+	 * into pinned memory: per ring slot of a step, the count of fired neurons
+	 * and the first m_readoutRoom of them; then the flag, the steps done */
+	DeviceArray<uint32_t> m_l2gDev;       /* m_l2g on the device (single networks) */
+	uint32_t* m_pinnedCounts = nullptr;   /* [NEMO_STEP_RING] */
+	uint32_t* m_pinnedLists = nullptr;    /* [NEMO_STEP_RING][m_readoutRoom] */
+	uint64_t* m_pinnedStepFlag = nullptr; /* steps whose firing is there */
+	unsigned m_readoutRoom = 0;
+	void ensureReadout();
+	void waitFlag(const uint64_t* flag, uint64_t value);
 	void waitStream(hipStream_t);
-	void growPinnedList(int half, size_t need, size_t keep);
-	unsigned long long* m_pinnedCounters = nullptr; /* [2][m_blockEvents.n]: the event counters at the
-	                                                   start and at the end of a run */
+	uint64_t* m_pinnedEvents = nullptr;   /* the event total at the start and at the end of a run */
 	std::vector<unsigned> m_firedOut;
 	std::chrono::steady_clock::time_point m_wallStart;
 
@@ -467,18 +461,19 @@ private:
 	void copyScalar(uint64_t* dst, uint64_t value);
 	void setBase(uint64_t base);
 	void enqueueSteps(uint64_t first, unsigned k, bool ext, bool fstim, hipEvent_t* ev = nullptr,
-			bool forkPending = true, bool advanceBase = false);
+			bool forkPending = true, bool advanceBase = false, bool readout = false);
 	void launchDelivery(const nemo_propagate_args& set, uint64_t offset, hipStream_t st, bool withStdp,
 			hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 	void flushStdp();
 	bool enqueueFlush();
 	void joinStdp();
 	template<typename Out> void decodeFiring(const uint64_t* bits, Out& out) const;
-	template<typename Out> void decodeFiringBatch(const uint64_t* bits, Out& out, std::vector<unsigned>& counts) const;
+	template<typename Out> void decodeListBatch(const uint32_t* fired, size_t n, Out& out, std::vector<unsigned>& counts) const;
 	void readBitmaps(uint64_t t0, unsigned k, uint64_t* dst = nullptr, hipStream_t st = nullptr);
 	uint64_t sumCounters(const DeviceArray<unsigned long long>& a);
-	/* the graph of k steps (forkPending: it runs the pending STDP batch first) */
-	hipGraphExec_t graphFor(unsigned k, bool forkPending = true);
+	/* the graph of k steps (forkPending: it runs the pending STDP batch first;
+	 * readout: it reads the steps' firing out) */
+	hipGraphExec_t graphFor(unsigned k, bool forkPending, bool readout);
 	void clearGraphs();
 	struct Snapshot;
 	void takeSnapshot(Snapshot& s);

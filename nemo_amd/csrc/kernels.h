@@ -127,12 +127,18 @@ hipError_t nemo_launch_direct_rebuild(hipStream_t, const nemo_hip_direct* r, siz
 hipError_t nemo_launch_gather_currents(hipStream_t, const nemo_hip_step_buffers* b, const uint32_t* dev_to_sim,
 		float* E, float* I, unsigned tiles, const nemo_host_signal* done);
 
-/* Firing readout of k steps from step t0 (their firing-bitmap ring slots,
- * words words each): counts[s] the neurons fired in step t0 + s, and list
- * their l2g entries, step after step, each step in ascending device index
- * (list holds up to k * words * 64 entries). */
-hipError_t nemo_launch_fired_list(hipStream_t, const uint64_t* bits, size_t words, uint64_t t0, unsigned k,
-		const uint32_t* l2g, uint32_t* counts, uint32_t* list);
+/* Firing readout of the k steps from clock base + offset on (their
+ * firing-bitmap ring slots, words words each) into pinned host memory: for
+ * step t, slot t % NEMO_STEP_RING, counts[slot] the neurons fired and
+ * list[slot * room ..] the first room of them in ascending device index, as
+ * index's entries (NULL: device indices).  Then the flag is set to done.value
+ * + base + offset. */
+hipError_t nemo_launch_fired_readout(hipStream_t, const nemo_hip_clock* clock, uint64_t offset, unsigned k,
+		const uint64_t* bits, size_t words, const uint32_t* index, uint32_t* counts, uint32_t* list, unsigned room,
+		const nemo_host_signal* done);
+/* *sum = the total of the n counters (sum in pinned host memory) */
+hipError_t nemo_launch_sum_counters(hipStream_t, const unsigned long long* counters, size_t n, uint64_t* sum,
+		const nemo_host_signal* done);
 
 /* The stimulus of a step: bits set for the nf device indices fidx, ext[iidx[i]]
  * = ival[i] (distinct indices); the lists may be pinned host memory. */

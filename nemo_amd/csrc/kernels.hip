@@ -187,53 +187,6 @@ invert_rcm_kernel(const uint32_t* rcm_fwd, uint32_t* rcm_of, size_t count)
 	}
 }
 
-/* ------------------------------------------------------ firing readout */
-
-/* Neurons fired in step t0 + blockIdx.x (its firing-bitmap ring slot) */
-__global__ void __launch_bounds__(NEMO_BLOCK)
-fired_count_kernel(const uint64_t* bits, size_t words, uint64_t t0, uint32_t* counts)
-{
-	const uint64_t* b = bits + ((t0 + blockIdx.x) & (NEMO_STEP_RING - 1)) * words;
-	uint32_t c = 0;
-	for(size_t w = threadIdx.x; w < words; w += NEMO_BLOCK) c += uint32_t(__popcll(b[w]));
-	uint32_t total;
-	nemo_dev::block_exclusive_scan<NEMO_BLOCK>(c, &total);
-	if(threadIdx.x == 0) counts[blockIdx.x] = total;
-}
-
-/* The neurons fired in step t0 + blockIdx.x, in ascending device index, as
- * l2g's indices, written after those of the steps before it (counts) */
-__global__ void __launch_bounds__(NEMO_BLOCK)
-fired_list_kernel(const uint64_t* bits, size_t words, uint64_t t0, const uint32_t* counts, const uint32_t* l2g,
-		uint32_t* list)
-{
-	__shared__ uint32_t s_off;
-	if(threadIdx.x < 64) {
-		uint32_t v = 0;
-		for(unsigned s = threadIdx.x; s < blockIdx.x; s += 64) v += counts[s];
-#pragma unroll
-		for(int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-		if(threadIdx.x == 0) s_off = v;
-	}
-	__syncthreads();
-	const uint64_t* b = bits + ((t0 + blockIdx.x) & (NEMO_STEP_RING - 1)) * words;
-	/* a contiguous run of words per thread keeps the list in device order */
-	const size_t per = (words + NEMO_BLOCK - 1) / NEMO_BLOCK;
-	const size_t w0 = min(words, size_t(threadIdx.x) * per), w1 = min(words, w0 + per);
-	uint32_t c = 0;
-	for(size_t w = w0; w < w1; ++w) c += uint32_t(__popcll(b[w]));
-	uint32_t total;
-	uint32_t pos = s_off + nemo_dev::block_exclusive_scan<NEMO_BLOCK>(c, &total);
-	for(size_t w = w0; w < w1; ++w) {
-		uint64_t x = b[w];
-		while(x) {
-			const unsigned bit = unsigned(__builtin_ctzll(x));
-			x &= x - 1;
-			list[pos++] = l2g[w * 64 + bit];
-		}
-	}
-}
-
 /* Tells the host, which polls done->flag in pinned memory, that the kernel's
  * writes to pinned memory are there: by the last of its blocks to get here,
  * every thread of which calls it (done->blocks counts them, and ends at 0). */
@@ -248,6 +201,67 @@ __device__ inline void signal_done(const nemo_host_signal& done)
 		__threadfence_system();
 	}
 	__hip_atomic_store(done.flag, done.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+/* ------------------------------------------------------ firing readout */
+
+constexpr unsigned READOUT_BLOCK = 512;
+/* entries of a step's list that its block puts in order in LDS */
+constexpr unsigned READOUT_STAGE = 4096;
+
+/* The neurons fired in step base + offset + blockIdx.x (its firing-bitmap ring
+ * slot), in ascending device index: counts[slot] of them, list[slot][..] the
+ * first room of them, as index's entries (or, index NULL, device indices).
+ * counts and list are pinned host memory, so that the host reads them without
+ * a copy: per 64 steps, two copies and the events between the streams took 65
+ * us.  The list goes out through LDS, in whole lines. */
+__global__ void __launch_bounds__(READOUT_BLOCK)
+fired_readout_kernel(const nemo_hip_clock* clock, uint64_t offset, const uint64_t* bits, size_t words,
+		const uint32_t* index, uint32_t* counts, uint32_t* list, unsigned room, nemo_host_signal done)
+{
+	__shared__ uint32_t s_list[READOUT_STAGE];
+	const uint64_t base = nemo_dev::clock_base(clock) + offset;
+	const size_t slot = (base + blockIdx.x) & (NEMO_STEP_RING - 1);
+	const uint64_t* b = bits + slot * words;
+	uint32_t* out = list + slot * room;
+	/* a contiguous run of words per thread keeps the list in device order */
+	const size_t per = (words + READOUT_BLOCK - 1) / READOUT_BLOCK;
+	const size_t w0 = min(words, size_t(threadIdx.x) * per), w1 = min(words, w0 + per);
+	uint32_t c = 0;
+	for(size_t w = w0; w < w1; ++w) c += uint32_t(__popcll(b[w]));
+	uint32_t total;
+	uint32_t pos = nemo_dev::block_exclusive_scan<READOUT_BLOCK>(c, &total);
+	if(threadIdx.x == 0) counts[slot] = total;
+	const bool staged = total <= READOUT_STAGE;
+	for(size_t w = w0; w < w1; ++w) {
+		for(uint64_t x = b[w]; x; x &= x - 1, ++pos) {
+			const uint32_t n = uint32_t(w * 64) + uint32_t(__builtin_ctzll(x));
+			const uint32_t v = index ? index[n] : n;
+			if(staged) s_list[pos] = v;
+			else if(pos < room) out[pos] = v;
+		}
+	}
+	if(staged) {
+		__syncthreads();
+		for(uint32_t i = threadIdx.x; i < min(total, room); i += READOUT_BLOCK) out[i] = s_list[i];
+	}
+	done.value += base;
+	signal_done(done);
+}
+
+/* *sum = the total of the n counters (sum in pinned host memory).  One block. */
+__global__ void __launch_bounds__(READOUT_BLOCK)
+sum_counters_kernel(const unsigned long long* counters, size_t n, uint64_t* sum, nemo_host_signal done)
+{
+	__shared__ unsigned long long s_sum;
+	if(threadIdx.x == 0) s_sum = 0;
+	__syncthreads();
+	unsigned long long x = 0;
+	for(size_t i = threadIdx.x; i < n; i += READOUT_BLOCK) x += counters[i];
+	if(x) atomicAdd(&s_sum, x);
+	__syncthreads();
+	if(threadIdx.x == 0) *sum = s_sum;
+	if(done.flag) signal_done(done);
 }
 
 /* ------------------------------------------- externally given firing */
@@ -587,15 +601,20 @@ hipError_t nemo_launch_gather_currents(hipStream_t st, const nemo_hip_step_buffe
 	return hipGetLastError();
 }
 
-hipError_t nemo_launch_fired_list(hipStream_t st, const uint64_t* bits, size_t words, uint64_t t0, unsigned k,
-		const uint32_t* l2g, uint32_t* counts, uint32_t* list)
+hipError_t nemo_launch_fired_readout(hipStream_t st, const nemo_hip_clock* clock, uint64_t offset, unsigned k,
+		const uint64_t* bits, size_t words, const uint32_t* index, uint32_t* counts, uint32_t* list, unsigned room,
+		const nemo_host_signal* done)
 {
-	if(k == 0) return hipSuccess;
-	if(k > NEMO_STEP_RING || !bits || !l2g || !counts || !list) return hipErrorInvalidValue;
-	hipLaunchKernelGGL(fired_count_kernel, dim3(k), dim3(NEMO_BLOCK), 0, st, bits, words, t0, counts);
-	const hipError_t e = hipGetLastError();
-	if(e != hipSuccess) return e;
-	hipLaunchKernelGGL(fired_list_kernel, dim3(k), dim3(NEMO_BLOCK), 0, st, bits, words, t0, counts, l2g, list);
+	if(k == 0 || k > NEMO_STEP_RING || !clock || !bits || !counts || !list || !done->flag) return hipErrorInvalidValue;
+	hipLaunchKernelGGL(fired_readout_kernel, dim3(k), dim3(READOUT_BLOCK), 0, st, clock, offset, bits, words, index, counts,
+			list, room, *done);
+	return hipGetLastError();
+}
+
+hipError_t nemo_launch_sum_counters(hipStream_t st, const unsigned long long* counters, size_t n, uint64_t* sum,
+		const nemo_host_signal* done)
+{
+	hipLaunchKernelGGL(sum_counters_kernel, dim3(1), dim3(READOUT_BLOCK), 0, st, counters, n, sum, *done);
 	return hipGetLastError();
 }
 

@@ -143,3 +143,40 @@ def test_maximum_delay_and_propagate_with_steps_in_between():
         counts, fired, _ = hip.run(130)
         assert counts.tolist() == [len(f) for f in want]
         assert fired.tolist() == [i for f in want for i in f]
+
+
+# ------------------------------------------------------- firing readout
+def sources_and_neurons(n, first, seed, order):
+    """n Poisson sources firing with rate 1 per ms (every step) or, past
+    4090, now and then, and 300 Izhikevich neurons, in either type order."""
+    rate = np.where(np.arange(n) < 4090, np.float32(1.0), np.float32(0.01)).astype(np.float32)
+    po = gen.NetworkSpec(blocks=[gen.NeuronBlock("PoissonSource", np.arange(first, first + n, dtype=np.uint32), [rate])])
+    iz = gen.random_izhikevich(300, 40, dmax=8, seed=seed, first_index=first + n)
+    return gen.merge(*((po, iz) if order else (iz, po)))
+
+
+@pytest.mark.parametrize("sizes", [(4000,), (4095,), (4200,), (9000,), (2500, 4090, 3000)])
+def test_readout_of_steps_around_its_room(sizes):
+    """Steps that fire fewer and more neurons than the readout has room for,
+    over several graphs, against the oracle: a single network and a batch
+    whose networks list their types in different orders."""
+    specs = [sources_and_neurons(n, 7, 30 + k, k % 2) for k, n in enumerate(sizes)]
+    refs, nets = [], []
+    for spec in specs:
+        for api, out in ((oa, refs), (nemo_amd, nets)):
+            net = api.Network()
+            spec.load(net)
+            out.append(oa.Simulation(net, oa.Configuration()) if api is oa else net)
+    steps = 131
+    conf = nemo_amd.Configuration()
+    if len(nets) == 1:
+        counts, fired, _ = nemo_amd.Simulation(nets[0], conf).run(steps)
+        got = [(counts, fired)]
+    else:
+        batch = nemo_amd.Batch(nets, conf)
+        counts, fired, _ = batch.run(steps)
+        got = batch.split(counts, fired)
+    for ref, (c, f) in zip(refs, got):
+        want = [ref.step() for _ in range(steps)]
+        assert c.tolist() == [len(x) for x in want]
+        assert f.tolist() == [i for x in want for i in x]
