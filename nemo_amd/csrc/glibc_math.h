@@ -281,6 +281,62 @@ NEMO_HD float expf_exact(float x)
 	return expf_exact_tab(x, T);
 }
 
+/* expf for -104 <= x <= 89, without the special cases: there the double's
+ * own rounding gives the underflow to 0 and the overflow to infinity.  The
+ * polynomial is summed by Horner's rule, one operation less than the
+ * published order, and the double differs from that order's in the last
+ * place; the float is the same for every float x of the range (the tests try
+ * them all).  tab repeats the 32 entries EXPF_REPEATS times, so that the
+ * index is the low byte of the rounded argument. */
+constexpr unsigned EXPF_REPEATS = 8;
+
+/* the part up to the table entry, which a caller may load ahead of the rest */
+struct ExpfParts {
+	double xd, kd;
+	uint32_t ki;
+	uint64_t t;
+};
+
+NEMO_HD ExpfParts expf_main_begin(float x, const uint64_t* tab)
+{
+	const double InvLn2N = 0x1.71547652b82fep+0 * 32;
+	const double SHIFT = 0x1.8p+52;
+	ExpfParts p;
+	p.xd = double(x);
+	p.kd = fma_d(InvLn2N, p.xd, SHIFT);
+	p.ki = uint32_t(asuint64(p.kd));
+	p.t = tab[p.ki & 0xff];
+	return p;
+}
+
+/* the polynomial, which does not need the table entry */
+NEMO_HD double expf_main_poly(const ExpfParts& p)
+{
+	const double InvLn2N = 0x1.71547652b82fep+0 * 32;
+	const double SHIFT = 0x1.8p+52;
+	const double C0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32;
+	const double C1 = 0x1.ebfce50fac4f3p-3 / 32 / 32;
+	const double C2 = 0x1.62e42ff0c52d6p-1 / 32;
+	const double r = fma_d(InvLn2N, p.xd, -(p.kd - SHIFT));
+	return fma_d(fma_d(fma_d(C0, r, C1), r, C2), r, 1.0);
+}
+
+NEMO_HD float expf_main_end(const ExpfParts& p, double y)
+{
+	/* ki << 47 reaches the high word alone */
+	uint32_t high = uint32_t(p.t >> 32) + (p.ki << 15);
+#ifdef __HIP_DEVICE_COMPILE__
+	asm("" : "+v"(high)); /* one 32-bit operation, not a 64-bit sum */
+#endif
+	return float(y * asdouble((uint64_t(high) << 32) | uint32_t(p.t)));
+}
+
+NEMO_HD float expf_main_tab(float x, const uint64_t* tab)
+{
+	const ExpfParts p = expf_main_begin(x, tab);
+	return expf_main_end(p, expf_main_poly(p));
+}
+
 /* ---------------------------------------------------------------- fmodf */
 
 /* x - n y for the integer n = trunc(x / y), which IEEE 754 defines exactly

@@ -180,3 +180,41 @@ def test_readout_of_steps_around_its_room(sizes):
         want = [ref.step() for _ in range(steps)]
         assert c.tolist() == [len(x) for x in want]
         assert f.tolist() == [i for x in want for i in x]
+
+
+# ------------------------------------------------- Hodgkin-Huxley substeps
+def hh_cells(api, v, gates, dirs):
+    net = api.Network()
+    t = net.add_neuron_type("HH")
+    n = len(v)
+    net.add_neuron(t, np.arange(n, dtype=np.uint32), np.asarray(v, np.float32), *[np.asarray(g, np.float32) for g in gates],
+                   np.asarray(dirs, np.float32))
+    return api.Simulation(net, api.Configuration())
+
+
+# y = v + 65: the quotients of alphan and alpham are by 0 at y = 10 and 25;
+# the substeps without special cases are for |y| <= 256
+HH_POTENTIALS = [-65.0, -55.0, -40.0, -45.0, -45.000004, -44.999996, 50.0, 191.0, 191.00002, -321.0, -321.00003, 2000.0,
+                 -3000.0, 1e6, -1e6, 1e30, -1e38, 3e38, np.inf, -np.inf, np.nan, -54.999996, -55.000004, -39.999996]
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 24, 257])
+def test_hh_substeps_match_oracle(n):
+    """State and firing equal the oracle's, step by step, with neighbours in a
+    wave that take the general path and ones that do not, and with currents
+    that turn the potential down from both sides of -45."""
+    rng = np.random.default_rng(n)
+    v = np.resize(np.asarray(HH_POTENTIALS, np.float32), n)
+    if n == 257:
+        v[24:] = (rng.random(n - 24, dtype=np.float32) * 120 - 80).astype(np.float32)
+    gates = [rng.random(n, dtype=np.float32) for _ in range(3)]
+    dirs = rng.choice(np.asarray([0.0, -1e-10, 1e-3, -0.5], np.float32), n)
+    sims = [hh_cells(api, v, gates, dirs) for api in (oa, nemo_amd)]
+    for t in range(30):
+        istim = [(i, float(x)) for i, x in enumerate(rng.normal(0, 40, n).astype(np.float32))]
+        fr, fh = (s.step(istim=istim) for s in sims)
+        assert list(fr) == list(fh), t
+        for k in range(5):
+            a, b = (np.asarray(s.neuron_states(k), np.float32) for s in sims)
+            same = (a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))
+            assert same.all(), (t, k, np.flatnonzero(~same)[:5])
