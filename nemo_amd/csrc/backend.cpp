@@ -50,6 +50,8 @@ void DeviceArray<T>::release()
 
 template struct DeviceArray<float>;
 template struct DeviceArray<double>;
+template struct DeviceArray<uint16_t>;
+template struct DeviceArray<nemo_float_row>;
 template struct DeviceArray<uint32_t>;
 template struct DeviceArray<int32_t>;
 template struct DeviceArray<int64_t>;

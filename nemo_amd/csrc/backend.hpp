@@ -13,6 +13,7 @@
 #ifndef NEMO_AMD_BACKEND_HPP
 #define NEMO_AMD_BACKEND_HPP
 
+#include "float_mode.h"
 #include <chrono>
 #include <map>
 #include <memory>
@@ -501,13 +502,14 @@ public:
 			float* S, float* V, double* ckpt);
 	/* The device memory the forward uses beyond its arguments */
 	struct ForwardWorkspace {
+		bool sliced;      /* wr in the slices' order */
 		float* wr;        /* weights in reverse order */
 		double* v;        /* state */
 		double* u;
 		uint32_t* bits;   /* [T][pitch] spike bitmaps */
 	};
-	size_t forwardWorkspaceBytes(unsigned T) const;
-	ForwardWorkspace carveWorkspace(void* base, unsigned T) const;
+	size_t forwardWorkspaceBytes(unsigned T, bool sliced) const;
+	ForwardWorkspace carveWorkspace(void* base, unsigned T, bool sliced) const;
 	void forwardWith(const ForwardWorkspace& ws, hipStream_t st, unsigned T, unsigned K, const float* w,
 			const float* a, const float* b, const float* c, const float* d, const float* v0, const float* u0,
 			const float* x, float* S, float* V, double* ckpt);
@@ -526,8 +528,16 @@ private:
 	int m_device = 0;
 	size_t m_n = 0, m_s = 0;
 	unsigned m_D = 1;
-	DeviceArray<uint32_t> m_fcmPtr, m_fcmTd;          /* network order is forward order */
+	DeviceArray<uint32_t> m_fcmPtr, m_fcmTd;          /* network order is forward order (not with m_push) */
+	bool m_push = false;                              /* backward steps stage the input adjoints in LDS */
+	unsigned m_tile = 0, m_pushPitch = 0, m_pushLanes = 1, m_slices = 0;
+	DeviceArray<uint32_t> m_rowSlices, m_rowUser;     /* their synapses by (source, delay) */
+	DeviceArray<nemo_float_row> m_rows;
+	DeviceArray<uint16_t> m_rowTarget;
+	DeviceArray<float> m_rowW, m_rowGw;
 	DeviceArray<uint32_t> m_rcmPtr, m_rcmSd, m_rcmUser;
+	DeviceArray<uint32_t> m_slicePtr, m_sliceSd, m_sliceUser; /* the same in slices of eight targets */
+	unsigned m_sliceLines = 0;                        /* of the longest */
 	DeviceArray<float> m_wr;
 	DeviceArray<double> m_v, m_u, m_seg;  /* state in double; segment: entry v, u and input I */
 	DeviceArray<double> m_LV, m_LU, m_LI; /* adjoint state and recent input adjoints */
@@ -538,6 +548,14 @@ private:
 	bool m_stage = false;
 
 	void prepare(unsigned T, unsigned K);
+
+	struct PushRows {
+		std::vector<uint32_t> ptr, at;
+		std::vector<nemo_float_row> rows;
+	};
+	PushRows pushRows(const std::vector<uint32_t>& rowLen);
+	std::vector<uint32_t> pullSlices(const std::vector<uint32_t>& ptr);
+	void sliceWeights(hipStream_t st, float* wr, const float* w);
 };
 
 } // namespace nemo_hip

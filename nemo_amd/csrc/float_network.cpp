@@ -42,6 +42,17 @@ FloatNetwork::FloatNetwork(const Network& net, int device) : m_device(device < 0
 	if(m_s >= (size_t(1) << 32)) throw Error(NEMO_API_UNSUPPORTED, "too many synapses for the float-weight mode");
 	m_D = std::max(1u, net.maxDelay);
 
+	/* NEMO_HIP_FLOAT_STAGE=0 stages nothing in LDS */
+	const char* env = std::getenv("NEMO_HIP_FLOAT_STAGE");
+	const bool mayStage = !env || std::string(env) != "0";
+	/* the backward's staged form, where a step's input adjoints fit in LDS
+	 * (20 224 neurons): 256 blocks share the neurons, one per compute unit,
+	 * since each stages all the adjoints */
+	m_tile = unsigned((m_n + 255) / 256);
+	m_pushPitch = nemo_float_push_pitch(unsigned(m_n));
+	m_push = mayStage && (size_t(m_pushPitch) + 2 + m_tile) * sizeof(double) <= NEMO_FLOAT_PUSH_LDS;
+	std::vector<uint32_t> rowLen(m_push ? m_n * m_D : 0, 0); /* synapses by (source, delay) */
+
 	/* forward order = network order: sources ascending, insertion order */
 	std::vector<uint32_t> fptr(m_n + 1, 0), ftd(std::max<size_t>(1, m_s)), tgtOf(std::max<size_t>(1, m_s));
 	std::vector<uint32_t> incoming(m_n + 1, 0);
@@ -56,6 +67,7 @@ FloatNetwork::FloatNetwork(const Network& net, int device) : m_device(device < 0
 			const uint32_t tgt = ax.target[i];
 			if(tgt >= m_n) throw Error(NEMO_INVALID_INPUT, "Invalid synapse target neuron " + std::to_string(tgt));
 			ftd[k] = tgt | (uint32_t(ax.delay[i] - 1) << 26);
+			if(!rowLen.empty()) rowLen[kv.first * size_t(m_D) + ax.delay[i] - 1] += 1;
 			tgtOf[k] = tgt;
 			incoming[tgt + 1] += 1;
 		}
@@ -80,24 +92,157 @@ FloatNetwork::FloatNetwork(const Network& net, int device) : m_device(device < 0
 	};
 	upload(m_fcmPtr, fptr);
 	upload(m_fcmTd, ftd);
+	PushRows push;
+	if(m_push) {
+		push = pushRows(rowLen);
+		m_push = !push.ptr.empty();
+	}
+	if(m_push) {
+		upload(m_rowSlices, push.ptr);
+		m_rows.allocate(push.rows.size());
+		HIP_CHECK(hipMemcpy(m_rows.ptr, push.rows.data(), m_rows.bytes(), hipMemcpyHostToDevice));
+		const size_t entries = std::max<size_t>(1, push.ptr.back()) * 256;
+		m_rowUser.allocate(entries);
+		m_rowTarget.allocate(entries);
+		m_rowW.allocate(entries);
+		m_rowGw.allocate(entries);
+		HIP_CHECK(hipMemset(m_rowUser.ptr, 0xff, m_rowUser.bytes()));
+		HIP_CHECK(hipMemsetD16(reinterpret_cast<hipDeviceptr_t>(m_rowTarget.ptr), uint16_t(m_pushPitch), entries));
+		DeviceArray<uint32_t> rowAt;
+		upload(rowAt, push.at);
+		nemo_float_rows_args fill = {};
+		fill.n = unsigned(m_n);
+		fill.dmax = m_D;
+		fill.lanes = m_pushLanes;
+		fill.fcm_ptr = m_fcmPtr.ptr;
+		fill.fcm_td = m_fcmTd.ptr;
+		fill.row_at = rowAt.ptr;
+		fill.row_user = m_rowUser.ptr;
+		fill.row_target = m_rowTarget.ptr;
+		HIP_CHECK(nemo_launch_float_fill_rows(nullptr, &fill));
+		HIP_CHECK(hipStreamSynchronize(nullptr));
+		m_fcmPtr.release();
+		m_fcmTd.release();
+		m_LI.allocate(2 * size_t(m_pushPitch) + size_t(m_D) * m_n);
+	} else {
+		m_LI.allocate(size_t(m_D + 1) * m_n);
+	}
 	upload(m_rcmPtr, incoming);
 	upload(m_rcmSd, rsd);
 	upload(m_rcmUser, ruser);
-	m_wr.allocate(std::max<size_t>(1, m_s));
 	m_v.allocate(m_n);
 	m_u.allocate(m_n);
 	m_LV.allocate(m_n);
 	m_LU.allocate(m_n);
-	m_LI.allocate(size_t(m_D + 1) * m_n);
 	m_pitch = nemo_float_bitmap_pitch(unsigned(m_n));
 	/* stage the recent spike bitmaps in LDS when they fit and cost fewer
 	 * cache lines than a block's (32 neurons') spike gathers would */
 	const size_t stage = nemo_float_stage_bytes(unsigned(m_n), m_D);
-	m_stage = stage <= NEMO_FLOAT_STAGE_MAX && stage / 64 <= 32 * (m_s / std::max<size_t>(1, m_n));
-	/* NEMO_HIP_FLOAT_STAGE=0 reads the bitmaps from global memory instead */
-	if(const char* e = std::getenv("NEMO_HIP_FLOAT_STAGE")) {
-		if(std::string(e) == "0") m_stage = false;
+	m_stage = mayStage && stage <= NEMO_FLOAT_STAGE_MAX && stage / 64 <= 32 * (m_s / std::max<size_t>(1, m_n));
+	/* the sliced form reads the staged bitmaps; where it cannot be, or where
+	 * its weights do not fit a workspace that the plain order fits, the sums
+	 * are the same */
+	if(m_stage) {
+		const std::vector<uint32_t> slices = pullSlices(incoming);
+		if(!slices.empty()) {
+			upload(m_slicePtr, slices);
+			const size_t entries = std::max<size_t>(1, slices.back()) * 256;
+			m_sliceSd.allocate(entries);
+			m_sliceUser.allocate(entries);
+			HIP_CHECK(hipMemset(m_sliceSd.ptr, 0, m_sliceSd.bytes()));
+			HIP_CHECK(hipMemset(m_sliceUser.ptr, 0xff, m_sliceUser.bytes()));
+			nemo_float_slice_args fill = {};
+			fill.n = unsigned(m_n);
+			fill.dmax = m_D;
+			fill.synapses = m_s;
+			fill.rcm_ptr = m_rcmPtr.ptr;
+			fill.rcm_sd = m_rcmSd.ptr;
+			fill.rcm_user = m_rcmUser.ptr;
+			fill.slice_ptr = m_slicePtr.ptr;
+			fill.slice_sd = m_sliceSd.ptr;
+			fill.slice_user = m_sliceUser.ptr;
+			HIP_CHECK(nemo_launch_float_fill_slices(nullptr, &fill));
+			HIP_CHECK(hipStreamSynchronize(nullptr));
+		}
 	}
+	HIP_CHECK(nemo_float_staged_attributes());
+	m_wr.allocate(std::max(std::max<size_t>(1, m_s), m_sliceUser.n));
+}
+
+/* The slices of backward_push_kernel: a block's rows of (source, delay), longest
+ * first.  rowLen holds each row's synapses. */
+FloatNetwork::PushRows FloatNetwork::pushRows(const std::vector<uint32_t>& rowLen)
+{
+	/* as many lanes per row as leave a wave for the neurons, and four
+	 * synapses or more per lane on average: 100 training steps of 10 000 x 200
+	 * (rows of 20, two lanes) take 1327 us, with one lane 1430, with four
+	 * 1424; 50 steps of 1000 x 100 (rows of 10, two lanes) 441, 493 and 443 */
+	const size_t rowsPerBlock = size_t(m_tile) * m_D;
+	const size_t perRow = m_s / std::max<size_t>(1, m_n * m_D);
+	m_pushLanes = 1;
+	while(m_pushLanes < 32 && rowsPerBlock * m_pushLanes * 2 <= 960 && m_pushLanes * 8 <= perRow) m_pushLanes *= 2;
+	const unsigned L = m_pushLanes;
+	const unsigned groups = 64 / L;
+	m_slices = unsigned((rowsPerBlock + groups - 1) / groups);
+	const size_t blocks = (m_n + m_tile - 1) / m_tile;
+
+	PushRows out;
+	out.ptr.assign(blocks * m_slices + 1, 0);
+	out.rows.assign(blocks * m_slices * 64, nemo_float_row{0, 0});
+	out.at.assign(m_n * m_D, 0);
+	std::vector<uint32_t> order, bins;
+	for(size_t b = 0; b < blocks; ++b) {
+		const size_t first = b * m_tile;
+		const size_t rows = std::min<size_t>(m_tile, m_n - first) * m_D;
+		const uint32_t* len = rowLen.data() + first * m_D;
+		const uint32_t longestRow = *std::max_element(len, len + rows);
+		bins.assign(longestRow + 2, 0);
+		for(size_t r = 0; r < rows; ++r) bins[longestRow - len[r] + 1] += 1;
+		for(size_t k = 0; k + 1 < bins.size(); ++k) bins[k + 1] += bins[k];
+		order.resize(rows);
+		for(size_t r = 0; r < rows; ++r) order[bins[longestRow - len[r]]++] = uint32_t(r);
+		for(unsigned s = 0; s < m_slices; ++s) {
+			const size_t slice = b * m_slices + s;
+			const size_t r0 = size_t(s) * groups;
+			const size_t longest = r0 < rows ? len[order[r0]] : 0;
+			const size_t base = out.ptr[slice];
+			const size_t next = base + (longest + 4 * L - 1) / (4 * L);
+			/* rows far longer than most would fill slices with nothing */
+			if(next * 256 > 2 * m_s + 256 * (slice + 1) || next * 256 > UINT32_MAX) return PushRows();
+			out.ptr[slice + 1] = uint32_t(next);
+			for(size_t g = 0; g < groups && r0 + g < rows; ++g) {
+				const uint32_t r = order[r0 + g];
+				for(unsigned l = 0; l < L; ++l)
+					out.rows[slice * 64 + g * L + l] = {uint16_t(r / m_D), uint16_t(r % m_D + 1)};
+				out.at[first * m_D + r] = uint32_t(base * 256 + g * L * 4);
+			}
+		}
+	}
+	return out;
+}
+
+/* The slices of forward_sliced_kernel, or nothing. */
+std::vector<uint32_t> FloatNetwork::pullSlices(const std::vector<uint32_t>& ptr)
+{
+	const size_t slices = (m_n + 7) / 8;
+	std::vector<uint32_t> out(slices + 1, 0);
+	m_sliceLines = 0;
+	for(size_t s = 0; s < slices; ++s) {
+		uint32_t longest = 0;
+		for(size_t j = 8 * s; j < std::min(m_n, 8 * s + 8); ++j) longest = std::max(longest, ptr[j + 1] - ptr[j]);
+		const uint32_t lines = longest / 32 + (longest % 32 != 0);
+		/* targets far beyond their neighbours would fill slices with nothing */
+		if((size_t(out[s]) + lines) * 256 > 2 * m_s + 256 * (s + 1) || lines > 65535) return {};
+		out[s + 1] = out[s] + lines;
+		m_sliceLines = std::max(m_sliceLines, lines);
+	}
+	return out;
+}
+
+void FloatNetwork::sliceWeights(hipStream_t st, float* wr, const float* w)
+{
+	HIP_CHECK(nemo_launch_float_slice_weights(st, wr, w, m_sliceUser.ptr, m_slicePtr.ptr, unsigned(m_slicePtr.n - 1),
+			m_sliceLines, m_s));
 }
 
 void FloatNetwork::prepare(unsigned T, unsigned K)
@@ -122,6 +267,7 @@ void FloatNetwork::forward(hipStream_t st, unsigned T, unsigned K, const float* 
 {
 	prepare(T, K);
 	ForwardWorkspace ws;
+	ws.sliced = m_sliceUser.n != 0;
 	ws.wr = m_wr.ptr;
 	ws.v = m_v.ptr;
 	ws.u = m_u.ptr;
@@ -144,31 +290,33 @@ void FloatNetwork::forwardStatic(hipStream_t st, unsigned T, unsigned K, const f
 	void* base = nullptr;
 	size_t cap = 0;
 	HIP_CHECK(nemo_float_scratch(&base, &cap));
-	const size_t need = forwardWorkspaceBytes(T);
+	const bool sliced = m_sliceUser.n && forwardWorkspaceBytes(T, true) <= cap;
+	const size_t need = forwardWorkspaceBytes(T, sliced);
 	if(need > cap) {
 		throw Error(NEMO_INVALID_INPUT, "the allocation-free forward of " + std::to_string(T) + " steps needs "
 				+ std::to_string(need) + " bytes of workspace; its static workspace holds " + std::to_string(cap));
 	}
-	forwardWith(carveWorkspace(base, T), st, T, K, w, a, b, c, d, v0, u0, x, S, V, ckpt);
+	forwardWith(carveWorkspace(base, T, sliced), st, T, K, w, a, b, c, d, v0, u0, x, S, V, ckpt);
 }
 
 /* Bytes of the forward's workspace for T steps, each part 256-byte aligned:
  * weights in reverse order (4 B per synapse), v and u in double (16 B per
  * neuron) and the spike bitmaps of every step. */
-size_t FloatNetwork::forwardWorkspaceBytes(unsigned T) const
+size_t FloatNetwork::forwardWorkspaceBytes(unsigned T, bool sliced) const
 {
 	auto up = [](size_t x) { return (x + 255) / 256 * 256; };
-	return up(std::max<size_t>(1, m_s) * sizeof(float)) + 2 * up(m_n * sizeof(double))
+	return up((sliced ? m_sliceUser.n : std::max<size_t>(1, m_s)) * sizeof(float)) + 2 * up(m_n * sizeof(double))
 		+ up(size_t(T) * m_pitch * sizeof(uint32_t));
 }
 
-FloatNetwork::ForwardWorkspace FloatNetwork::carveWorkspace(void* base, unsigned T) const
+FloatNetwork::ForwardWorkspace FloatNetwork::carveWorkspace(void* base, unsigned T, bool sliced) const
 {
 	auto up = [](size_t x) { return (x + 255) / 256 * 256; };
 	unsigned char* p = static_cast<unsigned char*>(base);
 	ForwardWorkspace ws;
+	ws.sliced = sliced;
 	ws.wr = reinterpret_cast<float*>(p);
-	p += up(std::max<size_t>(1, m_s) * sizeof(float));
+	p += up((sliced ? m_sliceUser.n : std::max<size_t>(1, m_s)) * sizeof(float));
 	ws.v = reinterpret_cast<double*>(p);
 	p += up(m_n * sizeof(double));
 	ws.u = reinterpret_cast<double*>(p);
@@ -187,9 +335,19 @@ void FloatNetwork::forwardWith(const ForwardWorkspace& ws, hipStream_t st, unsig
 	if(T == 0) throw Error(NEMO_INVALID_INPUT, "the float-weight mode needs at least one step");
 	if(K == 0) throw Error(NEMO_INVALID_INPUT, "checkpoint interval must be positive");
 	HIP_CHECK(hipSetDevice(m_device));
-	HIP_CHECK(nemo_launch_gather(st, ws.wr, w, m_rcmUser.ptr, m_s));
-	HIP_CHECK(nemo_launch_widen(st, ws.v, v0, m_n));
-	HIP_CHECK(nemo_launch_widen(st, ws.u, u0, m_n));
+	nemo_float_begin_forward_args begin = {};
+	begin.n = m_n;
+	begin.synapses = m_s;
+	begin.w = w;
+	begin.wr_entries = ws.sliced ? 0 : m_s;
+	begin.wr_user = m_rcmUser.ptr;
+	begin.wr = ws.wr;
+	begin.v0 = v0;
+	begin.u0 = u0;
+	begin.v = ws.v;
+	begin.u = ws.u;
+	HIP_CHECK(nemo_launch_float_begin_forward(st, &begin));
+	if(ws.sliced) sliceWeights(st, ws.wr, w);
 	nemo_float_step_args f = {};
 	f.n = unsigned(m_n);
 	f.rcm_ptr = m_rcmPtr.ptr;
@@ -211,6 +369,8 @@ void FloatNetwork::forwardWith(const ForwardWorkspace& ws, hipStream_t st, unsig
 	f.pitch = m_pitch;
 	f.dmax = m_D;
 	f.stage = m_stage;
+	f.slice_ptr = ws.sliced ? m_slicePtr.ptr : nullptr;
+	f.slice_sd = m_sliceSd.ptr;
 	for(unsigned t = 0; t < T; ++t) {
 		f.t = t;
 		HIP_CHECK(nemo_launch_float_forward_step(st, &f));
@@ -226,14 +386,28 @@ void FloatNetwork::backward(hipStream_t st, unsigned T, unsigned K, const float*
 		float* gv0, float* gu0)
 {
 	prepare(T, K);
-	HIP_CHECK(nemo_launch_gather(st, m_wr.ptr, w, m_rcmUser.ptr, m_s));
-	HIP_CHECK(nemo_launch_fill_double(st, m_LV.ptr, 0.0, m_n));
-	HIP_CHECK(nemo_launch_fill_double(st, m_LU.ptr, 0.0, m_n));
-	HIP_CHECK(nemo_launch_fill_double(st, m_LI.ptr, 0.0, m_LI.n));
-	HIP_CHECK(nemo_launch_fill(st, gw, 0.0f, m_s));
-	HIP_CHECK(nemo_launch_fill(st, ga, 0.0f, m_n));
-	HIP_CHECK(nemo_launch_fill(st, gb, 0.0f, m_n));
-	HIP_CHECK(nemo_launch_fill(st, gd, 0.0f, m_n));
+	nemo_float_begin_backward_args begin = {};
+	begin.n = m_n;
+	begin.synapses = m_s;
+	begin.li = m_LI.n;
+	begin.w = w;
+	const bool sliced = m_sliceUser.n && m_n <= NEMO_FLOAT_REPLAY_MAX && m_D < 58;
+	begin.wr_entries = sliced ? 0 : m_s;
+	begin.wr_user = m_rcmUser.ptr;
+	begin.wr = m_wr.ptr;
+	begin.row_user = m_rowUser.ptr;
+	begin.entries = m_push ? m_rowUser.n : 0;
+	begin.row_w = m_rowW.ptr;
+	begin.row_gw = m_rowGw.ptr;
+	begin.LI = m_LI.ptr;
+	begin.LV = m_LV.ptr;
+	begin.LU = m_LU.ptr;
+	begin.gw = gw;
+	begin.ga = ga;
+	begin.gb = gb;
+	begin.gd = gd;
+	HIP_CHECK(nemo_launch_float_begin_backward(st, &begin));
+	if(sliced) sliceWeights(st, m_wr.ptr, w);
 	const unsigned Kseg = std::min(K, T);
 	const size_t segPlane = size_t(Kseg) * m_n;
 
@@ -257,32 +431,64 @@ void FloatNetwork::backward(hipStream_t st, unsigned T, unsigned K, const float*
 	f.seg_v = m_seg.ptr;
 	f.seg_u = m_seg.ptr + segPlane;
 	f.seg_I = m_seg.ptr + 2 * segPlane;
+	f.slice_ptr = sliced ? m_slicePtr.ptr : nullptr;
+	f.slice_sd = m_sliceSd.ptr;
 
+	nemo_float_push_args p = {};
 	nemo_float_back_args g = {};
-	g.n = unsigned(m_n);
-	g.T = T;
-	g.ring = m_D + 1;
-	g.fcm_ptr = m_fcmPtr.ptr;
-	g.fcm_td = m_fcmTd.ptr;
-	g.wf = w;
-	g.pa = a;
-	g.pb = b;
-	g.pc = c;
-	g.pd = d;
-	g.S = S;
-	g.gS = gS;
-	g.gV = gV;
-	g.seg_v = f.seg_v;
-	g.seg_u = f.seg_u;
-	g.seg_I = f.seg_I;
-	g.LV = m_LV.ptr;
-	g.LU = m_LU.ptr;
-	g.LI = m_LI.ptr;
-	g.gw = gw;
-	g.ga = ga;
-	g.gb = gb;
-	g.gd = gd;
-	g.gx = gx;
+	if(m_push) {
+		p.n = unsigned(m_n);
+		p.T = T;
+		p.dmax = m_D;
+		p.tile = m_tile;
+		p.pitch = m_pushPitch;
+		p.lanes = m_pushLanes;
+		p.slices = m_slices;
+		p.slice_ptr = m_rowSlices.ptr;
+		p.rows = m_rows.ptr;
+		p.row_target = m_rowTarget.ptr;
+		p.row_w = m_rowW.ptr;
+		p.row_gw = m_rowGw.ptr;
+		p.pa = a;
+		p.pb = b;
+		p.S = S;
+		p.gS = gS;
+		p.gV = gV;
+		p.seg_v = f.seg_v;
+		p.seg_u = f.seg_u;
+		p.seg_I = f.seg_I;
+		p.LV = m_LV.ptr;
+		p.LU = m_LU.ptr;
+		p.LI = m_LI.ptr;
+		p.ring = m_LI.ptr + 2 * size_t(m_pushPitch);
+		p.ga = ga;
+		p.gb = gb;
+		p.gd = gd;
+		p.gx = gx;
+	} else {
+		g.n = unsigned(m_n);
+		g.T = T;
+		g.ring = m_D + 1;
+		g.fcm_ptr = m_fcmPtr.ptr;
+		g.fcm_td = m_fcmTd.ptr;
+		g.wf = w;
+		g.pa = a;
+		g.pb = b;
+		g.S = S;
+		g.gS = gS;
+		g.gV = gV;
+		g.seg_v = f.seg_v;
+		g.seg_u = f.seg_u;
+		g.seg_I = f.seg_I;
+		g.LV = m_LV.ptr;
+		g.LU = m_LU.ptr;
+		g.LI = m_LI.ptr;
+		g.gw = gw;
+		g.ga = ga;
+		g.gb = gb;
+		g.gd = gd;
+		g.gx = gx;
+	}
 
 	const unsigned segments = (T + K - 1) / K;
 	for(unsigned s = segments; s-- > 0;) {
@@ -293,14 +499,25 @@ void FloatNetwork::backward(hipStream_t st, unsigned T, unsigned K, const float*
 		f.v0 = ckpt + size_t(s) * 2 * m_n;
 		f.u0 = ckpt + size_t(s) * 2 * m_n + m_n;
 		HIP_CHECK(nemo_launch_float_replay(st, &f));
-		g.t0 = t0;
+		p.t0 = g.t0 = t0;
 		for(unsigned t = t1; t-- > t0;) {
-			g.t = t;
-			HIP_CHECK(nemo_launch_float_backward_step(st, &g));
+			p.t = g.t = t;
+			if(m_push) HIP_CHECK(nemo_launch_float_push_step(st, &p));
+			else HIP_CHECK(nemo_launch_float_backward_step(st, &g));
 		}
 	}
-	if(gv0) HIP_CHECK(nemo_launch_narrow(st, gv0, m_LV.ptr, m_n));
-	if(gu0) HIP_CHECK(nemo_launch_narrow(st, gu0, m_LU.ptr, m_n));
+	nemo_float_end_backward_args done = {};
+	done.n = m_n;
+	done.synapses = m_s;
+	done.entries = m_push ? m_rowUser.n : 0;
+	done.row_user = m_rowUser.ptr;
+	done.row_gw = m_rowGw.ptr;
+	done.gw = gw;
+	done.LV = m_LV.ptr;
+	done.LU = m_LU.ptr;
+	done.gv0 = gv0;
+	done.gu0 = gu0;
+	HIP_CHECK(nemo_launch_float_end_backward(st, &done));
 }
 
 } // namespace nemo_hip

@@ -218,3 +218,54 @@ def test_hh_substeps_match_oracle(n):
             a, b = (np.asarray(s.neuron_states(k), np.float32) for s in sims)
             same = (a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))
             assert same.all(), (t, k, np.flatnonzero(~same)[:5])
+
+
+# ------------------------------------------------- float mode's staged forms
+@pytest.mark.parametrize("n,m,dmax,T", [
+    (2, 1, 1, 5),          # one delay: every row starts its slot
+    (255, 7, 2, 9),        # an odd size, one neuron per block, slices of one row
+    (1025, 40, 3, 30),     # a last block of neurons that is not full
+    (400, 300, 5, 40),     # more synapses than a wave has in flight
+    (300, 40, 57, 60),     # the longest delay of the windowed replay
+    (600, 130, 64, 90),    # beyond it; more slices than waves
+    (12000, 25, 19, 40),   # a lane per row
+    (20280, 12, 5, 12),    # the largest network whose adjoints fit in LDS
+    (20500, 12, 5, 12),    # one beyond that and the windows
+])
+def test_float_staged_and_general_agree(n, m, dmax, T, monkeypatch):
+    """The kernels that read their synapses in slices, with spikes and adjoints
+    in LDS, and the general ones.  The forward sums in the same order, so
+    spikes and potentials are the same bits.  The backward sums the same
+    doubles in another order, so the gradients, which are accumulated over T
+    steps in float, differ by at most T roundings of 2^-24; fired sources,
+    steps before the first and after the last included."""
+    torch = pytest.importorskip("torch")
+    from nemo_amd.differentiable import FloatNetwork
+    spec = gen.random_izhikevich(n, m, dmax=dmax, seed=n)
+    rng = np.random.default_rng(n)
+    spec.weight = (spec.weight * np.float32(30.0 / m)).astype(np.float32)
+    a, b, c, d, _, u, v = [np.asarray(x, np.float32) * np.ones(n, np.float32) for x in spec.blocks[0].args]
+    x = (8.0 * rng.standard_normal((T, n))).astype(np.float32)
+    gS, gV = (rng.standard_normal((T, n)).astype(np.float32) for _ in range(2))
+    outs, grads = [], []
+    for stage in ("1", "0"):
+        monkeypatch.setenv("NEMO_HIP_FLOAT_STAGE", stage)
+        net = nemo_amd.Network()
+        spec.load(net)
+        fnet = FloatNetwork(net, 0)
+        p = {k: torch.tensor(t, device="cuda") for k, t in dict(w=spec.weight, a=a, b=b, d=d, x=x, v0=v, u0=u).items()}
+        for t in p.values():
+            t.requires_grad_(True)
+        for _ in range(2):  # the second pass starts from the first one's leavings
+            for t in p.values():
+                t.grad = None
+            S, V = fnet(p["w"], p["a"], p["b"], p["d"], p["x"], c=torch.tensor(c, device="cuda"), v0=p["v0"],
+                        u0=p["u0"], checkpoint_every=17)
+            torch.autograd.backward([S, V], [torch.tensor(gS, device="cuda"), torch.tensor(gV, device="cuda")])
+        outs.append((S.detach(), V.detach()))
+        grads.append({k: t.grad.double().cpu() for k, t in p.items()})
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    assert n == 2 or float(outs[0][0].sum()) > 0  # two neurons are silent
+    for k in grads[0]:
+        staged, general = grads[0][k], grads[1][k]
+        assert float((staged - general).norm()) <= T * 2.0 ** -24 * float(general.norm()), k
