@@ -48,6 +48,12 @@ void DeviceArray<T>::release()
 	n = 0;
 }
 
+/* Plastic synapses from which applyStdp goes over tiles (apply_stdp_kernel): a
+ * call and a step take 108 us without and 101 with them at 1.6e6, 185 and 178
+ * at 8e6, 276 and 261 at 1.6e7, 620 and 483 at 3.2e7; below, the gain does
+ * not pay for the second copy of the accumulators. */
+static const size_t APPLY_TILE_MIN = size_t(12) << 20;
+
 template struct DeviceArray<float>;
 template struct DeviceArray<double>;
 template struct DeviceArray<uint16_t>;
@@ -1087,8 +1093,18 @@ void Simulation::buildConnectivity(const std::vector<const Network*>& nets, cons
 		HIP_CHECK(hipMemcpy(m_rcmFwd.ptr, rcmFwd.data(), m_rcmFwd.bytes(), hipMemcpyHostToDevice));
 		HIP_CHECK(hipMemset(m_rcmAcc.ptr, 0, m_rcmAcc.bytes()));
 		m_rcmOf.allocate(m_fcm.n);
-		HIP_CHECK(nemo_launch_invert_rcm(nullptr, m_rcmFwd.ptr, m_rcmOf.ptr, rcmFwd.size(), m_fcm.n));
-		HIP_CHECK(hipDeviceSynchronize());
+		if(m_nplastic >= APPLY_TILE_MIN) {
+			m_rcmTile.allocate(m_nplastic);
+			m_applyTile.allocate(m_fcm.n);
+			DeviceArray<uint32_t> used;
+			used.allocate(m_fcm.n / NEMO_APPLY_TILE + 1);
+			HIP_CHECK(nemo_launch_assign_tiles(nullptr, m_rcmFwd.ptr, m_rcmOf.ptr, m_rcmTile.ptr, used.ptr, m_nplastic,
+					m_fcm.n));
+			HIP_CHECK(hipDeviceSynchronize());
+		} else {
+			HIP_CHECK(nemo_launch_invert_rcm(nullptr, m_rcmFwd.ptr, m_rcmOf.ptr, rcmFwd.size(), m_fcm.n));
+			HIP_CHECK(hipDeviceSynchronize());
+		}
 	}
 }
 
@@ -2645,6 +2661,8 @@ void Simulation::applyStdp(float reward)
 	a.rcm_of = m_rcmOf.ptr;
 	a.fcm_count = m_fcm.n;
 	a.rcm_acc = m_rcmAcc.ptr;
+	a.tile = m_applyTile.ptr;
+	a.rcm_tile = m_rcmTile.ptr;
 	a.fcm = m_fcm.ptr;
 	a.count = m_nplastic;
 	a.reward = fx_reward;

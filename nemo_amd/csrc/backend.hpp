@@ -359,6 +359,8 @@ private:
 	DeviceArray<unsigned> m_status;   /* NEMO_HIP_STATUS_* bits set by the kernels */
 	bool m_checkStatus = false;       /* some model may set status bits */
 	DeviceArray<int32_t> m_rcmAcc;
+	DeviceArray<uint32_t> m_rcmTile;  /* applyStdp with tiles: per accumulator, its place in */
+	DeviceArray<int32_t> m_applyTile;
 	DeviceArray<int2> m_bins;
 	DeviceArray<uint32_t> m_binTable;
 	DeviceArray<uint32_t> m_pairBounds, m_binRange;

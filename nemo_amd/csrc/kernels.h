@@ -91,8 +91,10 @@ hipError_t nemo_launch_propagate_sets(hipStream_t, const nemo_propagate_args* a,
 /* applyStdp (ConnectivityMatrix::applyStdp, ConnectivityMatrix.cpp:272-325 and
  * StdpProcess::updatedWeight, StdpProcess.cpp:128-138). */
 typedef struct nemo_apply_args {
-	const uint32_t* rcm_of;          /* per FCM synapse: its accumulator index, or ~0 if static */
+	const uint32_t* rcm_of;          /* per FCM synapse: its accumulator index (in tile, if any), or ~0 if static */
 	int32_t* rcm_acc;
+	int32_t* tile;                   /* accumulators by FCM synapse / NEMO_APPLY_TILE, or NULL */
+	const uint32_t* rcm_tile;        /* with tile: per accumulator, its place there */
 	int2* fcm;
 	size_t count;                    /* plastic synapses */
 	size_t fcm_count;                /* FCM synapses */
@@ -101,7 +103,12 @@ typedef struct nemo_apply_args {
 	unsigned fbits;
 } nemo_apply_args;
 
+#define NEMO_APPLY_TILE (1u << 19)
 hipError_t nemo_launch_apply_stdp(hipStream_t, const nemo_apply_args*);
+/* rcm_of (fcm_count entries) and rcm_tile (count entries) for an applyStdp
+ * with tiles of fcm_count entries in all; used: an entry per tile. */
+hipError_t nemo_launch_assign_tiles(hipStream_t, const uint32_t* rcm_fwd, uint32_t* rcm_of, uint32_t* rcm_tile,
+		uint32_t* used, size_t count, size_t fcm_count);
 /* rcm_of (fcm_count entries): the accumulator index of every plastic
  * synapse, ~0 for the others, from rcm_fwd (count entries). */
 hipError_t nemo_launch_invert_rcm(hipStream_t, const uint32_t* rcm_fwd, uint32_t* rcm_of, size_t count,

@@ -142,39 +142,132 @@ __global__ void stdp_flush_done_kernel(nemo_hip_clock* clock, uint64_t offset)
  * (rcm_of[j] its accumulator) takes its weight change; reading the weights in
  * order and the accumulators scattered costs one random read per synapse,
  * where the reverse order costs a random read and write of the weight.  The
- * accumulators are cleared afterwards by a separate fill. */
+ * accumulators are cleared afterwards by a separate fill.
+ *
+ * The random reads are cache lines that an XCD's L2 does not hold: 1660 us at
+ * 1e8 synapses, 8e7 of them plastic.  So in large networks (a.tile) the
+ * accumulators are first moved to tiles of APPLY_TILE consecutive FCM synapses
+ * each (apply_collect_kernel, which also clears them), and the blocks of an
+ * XCD, which are those of one number modulo 8, pass a tile together: it stays
+ * in their L2: 372 + 638 us, of 2.3 + 1.3 GB.  Tiles of half or twice the size
+ * take the same in sum. */
+__device__ inline int32_t applied_weight(const nemo_apply_args& a, int32_t w, int32_t acc)
+{
+	const int32_t x = stdp_wrap_add(w, int32_t((int64_t(a.reward) * int64_t(acc)) >> a.fbits));
+	return w > 0 ? min(a.maxE, max(x, a.minE)) : w < 0 ? min(a.minI, max(x, a.maxI)) : 0;
+}
+
 __global__ void __launch_bounds__(NEMO_BLOCK)
 apply_stdp_kernel(nemo_apply_args a)
 {
-	/* APPLY_ILP synapses per thread at a time: their index and weight loads,
-	 * then their accumulator gathers, are in flight together */
+	/* APPLY_ILP pairs of synapses per thread at a time: their index and weight
+	 * loads, then their accumulator gathers, are in flight together */
 	constexpr unsigned APPLY_ILP = 4;
-	const size_t stride = size_t(gridDim.x) * NEMO_BLOCK * APPLY_ILP;
-	for(size_t j0 = size_t(blockIdx.x) * NEMO_BLOCK * APPLY_ILP + threadIdx.x; j0 < a.fcm_count; j0 += stride) {
-		uint32_t k[APPLY_ILP];
-		int32_t w_old[APPLY_ILP], acc[APPLY_ILP];
+	constexpr size_t PIECE = NEMO_BLOCK * APPLY_ILP; /* pairs */
+	constexpr size_t PIECES = NEMO_APPLY_TILE / 2 / PIECE; /* of a tile */
+	size_t piece = blockIdx.x;
+	if(a.tile) {
+		const size_t g = blockIdx.x / 8;
+		piece = (g / PIECES * 8 + blockIdx.x % 8) * PIECES + g % PIECES;
+	}
+	const size_t stride = size_t(gridDim.x) * PIECE;
+	const size_t pairs = a.fcm_count / 2;
+	const int32_t* source = a.tile ? a.tile : a.rcm_acc;
+	const uint2* of = reinterpret_cast<const uint2*>(a.rcm_of);
+	int4* fcm = reinterpret_cast<int4*>(a.fcm);
+	for(size_t j0 = piece * PIECE + threadIdx.x; j0 < pairs; j0 += stride) {
+		uint2 k[APPLY_ILP];
+		int4 w[APPLY_ILP];
+		int2 acc[APPLY_ILP];
 #pragma unroll
 		for(unsigned u = 0; u < APPLY_ILP; ++u) {
 			const size_t j = j0 + u * NEMO_BLOCK;
-			k[u] = j < a.fcm_count ? a.rcm_of[j] : ~0u;
-			w_old[u] = j < a.fcm_count ? a.fcm[j].y : 0;
+			k[u] = j < pairs ? of[j] : make_uint2(~0u, ~0u);
+			w[u] = j < pairs ? fcm[j] : make_int4(0, 0, 0, 0);
 		}
-#pragma unroll
-		for(unsigned u = 0; u < APPLY_ILP; ++u) acc[u] = k[u] != ~0u && a.reward != 0 ? a.rcm_acc[k[u]] : 0;
 #pragma unroll
 		for(unsigned u = 0; u < APPLY_ILP; ++u) {
-			if(k[u] == ~0u) continue;
-			const int32_t dw = int32_t((int64_t(a.reward) * int64_t(acc[u])) >> a.fbits);
-			int32_t w_new = 0;
-			if(w_old[u] > 0) {
-				const int32_t x = stdp_wrap_add(w_old[u], dw);
-				w_new = min(a.maxE, max(x, a.minE));
-			} else if(w_old[u] < 0) {
-				const int32_t x = stdp_wrap_add(w_old[u], dw);
-				w_new = min(a.minI, max(x, a.maxI));
-			}
-			if(w_new != w_old[u]) a.fcm[j0 + u * NEMO_BLOCK].y = w_new;
+			acc[u].x = k[u].x != ~0u && a.reward != 0 ? source[k[u].x] : 0;
+			acc[u].y = k[u].y != ~0u && a.reward != 0 ? source[k[u].y] : 0;
 		}
+#pragma unroll
+		for(unsigned u = 0; u < APPLY_ILP; ++u) {
+			const int32_t x = k[u].x != ~0u ? applied_weight(a, w[u].y, acc[u].x) : w[u].y;
+			const int32_t y = k[u].y != ~0u ? applied_weight(a, w[u].w, acc[u].y) : w[u].w;
+			/* changed or not: whole lines are written faster than some words of
+			 * them (638 against 685 us at 1e8 synapses, a third changed) */
+			if(k[u].x != ~0u || k[u].y != ~0u) fcm[j0 + u * NEMO_BLOCK] = make_int4(w[u].x, x, w[u].z, y);
+		}
+	}
+	if(a.fcm_count % 2 && blockIdx.x == 0 && threadIdx.x == 0) {
+		const size_t j = a.fcm_count - 1;
+		const uint32_t k = a.rcm_of[j];
+		if(k != ~0u) a.fcm[j].y = applied_weight(a, a.fcm[j].y, a.reward != 0 ? source[k] : 0);
+	}
+}
+
+/* The accumulators to their tiles, and cleared: in target order, in which they
+ * are read and the places in a tile run on. */
+__global__ void __launch_bounds__(NEMO_BLOCK)
+apply_collect_kernel(nemo_apply_args a)
+{
+	constexpr unsigned ILP = 4;
+	const size_t quads = a.count / 4;
+	const size_t stride = size_t(gridDim.x) * NEMO_BLOCK * ILP;
+	for(size_t q0 = size_t(blockIdx.x) * NEMO_BLOCK * ILP + threadIdx.x; q0 < quads; q0 += stride) {
+		int4 acc[ILP];
+		uint4 at[ILP];
+#pragma unroll
+		for(unsigned u = 0; u < ILP; ++u) {
+			const size_t q = q0 + u * NEMO_BLOCK;
+			if(q >= quads) continue;
+			acc[u] = reinterpret_cast<const int4*>(a.rcm_acc)[q];
+			at[u] = reinterpret_cast<const uint4*>(a.rcm_tile)[q];
+		}
+#pragma unroll
+		for(unsigned u = 0; u < ILP; ++u) {
+			const size_t q = q0 + u * NEMO_BLOCK;
+			if(q >= quads) continue;
+			a.tile[at[u].x] = acc[u].x;
+			a.tile[at[u].y] = acc[u].y;
+			a.tile[at[u].z] = acc[u].z;
+			a.tile[at[u].w] = acc[u].w;
+			reinterpret_cast<int4*>(a.rcm_acc)[q] = make_int4(0, 0, 0, 0);
+		}
+	}
+	const size_t k = quads * 4 + threadIdx.x;
+	if(blockIdx.x == 0 && k < a.count) {
+		a.tile[a.rcm_tile[k]] = a.rcm_acc[k];
+		a.rcm_acc[k] = 0;
+	}
+}
+
+/* The place of every plastic synapse k in the tiles: rcm_tile[k] =
+ * rcm_of[rcm_fwd[k]] (rcm_of filled with ~0 before), in tile rcm_fwd[k] /
+ * APPLY_TILE, where a block's synapses, of neighbouring targets, follow each
+ * other; used counts the places taken of each tile (zero before). */
+constexpr unsigned TILE_SPAN = 16384; /* synapses per block */
+constexpr unsigned TILE_MAX = 8192;   /* tiles: of 2^32 synapses */
+
+__global__ void __launch_bounds__(NEMO_BLOCK)
+assign_tiles_kernel(const uint32_t* rcm_fwd, uint32_t* rcm_of, uint32_t* rcm_tile, uint32_t* used, unsigned tiles,
+		size_t count)
+{
+	__shared__ uint32_t place[TILE_MAX];
+	const size_t first = size_t(blockIdx.x) * TILE_SPAN;
+	const size_t last = min(count, first + TILE_SPAN);
+	for(unsigned t = threadIdx.x; t < tiles; t += NEMO_BLOCK) place[t] = 0;
+	__syncthreads();
+	for(size_t k = first + threadIdx.x; k < last; k += NEMO_BLOCK) atomicAdd(&place[rcm_fwd[k] / NEMO_APPLY_TILE], 1u);
+	__syncthreads();
+	for(unsigned t = threadIdx.x; t < tiles; t += NEMO_BLOCK)
+		if(place[t]) place[t] = t * NEMO_APPLY_TILE + atomicAdd(&used[t], place[t]);
+	__syncthreads();
+	for(size_t k = first + threadIdx.x; k < last; k += NEMO_BLOCK) {
+		const uint32_t f = rcm_fwd[k];
+		const uint32_t at = atomicAdd(&place[f / NEMO_APPLY_TILE], 1u);
+		rcm_tile[k] = at;
+		rcm_of[f] = at;
 	}
 }
 
@@ -546,7 +639,20 @@ hipError_t nemo_launch_propagate_sets(hipStream_t st, const nemo_propagate_args*
 hipError_t nemo_launch_apply_stdp(hipStream_t st, const nemo_apply_args* a)
 {
 	if(a->count == 0) return hipSuccess;
-	size_t blocks = (a->fcm_count + 4 * NEMO_BLOCK - 1) / (4 * NEMO_BLOCK);
+	if(a->tile) {
+		if(!a->rcm_tile) return hipErrorInvalidValue;
+		size_t blocks = (a->count + 16 * NEMO_BLOCK - 1) / (16 * NEMO_BLOCK);
+		if(blocks > 16384) blocks = 16384;
+		hipLaunchKernelGGL(apply_collect_kernel, dim3(unsigned(blocks)), dim3(NEMO_BLOCK), 0, st, *a);
+		hipError_t e = hipGetLastError();
+		if(e != hipSuccess) return e;
+		/* whole tiles for each XCD */
+		const size_t tiles = (a->fcm_count + NEMO_APPLY_TILE - 1) / NEMO_APPLY_TILE;
+		blocks = (tiles + 7) / 8 * 8 * (NEMO_APPLY_TILE / (8 * NEMO_BLOCK));
+		hipLaunchKernelGGL(apply_stdp_kernel, dim3(unsigned(blocks)), dim3(NEMO_BLOCK), 0, st, *a);
+		return hipGetLastError();
+	}
+	size_t blocks = (a->fcm_count + 8 * NEMO_BLOCK - 1) / (8 * NEMO_BLOCK);
 	if(blocks > 16384) blocks = 16384;
 	hipLaunchKernelGGL(apply_stdp_kernel, dim3(unsigned(blocks)), dim3(NEMO_BLOCK), 0, st, *a);
 	hipError_t e = hipGetLastError();
@@ -562,6 +668,20 @@ hipError_t nemo_launch_invert_rcm(hipStream_t st, const uint32_t* rcm_fwd, uint3
 	size_t blocks = (count + NEMO_BLOCK - 1) / NEMO_BLOCK;
 	if(blocks > 16384) blocks = 16384;
 	hipLaunchKernelGGL(invert_rcm_kernel, dim3(unsigned(blocks)), dim3(NEMO_BLOCK), 0, st, rcm_fwd, rcm_of, count);
+	return hipGetLastError();
+}
+
+hipError_t nemo_launch_assign_tiles(hipStream_t st, const uint32_t* rcm_fwd, uint32_t* rcm_of, uint32_t* rcm_tile,
+		uint32_t* used, size_t count, size_t fcm_count)
+{
+	const size_t tiles = (fcm_count + NEMO_APPLY_TILE - 1) / NEMO_APPLY_TILE;
+	if(tiles > TILE_MAX) return hipErrorInvalidValue;
+	hipError_t e = hipMemsetAsync(rcm_of, 0xff, fcm_count * sizeof(uint32_t), st);
+	if(e == hipSuccess) e = hipMemsetAsync(used, 0, tiles * sizeof(uint32_t), st);
+	if(e != hipSuccess || count == 0) return e;
+	const size_t blocks = (count + TILE_SPAN - 1) / TILE_SPAN;
+	hipLaunchKernelGGL(assign_tiles_kernel, dim3(unsigned(blocks)), dim3(NEMO_BLOCK), 0, st, rcm_fwd, rcm_of, rcm_tile,
+			used, unsigned(tiles), count);
 	return hipGetLastError();
 }
 

@@ -269,3 +269,30 @@ def test_float_staged_and_general_agree(n, m, dmax, T, monkeypatch):
     for k in grads[0]:
         staged, general = grads[0][k], grads[1][k]
         assert float((staged - general).norm()) <= T * 2.0 ** -24 * float(general.norm()), k
+
+
+# ------------------------------------------------- applyStdp over tiles
+@pytest.mark.parametrize("n,m", [(14000, 1200), (9001, 1777)])
+def test_apply_stdp_over_tiles(n, m):
+    """From 12 x 2^20 plastic synapses on, applyStdp moves the accumulators to
+    tiles of the forward matrix (more than 8 of them, the last one partial, an
+    odd number of synapses in the second case).  The weights equal the ones
+    that the reward's definition gives for the accumulators read before, in
+    whole numbers, and the accumulators are zero afterwards; twice, and with a
+    reward of zero, which only clears them."""
+    spec = gen.random_izhikevich(n, m, dmax=12, seed=n, stdp=True)
+    assert spec.plastic.sum() > 12 << 20
+    net = nemo_amd.Network()
+    spec.load(net)
+    sim = nemo_amd.Simulation(net, stdp(nemo_amd.Configuration()))
+    for reward in (1.0, -0.5, 0.0):
+        sim.run(60)
+        acc, w = np.asarray(sim.stdp_accumulators(), np.int64), np.asarray(sim.fixed_weights(), np.int64)
+        assert np.count_nonzero(acc) > 1000
+        sim.apply_stdp(reward)
+        dw = (int(reward * (1 << 20)) * acc) >> 20
+        top, bottom = 10 << 20, -(10 << 20)
+        want = np.where(w > 0, np.clip(w + dw, 0, top), np.where(w < 0, np.clip(w + dw, bottom, 0), 0))
+        want = np.where(spec.plastic != 0, want, w)
+        assert np.array_equal(np.asarray(sim.fixed_weights(), np.int64), want), reward
+        assert not np.any(sim.stdp_accumulators())
