@@ -194,9 +194,13 @@ apply_stdp_kernel(nemo_apply_args a)
 		for(unsigned u = 0; u < APPLY_ILP; ++u) {
 			const int32_t x = k[u].x != ~0u ? applied_weight(a, w[u].y, acc[u].x) : w[u].y;
 			const int32_t y = k[u].y != ~0u ? applied_weight(a, w[u].w, acc[u].y) : w[u].w;
-			/* changed or not: whole lines are written faster than some words of
-			 * them (638 against 685 us at 1e8 synapses, a third changed) */
-			if(k[u].x != ~0u || k[u].y != ~0u) fcm[j0 + u * NEMO_BLOCK] = make_int4(w[u].x, x, w[u].z, y);
+			/* in the large networks changed or not: whole lines are written to
+			 * memory faster than some words of them (638 against 685 us at 1e8
+			 * synapses, a third changed; at 1e7, which stay in the
+			 * memory-side cache, 91 against 85) */
+			const bool plastic = k[u].x != ~0u || k[u].y != ~0u;
+			if(plastic && (a.tile || x != w[u].y || y != w[u].w))
+				fcm[j0 + u * NEMO_BLOCK] = make_int4(w[u].x, x, w[u].z, y);
 		}
 	}
 	if(a.fcm_count % 2 && blockIdx.x == 0 && threadIdx.x == 0) {

@@ -38,6 +38,14 @@ constexpr int CARRIED_EVENT_ILP = 6;
  * and of a flush's batch, which nothing runs beside */
 constexpr int STDP_BATCH_ILP = 5;
 constexpr int STDP_FLUSH_ILP = 8;
+
+/* Synapses per listed target, on average, from which a wave passes a target by
+ * itself (stdp_batch_rows; below, its last lanes idle for longer than the
+ * search takes).  Flush of 50 steps in us, search / wave per target: 30000
+ * neurons of 80 plastic synapses each 13.6 / 14.3, 128 17.2 / 16.3, 200 25.6 /
+ * 19.8; 32 networks of 40 to 800 111 / 95; 100000 of 800 287 / 267, and the
+ * batch of 64 steps beside the steps 1020 / 888. */
+constexpr uint32_t STDP_WAVE_ROW = 112;
 /* staged events per thread the delivery sort keeps in registers */
 constexpr unsigned SORT_REGS = 8;
 
@@ -390,6 +398,78 @@ __device__ inline uint64_t history_window(uint64_t c, uint64_t s, unsigned n, un
 	return y == 0 ? lo : y < 64 ? (lo >> y) | (hi << (64 - y)) : hi;
 }
 
+/* stdp_update_region of the arrivals that a region has before the spike
+ * (after) and behind it (post): a side that the region has not, which most
+ * regions have, is a branch that a wave does not take. */
+__device__ inline int32_t stdp_update_sides(uint64_t arrivals, uint64_t pre_mask, uint64_t post_mask, unsigned post_window,
+		const int32_t* s_fn)
+{
+	const unsigned NONE = ~0u;
+	unsigned dt_pre = NONE, dt_post = NONE;
+	if(pre_mask) {
+		const uint64_t pre = arrivals & pre_mask;
+		if(pre) dt_pre = unsigned(__builtin_ctzll(pre >> post_window));
+	}
+	if(post_mask) {
+		const uint64_t post = arrivals & post_mask;
+		if(post) dt_post = unsigned(__builtin_clzll(post << (64 - post_window)));
+	}
+	if(dt_pre < dt_post) return s_fn[dt_pre];
+	if(dt_post < dt_pre) return s_fn[64 + dt_post];
+	return 0;
+}
+
+/* The listed targets' synapses for all their steps, a wave per target: its
+ * steps and row are then the wave's, in scalar registers, and no lane looks up
+ * which target its synapse belongs to. */
+template<unsigned THREADS, int SYN_ILP>
+__device__ inline void stdp_batch_rows(const nemo_hip_stdp& st, const ulonglong2* rec, unsigned cur_slot, unsigned n,
+		const int32_t* s_fn, const uint32_t* s_rb, const uint32_t* s_pos, const uint64_t* s_post, uint32_t nfired)
+{
+	const unsigned lane = threadIdx.x % 64;
+	const unsigned P = st.post_window;
+	for(unsigned idx = __builtin_amdgcn_readfirstlane(threadIdx.x / 64); idx < nfired; idx += THREADS / 64) {
+		const uint32_t rb = __builtin_amdgcn_readfirstlane(s_rb[idx]);
+		const uint32_t len = __builtin_amdgcn_readfirstlane(s_pos[idx + 1] - s_pos[idx]);
+		const uint64_t steps = uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(s_post[idx] >> 32)))) << 32
+			| uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(s_post[idx])));
+		const uint32_t* sds = st.rcm_sd + rb;
+		int32_t* accs = st.rcm_acc + rb;
+		for(uint32_t e0 = 0; e0 < len; e0 += SYN_ILP * 64) {
+			uint32_t sd[SYN_ILP];
+			int32_t acc[SYN_ILP];
+#pragma unroll
+			for(int u = 0; u < SYN_ILP; ++u) {
+				const uint32_t e = e0 + u * 64 + lane;
+				sd[u] = e < len ? sds[e] : 0u;
+				acc[u] = e < len ? accs[e] : 0;
+			}
+			uint64_t hc[SYN_ILP], hs[SYN_ILP];
+#pragma unroll
+			for(int u = 0; u < SYN_ILP; ++u) {
+				const ulonglong2 v = rec[sd[u] & 0x3ffffffu];
+				hc[u] = cur_slot ? v.y : v.x;
+				hs[u] = cur_slot ? v.x : v.y;
+			}
+#pragma unroll
+			for(int u = 0; u < SYN_ILP; ++u) {
+				if(e0 + u * 64 >= len) break;
+				const unsigned d = (sd[u] >> 26) + 1;
+				int32_t dw = 0;
+				for(uint64_t m = steps; m; m &= m - 1) {
+					const uint64_t h = history_window(hc[u], hs[u], n, unsigned(__builtin_ctzll(m)));
+					const uint64_t arrivals = d >= 64 ? 0 : (h >> d);
+					dw = stdp_wrap_add(dw, stdp_wrap_add(
+							stdp_update_sides(arrivals, st.potentiation & st.pre_post, st.potentiation & st.post_pre, P, s_fn),
+							stdp_update_sides(arrivals, st.depression & st.pre_post, st.depression & st.post_pre, P, s_fn)));
+				}
+				const uint32_t e = e0 + u * 64 + lane;
+				if(dw != 0 && e < len) accs[e] = stdp_wrap_add(acc[u], dw);
+			}
+		}
+	}
+}
+
 /* The pending STDP accumulation (clock->stdp_first, stdp_count: 1..64
  * steps r0 .. rl) for the targets of block sb's bitmap words, from the two
  * history snapshots only: after rl (slot stdp_snaps % 2 of stdp_snap) and
@@ -474,6 +554,10 @@ __device__ inline void stdp_batch_block(const nemo_propagate_args& a, unsigned s
 		__syncthreads();
 		if(total == 0) continue;
 
+		if(total >= STDP_WAVE_ROW * nfired) {
+			stdp_batch_rows<THREADS, SYN_ILP>(st, rec, cur_slot, n, s_fn, s_rb, s_pos, s_post, nfired);
+			continue;
+		}
 		for(uint32_t e0 = tid; e0 < total; e0 += SYN_ILP * THREADS) {
 			uint32_t k[SYN_ILP];
 			uint32_t sd[SYN_ILP];

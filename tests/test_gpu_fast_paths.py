@@ -296,3 +296,26 @@ def test_apply_stdp_over_tiles(n, m):
         want = np.where(spec.plastic != 0, want, w)
         assert np.array_equal(np.asarray(sim.fixed_weights(), np.int64), want), reward
         assert not np.any(sim.stdp_accumulators())
+
+
+# ------------------------------------------------- STDP rows by waves
+@pytest.mark.parametrize("n,m", [
+    (300, 130),   # about 104 plastic synapses per target: looked up one by one
+    (300, 150),   # about 120: a wave per target, most of a second chunk idle
+    (257, 640),   # exactly as many loads in flight as a wave takes, and a last word of one target
+    (700, 1300),  # more than one round of them
+])
+def test_stdp_rows_match_oracle(n, m):
+    """Accumulators and weights equal the oracle's after batches beside the
+    steps, a flush and an applyStdp."""
+    spec = gen.random_izhikevich(n, m, dmax=9, seed=n + m, stdp=True)
+    ref, hip = pair(spec, True)
+    for steps in (150, 7):
+        for _ in range(steps):
+            ref.step()
+        hip.run(steps)
+        assert np.array_equal(ref.stdp_accumulators(n * m), hip.stdp_accumulators())
+        assert np.any(hip.stdp_accumulators())
+        for sim in (ref, hip):
+            sim.apply_stdp(0.5)
+        assert np.array_equal(ref.fixed_weights(n * m), hip.fixed_weights())
