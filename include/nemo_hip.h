@@ -255,7 +255,8 @@ nemo_status_t nemo_hip_prepare(nemo_simulation_t, unsigned nsteps, unsigned stdp
  * carries the STDP blocks of STDP mode 2), 3 as in 2 with the update's tiles
  * delivering the delay-1 events of their own firing too, so that every step
  * of a run after the first is one launch.  Every shape gives identical
- * results. */
+ * results.  A network of up to 16 x 2^20 synapses delivers its events without
+ * bins, whatever shape is read, until a shape is set. */
 #define NEMO_HIP_SHAPE_FIELDS 6
 nemo_status_t nemo_hip_get_launch_shape(nemo_simulation_t, unsigned shape[NEMO_HIP_SHAPE_FIELDS]);
 nemo_status_t nemo_hip_set_launch_shape(nemo_simulation_t, const unsigned shape[NEMO_HIP_SHAPE_FIELDS]);
@@ -299,7 +300,7 @@ nemo_status_t nemo_hip_float_forward(nemo_hip_float_network_t, void* stream, uns
  * callers that cannot allocate device memory (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  Same arguments and
  * results; the forward's workspace -- weights in reverse order (4 B per
- * synapse), the state in double (16 B per neuron) and the spike bitmaps
+ * synapse; in an order with empty places where that fits too), the state in double (16 B per neuron) and the spike bitmaps
  * (4 B per 32 neurons, rounded up to 16 B, per step) -- is carved from a
  * static device array of 64 MiB per device instead of the handle's own
  * allocations, and nothing is allocated or freed.  Fails with

@@ -222,6 +222,7 @@ typedef struct nemo_propagate_args {
 	                                     column, then one per 64 device indices (pushed events) */
 	/* STDP in its own launch */
 	unsigned stdp_words;             /* bitmap words (64 targets) per STDP block */
+	unsigned stdp_rows;              /* batches: a wave may pass a target by itself */
 	uint64_t* hist;                  /* two planes of hist_pitch words (NEMO_HIST_INDEX) */
 	size_t hist_pitch;
 	uint64_t* stdp_snap;             /* STDP batches: two history snapshot slots per neuron (2n, 2n+1) */

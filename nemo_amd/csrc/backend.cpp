@@ -1214,11 +1214,14 @@ static Partition partitionPairs(const std::vector<uint64_t>& pairWeight, const s
  * atomics of all of them (23 G a second), the binned delivery a chain of
  * dependent phases that is nearly as long for 1000 neurons as for 30,000.
  * Measured on 80/20 Izhikevich networks firing at 6 to 9 Hz (neurons x
- * synapses, us a step, direct / binned): 500 x 50 5.8 / 9.4, 1000 x 100 5.5 /
- * 8.9, 10000 x 200 6.2 / 10.0, 10000 x 1000 9.1 / 12.3, 30000 x 333 8.6 /
- * 11.3, 100000 x 100 8.8 / 20.4, 30000 x 600 11.0 / 11.8, 50000 x 400 11.2 /
- * 11.6, 30000 x 1000 16.5 / 12.5, 100000 x 400 18.9 / 13.3.  So up to
- * DIRECT_MAX_SYNAPSES synapses, of which such a step delivers under 1%; the
+ * synapses, us a step, direct / binned): when it came 500 x 50 5.8 / 9.4,
+ * 1000 x 100 5.5 / 8.9, 10000 x 200 6.2 / 10.0, 10000 x 1000 9.1 / 12.3,
+ * 30000 x 333 8.6 / 11.3, 100000 x 100 8.8 / 20.4; with both as they are now
+ * 30000 x 600 10.6 / 9.4, 60000 x 300 10.3 / 10.0, 30000 x 1000 17.1 / 10.7,
+ * 60000 x 600 18.2 / 10.7, 100000 x 400 17.8 / 11.6.  So up to
+ * DIRECT_MAX_SYNAPSES synapses, of which such a step delivers under 1% (some
+ * networks beyond it would gain, 100000 x 200 10.4 / 12.4 and 200000 x 200
+ * 17.4 / 21.9, whose rows of ten synapses suit the blocks badly); the
  * ring of accumulators must not be out of proportion either (many neurons of
  * few synapses and long delays).  The tuning variables of the binned
  * delivery, or of the STDP placement, ask for that delivery. */
@@ -1478,6 +1481,11 @@ void Simulation::applyShape(const LaunchShape& s)
 	a.acc_pitch = m_accPitch;
 	a.block_events = m_blockEvents.ptr;
 	a.stdp_words = m_stdpBlocks ? s.stdpWords : 0;
+	/* beside direct steps, which leave much of the chip idle, a batch takes its
+	 * faster form; beside binned ones, which fill it, that slows the steps by
+	 * more than the batch gains (100000 x 1000, 250 steps 5681 us without and
+	 * 5782 with it; directly delivered, 30011 x 333, 150 steps 1394 and 1370) */
+	a.stdp_rows = s.direct;
 	a.hist = m_hist.ptr;
 	a.hist_pitch = m_accPitch;
 	a.stdp_snap = m_stdpSnap.ptr;
@@ -1950,6 +1958,7 @@ bool Simulation::enqueueFlush()
 		 * flushed step relative to the device's base, modulo 2^64) */
 		nemo_propagate_args a = m_propagate;
 		a.stdp_words = 1;
+		a.stdp_rows = 1;
 		const unsigned blocks = unsigned((m_firedWords + a.stdp_words - 1) / a.stdp_words);
 		HIP_CHECK(nemo_launch_stdp_flush(m_stream, &a, blocks, m_hostStep - 1 - m_base));
 		m_flushed = m_hostStep - 1;

@@ -43,8 +43,7 @@ constexpr int STDP_FLUSH_ILP = 8;
  * itself (stdp_batch_rows; below, its last lanes idle for longer than the
  * search takes).  Flush of 50 steps in us, search / wave per target: 30000
  * neurons of 80 plastic synapses each 13.6 / 14.3, 128 17.2 / 16.3, 200 25.6 /
- * 19.8; 32 networks of 40 to 800 111 / 95; 100000 of 800 287 / 267, and the
- * batch of 64 steps beside the steps 1020 / 888. */
+ * 19.8; 32 networks of 40 to 800 111 / 95; 100000 of 800 287 / 267. */
 constexpr uint32_t STDP_WAVE_ROW = 112;
 /* staged events per thread the delivery sort keeps in registers */
 constexpr unsigned SORT_REGS = 8;
@@ -192,7 +191,7 @@ __device__ inline void deliver_block(const nemo_propagate_args& a, uint64_t t, u
 			const uint32_t first = wave_append(L.pieces, np);
 			const uint32_t place = wave_append(L.fill, len);
 			for(uint32_t p0 = 0;; p0 += PIECES) {
-				/* this round's pieces */
+				/* the pieces of this pass */
 				for(uint32_t i = max(first, p0); i < min(first + np, p0 + PIECES); ++i) {
 					const uint32_t e = PIECE * (i - first);
 					L.piece[i - p0] = make_uint2(rb + e, (min(PIECE, len - e) << 25) | min(PLACES, place + e));
@@ -554,7 +553,7 @@ __device__ inline void stdp_batch_block(const nemo_propagate_args& a, unsigned s
 		__syncthreads();
 		if(total == 0) continue;
 
-		if(total >= STDP_WAVE_ROW * nfired) {
+		if(a.stdp_rows && total >= STDP_WAVE_ROW * nfired) {
 			stdp_batch_rows<THREADS, SYN_ILP>(st, rec, cur_slot, n, s_fn, s_rb, s_pos, s_post, nfired);
 			continue;
 		}
