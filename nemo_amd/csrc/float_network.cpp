@@ -46,7 +46,7 @@ FloatNetwork::FloatNetwork(const Network& net, int device) : m_device(device < 0
 	const char* env = std::getenv("NEMO_HIP_FLOAT_STAGE");
 	const bool mayStage = !env || std::string(env) != "0";
 	/* the backward's staged form, where a step's input adjoints fit in LDS
-	 * (20 224 neurons): 256 blocks share the neurons, one per compute unit,
+	 * (20 398 neurons): 256 blocks share the neurons, one per compute unit,
 	 * since each stages all the adjoints */
 	m_tile = unsigned((m_n + 255) / 256);
 	m_pushPitch = nemo_float_push_pitch(unsigned(m_n));

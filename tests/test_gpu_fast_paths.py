@@ -221,33 +221,17 @@ def test_hh_substeps_match_oracle(n):
 
 
 # ------------------------------------------------- float mode's staged forms
-@pytest.mark.parametrize("n,m,dmax,T", [
-    (2, 1, 1, 5),          # one delay: every row starts its slot
-    (255, 7, 2, 9),        # an odd size, one neuron per block, slices of one row
-    (1025, 40, 3, 30),     # a last block of neurons that is not full
-    (400, 300, 5, 40),     # more synapses than a wave has in flight
-    (300, 40, 57, 60),     # the longest delay of the windowed replay
-    (600, 130, 64, 90),    # beyond it; more slices than waves
-    (12000, 25, 19, 40),   # a lane per row
-    (20280, 12, 5, 12),    # the largest network whose adjoints fit in LDS
-    (20500, 12, 5, 12),    # one beyond that and the windows
-])
-def test_float_staged_and_general_agree(n, m, dmax, T, monkeypatch):
-    """The kernels that read their synapses in slices, with spikes and adjoints
-    in LDS, and the general ones.  The forward sums in the same order, so
-    spikes and potentials are the same bits.  The backward sums the same
-    doubles in another order, so the gradients, which are accumulated over T
-    steps in float, differ by at most T roundings of 2^-24; fired sources,
-    steps before the first and after the last included."""
+def float_results(spec, n, T, monkeypatch):
+    """Spikes, potentials and gradients with the staged kernels and with the
+    general ones, the second pass of each (which starts from the first one's
+    leavings)."""
     torch = pytest.importorskip("torch")
     from nemo_amd.differentiable import FloatNetwork
-    spec = gen.random_izhikevich(n, m, dmax=dmax, seed=n)
     rng = np.random.default_rng(n)
-    spec.weight = (spec.weight * np.float32(30.0 / m)).astype(np.float32)
     a, b, c, d, _, u, v = [np.asarray(x, np.float32) * np.ones(n, np.float32) for x in spec.blocks[0].args]
     x = (8.0 * rng.standard_normal((T, n))).astype(np.float32)
-    gS, gV = (rng.standard_normal((T, n)).astype(np.float32) for _ in range(2))
-    outs, grads = [], []
+    gS, gV = (torch.tensor(rng.standard_normal((T, n)).astype(np.float32), device="cuda") for _ in range(2))
+    out = []
     for stage in ("1", "0"):
         monkeypatch.setenv("NEMO_HIP_FLOAT_STAGE", stage)
         net = nemo_amd.Network()
@@ -256,19 +240,76 @@ def test_float_staged_and_general_agree(n, m, dmax, T, monkeypatch):
         p = {k: torch.tensor(t, device="cuda") for k, t in dict(w=spec.weight, a=a, b=b, d=d, x=x, v0=v, u0=u).items()}
         for t in p.values():
             t.requires_grad_(True)
-        for _ in range(2):  # the second pass starts from the first one's leavings
+        for _ in range(2):
             for t in p.values():
                 t.grad = None
             S, V = fnet(p["w"], p["a"], p["b"], p["d"], p["x"], c=torch.tensor(c, device="cuda"), v0=p["v0"],
                         u0=p["u0"], checkpoint_every=17)
-            torch.autograd.backward([S, V], [torch.tensor(gS, device="cuda"), torch.tensor(gV, device="cuda")])
-        outs.append((S.detach(), V.detach()))
-        grads.append({k: t.grad.double().cpu() for k, t in p.items()})
-    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
-    assert n == 2 or float(outs[0][0].sum()) > 0  # two neurons are silent
-    for k in grads[0]:
-        staged, general = grads[0][k], grads[1][k]
-        assert float((staged - general).norm()) <= T * 2.0 ** -24 * float(general.norm()), k
+            torch.autograd.backward([S, V], [gS, gV])
+        out.append((S.detach().cpu().numpy(), V.detach().cpu().numpy(),
+                    {k: t.grad.double().cpu().numpy() for k, t in p.items()}))
+    return out
+
+
+def check_float_results(staged, general, T):
+    """The forward sums in the same order, so spikes and potentials are the
+    same bits.  The backward sums the same doubles in another order, so the
+    gradients, which are accumulated over T steps in float, differ by at most T
+    roundings of 2^-24."""
+    assert np.array_equal(staged[0], general[0]) and same_f32(staged[1], general[1])
+    for k in staged[2]:
+        a, b = staged[2][k], general[2][k]
+        assert np.linalg.norm(a - b) <= T * 2.0 ** -24 * np.linalg.norm(b), k
+
+
+@pytest.mark.parametrize("n,m,dmax,T", [
+    (2, 1, 1, 5),          # one delay: every row starts its slot
+    (255, 7, 2, 9),        # an odd size, one neuron per block, slices of one row
+    (1025, 40, 3, 30),     # a last block of neurons that is not full
+    (400, 300, 5, 40),     # more synapses than a wave has in flight
+    (300, 40, 57, 60),     # the longest delay of the windowed replay
+    (600, 130, 64, 90),    # beyond it; more slices than waves
+    (12000, 25, 19, 40),   # a lane per row
+    (20398, 12, 5, 12),    # the largest network whose adjoints fit in LDS
+    (20480, 12, 5, 12),    # beyond that, the largest whose windows do
+    (20481, 12, 5, 12),    # beyond both
+])
+def test_float_staged_and_general_agree(n, m, dmax, T, monkeypatch):
+    """The kernels that read their synapses in slices, with spikes and adjoints
+    in LDS, and the general ones; fired sources, steps before the first and
+    after the last included."""
+    spec = gen.random_izhikevich(n, m, dmax=dmax, seed=n)
+    spec.weight = (spec.weight * np.float32(30.0 / m)).astype(np.float32)
+    staged, general = float_results(spec, n, T, monkeypatch)
+    assert n == 2 or staged[0].sum() > 0  # two neurons are silent
+    check_float_results(staged, general, T)
+
+
+@pytest.mark.parametrize("n,count,sources,targets", [
+    (500, 25000, None, 7),     # one target has all synapses: its slice would be mostly empty
+    (500, 20000, 3, None),     # one source: its row would be
+    (700, 9000, 2.0, 1.5),     # uneven, to powers of a uniform draw
+    (40, 30000, None, None),   # several synapses from each neuron to each
+])
+def test_float_uneven_networks_agree(n, count, sources, targets, monkeypatch):
+    """The same where degrees are uneven, on both sides of the rule that gives
+    such networks to the general kernels."""
+    rng = np.random.default_rng(count)
+
+    def draw(kind):
+        if isinstance(kind, int):
+            return np.full(count, kind)
+        return (n * rng.random(count) ** (kind or 1.0)).astype(np.int64)
+
+    src = np.sort(draw(sources))
+    spec = gen.random_izhikevich(n, 0, dmax=1, seed=3)
+    spec.source, spec.target = src.astype(np.uint32), draw(targets).astype(np.uint32)
+    spec.delay = rng.integers(1, 9, count).astype(np.uint32)
+    spec.weight = (rng.random(count) * 0.05).astype(np.float32)
+    spec.plastic = np.zeros(count, np.uint8)
+    staged, general = float_results(spec, n, 60, monkeypatch)
+    assert staged[0].sum() > 0
+    check_float_results(staged, general, 60)
 
 
 # ------------------------------------------------- applyStdp over tiles
